@@ -114,7 +114,7 @@ def granular(steps=500, check_steps=300):
     return out, samples
 
 
-STEP_KERNELS = ("hash", "scan", "scatter", "rank_move", "shepard", "nl_build", "init_tmp", "wc_eos", "wc_bdy",
+STEP_KERNELS = ("sort_small", "hash", "scan", "scatter", "rank_move", "shepard", "nl_build", "init_tmp", "wc_eos", "wc_bdy",
                 "wc_fluid", "lf_half", "lf_full", "advect_pos", "chk_density", "finish")
 
 

@@ -42,6 +42,7 @@ struct SceneDev {
   int32_t gn[3];
   int32_t tile_first, n_tiles;
   int32_t pbase, n, cbase, ncell;
+  int32_t sbase, total;  // particles of the scenes with lower cells, of all scenes
   double grid, vds[3], dstart[3], dend[3], radius, dt_d;
   float g, rs2, h1, kW, kC, eps;
   float kG, kGc;  // gradient factors: -5 kW h1^2 (Wendland C2), kC h1^2 (cubic)

@@ -133,9 +133,12 @@ struct Timing {
 struct StepFlags {
   int ti = 2;
   bool xsph = false, collide = false, kcorr = false, rigid = false, rep = false;
+  // cells of the largest resident scene, rounded up to a power of two, if
+  // every one is small enough for k_sort_small; 0 otherwise
+  int small_cells = 0;
   bool operator==(const StepFlags& o) const {
     return ti == o.ti && xsph == o.xsph && collide == o.collide && kcorr == o.kcorr &&
-           rigid == o.rigid && rep == o.rep;
+           rigid == o.rigid && rep == o.rep && small_cells == o.small_cells;
   }
 };
 
@@ -299,6 +302,7 @@ int ensure_rigid(tsph_engine* E) {
 struct Launcher {
   tsph_engine* E;
   int status = TSPH_OK;
+  int lds = 0;  // dynamic LDS of the next launches, bytes
   template <class K, class... Args>
   void go(const char* name, K kernel, int grid, int block, Args... args) {
     if (status != TSPH_OK || grid <= 0) return;
@@ -318,7 +322,7 @@ struct Launcher {
       T.pool.pop_back();
       hipEventRecord(rec.a, E->stream);
     }
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, E->stream, args...);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, E->stream, args...);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) status = fail(TSPH_ERR_HIP, std::string(name) + ": " + hipGetErrorString(e));
     if (timed) {
@@ -356,14 +360,19 @@ struct Seq {
   void sort(bool fuse_init = false) {
     KArgs a = E->args();
     const int eb = E->elem_block;
-    L.go("hash", k_hash<DIM>, tb(), eb, a);
-    const int n = E->ccap;
-    const int nb = (n + kScanTile - 1) / kScanTile;
-    L.go("scan", k_scan_reduce, nb, kScanBlock, (const int32_t*)E->w.count, E->w.bsum, n);
-    L.go("scan", k_scan_bsum, 1, kScanBlock, E->w.bsum, nb, E->w.start, n);
-    L.go("scan", k_scan_down, nb, kScanBlock, E->w.count, (const int32_t*)E->w.bsum, E->w.start,
-         E->w.cflow, n);
-    L.go("scatter", k_scatter, tb(), eb, a);
+    if (const int cells = step_flags(E).small_cells) {
+      L.lds = cells * (int)sizeof(int32_t);
+      L.go("sort_small", k_sort_small<DIM>, E->max_scenes, kSmallBlock, a);
+      L.lds = 0;
+    } else {
+      L.go("hash", k_hash<DIM>, tb(), eb, a);
+      const int n = E->ccap;
+      const int nb = (n + kScanTile - 1) / kScanTile;
+      L.go("scan", k_scan_reduce, nb, kScanBlock, (const int32_t*)E->w.count, E->w.bsum, n);
+      L.go("scan", k_scan_down, nb, kScanBlock, E->w.count, (const int32_t*)E->w.bsum, E->w.start,
+           E->w.cflow, n);
+      L.go("scatter", k_scatter, tb(), eb, a);
+    }
     L.go("rank_move", k_rank_move, (E->cap + eb - 1) / eb, eb, a, 1, E->method == kMUI ? 1 : 0,
          E->method == kDP ? 1 : 0, fuse_init ? 1 : 0);
     E->parity ^= 1;
@@ -542,9 +551,12 @@ struct Seq {
 
 StepFlags step_flags(tsph_engine* E) {
   StepFlags f;
-  bool first = true;
+  bool first = true, small = true;
+  int cells = 0;
   for (size_t s = 0; s < E->scenes.size(); ++s) {
     if (!E->scenes[s].active) continue;
+    small = small && E->scenes[s].n <= kSmallParticles && E->scenes[s].ncell <= kSmallCells;
+    cells = std::max(cells, E->scenes[s].ncell);
     if (first) f.ti = E->scenes[s].ti;
     first = false;
     f.xsph = f.xsph || E->scenes[s].xsph;
@@ -552,6 +564,10 @@ StepFlags step_flags(tsph_engine* E) {
     f.kcorr = f.kcorr || E->scenes[s].kcorr != 0;
     f.rigid = f.rigid || E->scenes[s].nrig > 0;
     f.rep = f.rep || E->scenes[s].rep != 0;
+  }
+  if (small && !first) {
+    f.small_cells = 64;
+    while (f.small_cells < cells) f.small_cells *= 2;
   }
   return f;
 }
@@ -612,6 +628,17 @@ int upload_tables(tsph_engine* E) {
       S.n_tiles++;
     }
   }
+  // particles in cell order: where each scene's cells start in the sorted run
+  std::vector<SceneDev*> order;
+  int total = 0;
+  for (SceneDev& S : E->scenes)
+    if (S.active) order.push_back(&S);
+  std::sort(order.begin(), order.end(), [](const SceneDev* x, const SceneDev* y) { return x->cbase < y->cbase; });
+  for (SceneDev* S : order) {
+    S->sbase = total;
+    total += S->n;
+  }
+  for (SceneDev* S : order) S->total = total;
   HIP_TRY(hipMemcpyAsync(E->d_tiles, E->tiles.data(), E->tiles.size() * sizeof(int2),
                          hipMemcpyHostToDevice, E->stream));
   HIP_TRY(hipMemcpyAsync(E->d_scenes, E->scenes.data(), E->scenes.size() * sizeof(SceneDev),
