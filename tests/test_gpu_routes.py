@@ -53,3 +53,55 @@ def test_sort_route_of_small_scenes(dim, block):
     alone, beside = run([sc], 5), run([sc, wide], 5)
     for f in STATE:
         np.testing.assert_array_equal(alone[f], beside[f], err_msg=f)
+
+
+def uneven(method, dim, nan, seed=3):
+    """A scene whose flow particles lie from far apart to ~80 per cell (lists
+    longer than the engine keeps, cells of more than 32 particles, windows
+    wider than a cell tile), in any order; ``nan``: one offset is not a
+    number and one is infinite."""
+    r = 0.006 if dim == 2 else 0.016
+    sc = build_scene(tiny_cfg(method=method, dim=dim, xsph=True, r=r, domain=(1.0, 0.6, 0.24),
+                              block=(0.6, 0.3, 0.24) if dim == 2 else (0.4, 0.3, 0.24)))
+    rng = np.random.default_rng(seed)
+    flow = np.flatnonzero((sc.mat_type == 1) | (sc.mat_type == 2))
+    n = flow.size
+    # x crowds towards 0: the density falls off exponentially along x
+    x = np.stack([rng.exponential(0.05, n) % 0.9, rng.uniform(0.02, 0.5, n), rng.uniform(0.02, 0.2, n)], 1)
+    sc.pos[flow, :dim] = (x + 0.02)[:, :dim]
+    sc.vel[flow, :dim] = rng.uniform(-0.1, 0.1, (n, dim))
+    bad = {int(flow[5]): np.nan, int(flow[70]): np.inf} if nan else {}
+    return sc, bad
+
+
+@pytest.mark.parametrize("method,dim,nan", [(1, 2, False), (1, 3, False), (2, 2, False), (3, 2, False), (3, 3, False),
+                                            (1, 2, True)])
+def test_list_modes_agree_on_uneven_scenes(method, dim, nan):
+    """Walk in every pass (mode 0), lists from the walk (1) and from staged
+    windows (2, every cell tile) give the same bits."""
+    sc, bad = uneven(method, dim, nan)
+    fields = STATE + (["stress"] if method != 1 else [])
+    ref = None
+    for mode, tile in [(0, 256), (1, 256), (2, 128), (2, 256), (2, 512)]:
+        eng = L.Engine(sc.method, dim, sc.n, sc.geo.grid_num_total, 1)
+        eng.set_neighbor_list(mode)
+        eng.set_cell_tile(tile)
+        slot = eng.add_scene(sc.desc())
+        L.upload_scene(eng, slot, sc)
+        if bad:
+            off = eng.download(slot, "offset")
+            for i, v in bad.items():
+                off[i, 0] = v
+            eng.upload(slot, "offset", off)
+        if mode == 2 and not nan:
+            eng.run("sort")
+            eng.run("shepard")
+            count = eng.neighbor_lists(slot)[0]
+            assert (count == -1).any() and (count == 0).any() and (count > 0).any()
+        eng.step(2)
+        out = {f: eng.download(slot, f) for f in fields}
+        eng.close()
+        if ref is None:
+            ref = out
+        for f in fields:
+            np.testing.assert_array_equal(out[f], ref[f], err_msg=f"mode {mode} tile {tile}: {f}")

@@ -121,6 +121,7 @@ struct PWork {
   double* gout;      // globals per slot (4 each)
   uint32_t* nl;      // neighbour lists, blocked per 64-particle tile (nl_base / nl_at)
   int32_t* nlc;      // neighbour count per particle (> nl_cap: walk instead)
+  int32_t* tflag;    // per tile: what the pair passes find there (kTile*)
   // colour feed (allocated on first use)
   double* val;       // colour value per particle (current order)
   float4* rgb;       // colour per particle (current order)
@@ -141,6 +142,7 @@ struct KArgs {
   int32_t ccap;    // cell capacity
   int32_t stride;  // component stride of 6-vectors (== cap)
   int32_t nl_cap;  // neighbour-list capacity per particle
+  uint32_t nl_pad; // list entry of the null particle (pads lists to kNlPad)
 };
 
 // ---------------------------------------------------------- pair distance
@@ -199,14 +201,21 @@ __device__ __forceinline__ float kernel_gradfac(const SceneDev& S, float rn) {
 // branch (both cubic pieces are formed and one is selected): identical
 // values, but a pair loop built on them is straight-line code, so the
 // loads of several neighbours can be in flight together.
+// 1 - q / 2 clamped to [0, 1] (the instruction's output modifier): q <= 2
+// exactly where 1 - q / 2 >= 0, and beyond it W = 0 and W'(r)/r = +-0 follow
+// from the zero, so the Wendland functions need no test of q.
+__device__ __forceinline__ float wendland_q1(float q) {
+  return __builtin_amdgcn_fmed3f(1.0f - 0.5f * q, 0.0f, 1.0f);
+}
 template <int KT>
 __device__ __forceinline__ float kernel_W_t(const SceneDev& S, float rn) {
   const float q = rn * S.h1;
   float w;
   if (KT == 1) {
-    const float q1 = 1.0f - 0.5f * q;
+    const float q1 = wendland_q1(q);
     const float q2 = q1 * q1;
     w = S.kW * (q2 * q2) * (1.0f + 2.0f * q);
+    return rn > S.eps ? w : 0.0f;
   } else {
     const float qq = q * q;
     const float wi = S.kC * (0.5f * (qq * q) - qq + (float)(2.0 / 3.0));
@@ -221,8 +230,9 @@ __device__ __forceinline__ float kernel_gradfac_t(const SceneDev& S, float rn) {
   const float q = rn * S.h1;
   float f;
   if (KT == 1) {
-    const float q1 = 1.0f - 0.5f * q;
+    const float q1 = wendland_q1(q);
     f = S.kG * ((q1 * q1) * q1);
+    return rn > S.eps ? f : 0.0f;
   } else {
     const float fi = S.kGc * (1.5f * q - 2.0f);
     const float t = 2.0f - q;
@@ -427,80 +437,146 @@ constexpr int kNlShift = 6;
 __device__ __forceinline__ uint32_t nl_entry(int j, int code) {
   return ((uint32_t)j << kNlShift) | (uint32_t)code;
 }
-// Storage of the lists, blocked per 64-particle tile and, inside a tile,
-// in runs of 16 entries per particle: entry k of particle p sits at
-// nl_base(p) + nl_at(k) with nl_base = tile * 64 * nl_cap + lane * 16 and
-// nl_at(k) = (k / 16) * 1024 + k % 16.  A wave's lists are one contiguous
-// run of 64 * nl_cap entries whatever the engine capacity (its traffic
-// stays within a page or two); each lane appends into its own 64-byte run
-// (four entries per aligned 16-byte store), and the replay loads a lane's
-// entries k..k+3 with one 16-byte load.  (Runs of 4, which make the
-// replay's loads one contiguous kilobyte per wave, measured ~4 % slower per
-// step.)  nl_cap is a multiple of 16.
+// Storage of the lists, blocked per 64-particle tile: entry k of particle p
+// is at nl_base(p) + nl_at(k), the tile's piece of 64 nl_cap entries being
+// rows of 256, four entries (16 bytes) of each particle.  A replay load (16
+// particles, a quad of lanes each) is 256 contiguous bytes and a build store
+// (64 particles, four entries each) a contiguous kilobyte; a tile's lists
+// are one piece whatever the engine capacity.  nl_cap is a multiple of 4.
 __host__ __device__ __forceinline__ size_t nl_base(int p, int nl_cap) {
-  return (size_t)(p >> 6) * ((size_t)nl_cap << 6) + ((size_t)(p & 63) << 4);
+  return (size_t)(p >> 6) * ((size_t)nl_cap << 6) + ((size_t)(p & 63) << 2);
 }
 __host__ __device__ __forceinline__ size_t nl_at(int k) {
-  return ((size_t)(k >> 4) << 10) + (size_t)(k & 15);
+  return ((size_t)(k >> 2) << 8) + (size_t)(k & 3);
 }
 
-// Per-thread table of the list replay (one 9 KiB LDS array per kernel that
-// replays lists, shared by all its replays: a thread only ever touches its
-// own column).
+// Lanes per particle of the list replay: L = 4 lanes of a quad share one
+// particle (L = 1: the stencil walk).  Lane q forms the terms of the list
+// entries k + q, and every lane then adds the four terms in list order, the
+// other lanes' read through DPP quad permutations: the same additions in the
+// same order as with one lane, so the sums have the same bits.
+// Lists are padded to a multiple of kNlPad entries with the null particle
+// (m_V = 0: every term it gives is +-0, which changes no sum, since a sum
+// that starts at +0 is never -0 in round-to-nearest).
 constexpr int kMaxBlock = 256;  // largest threads per block of a pair kernel
-__device__ __forceinline__ float* shift_table() {
-  __shared__ float tab[9 * kMaxBlock];
+constexpr int kNlPad = 4;
+constexpr int kLanes = 4;
+
+// x of lane SRC of this lane's group of L.
+template <int L, int SRC>
+__device__ __forceinline__ float group_read(float x) {
+  static_assert(L == 4, "a quad");
+  constexpr int ctrl = SRC * 0x55;  // quad_perm [SRC, SRC, SRC, SRC]
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+// acc += the terms of the group's lanes, lane 0 first.
+template <int L, int NT>
+__device__ __forceinline__ void ordered_add(float (&acc)[NT], const float (&t)[NT]) {
+#pragma unroll
+  for (int c = 0; c < NT; ++c) {
+    if (L == 1) {
+      acc[c] += t[c];
+    } else {
+      acc[c] += group_read<4, 0>(t[c]);
+      acc[c] += group_read<4, 1>(t[c]);
+      acc[c] += group_read<4, 2>(t[c]);
+      acc[c] += group_read<4, 3>(t[c]);
+    }
+  }
+}
+
+// Tables of the list replay: one LDS array per kernel, shared by all its
+// replays (an array inside the template below would be one per instance).
+constexpr int kTabCols = kMaxBlock / 4;
+__device__ __forceinline__ float2* xy_table() {
+  __shared__ float2 tab[11 * kTabCols];
+  return tab;
+}
+__device__ __forceinline__ float* z_table() {
+  __shared__ float tab[3 * kTabCols];
   return tab;
 }
 
-template <int DIM, class Fn>
-__device__ __forceinline__ void for_list(const SceneDev& S, const uint32_t* __restrict__ nl,
-                                         int n, int nl_cap, const float4* __restrict__ pos, int i,
-                                         float oix, float oiy, float oiz, Fn&& fn) {
-  const uint32_t* __restrict__ li = nl + nl_base(i, nl_cap);
+// A particle with the start of its list.
+struct Own {
+  float4 P;
+  int n;            // list length
+  uint32_t e0, e1;  // this lane's entries of the first two quads
+};
+
+// acc[c] += term c of every neighbour of particle i, in list order.
+// fn(j, x, y, z, r2, m_V_j, t) forms the terms t of one pair.
+template <int DIM, int NT, class Fn>
+__device__ __forceinline__ void sum_list(const SceneDev& S, const uint32_t* __restrict__ nl, int nl_cap,
+                                         const float4* __restrict__ pos, int i, const Own& o,
+                                         float (&acc)[NT], Fn&& fn) {
+  const int n = o.n;
+  const float oix = o.P.x, oiy = o.P.y, oiz = o.P.z;
+  const uint32_t* __restrict__ li = nl + nl_base(i, nl_cap) + (threadIdx.x & 3);
   // shifted centres oi + (c_i - c_j) g for c_j - c_i = -1, 0, +1 (exact
-  // products, rounded once: the same values the walk forms), kept in LDS as
-  // row 3 * axis + code digit, column = thread, so that a pair looks its
-  // three up by address (conflict-free: every lane reads its own column)
-  // instead of by four compares and selects per axis
-  float* __restrict__ tab = shift_table();
-  const int t = (int)threadIdx.x;
-  tab[0 * kMaxBlock + t] = oix + S.g;
-  tab[1 * kMaxBlock + t] = oix;
-  tab[2 * kMaxBlock + t] = oix + (-1.0f) * S.g;
-  tab[3 * kMaxBlock + t] = oiy + S.g;
-  tab[4 * kMaxBlock + t] = oiy;
-  tab[5 * kMaxBlock + t] = oiy + (-1.0f) * S.g;
+  // products, rounded once: the same values the walk forms), kept in LDS
+  // (one table per kernel, a wave only ever touches its own columns, one per
+  // particle): x and y together in row (x digit, y digit) of the stencil
+  // code, z in a table of its own, so a pair looks them up by address
+  // instead of by compares and selects
+  constexpr int kCols = kTabCols;
+  float2* __restrict__ txy = xy_table();
+  float* __restrict__ tz = DIM == 3 ? z_table() : nullptr;
+  const int col = (int)threadIdx.x >> 2;
+#pragma unroll
+  for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+      txy[(dx * 4 + dy) * kCols + col] =
+          make_float2(dx == 0 ? oix + S.g : (dx == 1 ? oix : oix + (-1.0f) * S.g),
+                      dy == 0 ? oiy + S.g : (dy == 1 ? oiy : oiy + (-1.0f) * S.g));
   if (DIM == 3) {
-    tab[6 * kMaxBlock + t] = oiz + S.g;
-    tab[7 * kMaxBlock + t] = oiz;
-    tab[8 * kMaxBlock + t] = oiz + (-1.0f) * S.g;
+    tz[0 * kCols + col] = oiz + S.g;
+    tz[1 * kCols + col] = oiz;
+    tz[2 * kCols + col] = oiz + (-1.0f) * S.g;
   }
-  auto pair = [&](uint32_t e, const float4& pj) {
+  auto pair = [&](uint32_t e, const float4& pj, float (&tm)[NT]) {
     const int j = (int)(e >> kNlShift);
-    const int code = (int)(e & 63u);
-    const float x = tab[(int)((e >> 4) & 3u) * kMaxBlock + t] - pj.x;
-    const float y = tab[(3 + (int)((e >> 2) & 3u)) * kMaxBlock + t] - pj.y;
-    const float z = DIM == 3 ? tab[(6 + (int)(e & 3u)) * kMaxBlock + t] - pj.z : 0.0f;
-    const float r2 = fmaf(z, z, fmaf(y, y, x * x));
-    fn(j, x, y, z, r2, pj.w, code);
+    const float2 c = txy[(int)((e >> 2) & 15u) * kCols + col];
+    const float x = c.x - pj.x;
+    const float y = c.y - pj.y;
+    const float z = DIM == 3 ? tz[(int)(e & 3u) * kCols + col] - pj.z : 0.0f;
+    const float r2 = DIM == 3 ? fmaf(z, z, fmaf(y, y, x * x)) : fmaf(y, y, x * x);
+    fn(j, x, y, z, r2, pj.w, tm);
   };
+  auto rec = [&](uint32_t e) {
+    float4 v = pos[e >> kNlShift];
+    // whole 16-byte record: in 2D z is unused, and the compiler would split
+    // the load into two
+    if (DIM == 2) asm volatile("" : "+v"(v.z));
+    return v;
+  };
+  if (n <= 0) return;
+  // Two quads of entries per turn, the next turn's loaded while this turn's
+  // neighbours arrive (and none past the list's end: a line of list that no
+  // pair needs cost the batched 2D pass 20 %).
+  uint32_t e0 = o.e0, e1 = o.e1;
+  float t[NT];
   int k = 0;
-  // Four entries at a time: one 16-byte load (a lane's entries k..k+3 are
-  // contiguous), then the four neighbours' loads together, then the four
-  // pairs in list order.
-  for (; k + 4 <= n; k += 4) {
-    const uint4 e4 = *reinterpret_cast<const uint4*>(li + nl_at(k));
-    const float4 p0 = pos[e4.x >> kNlShift], p1 = pos[e4.y >> kNlShift];
-    const float4 p2 = pos[e4.z >> kNlShift], p3 = pos[e4.w >> kNlShift];
-    pair(e4.x, p0);
-    pair(e4.y, p1);
-    pair(e4.z, p2);
-    pair(e4.w, p3);
+  for (; k + 8 <= n; k += 8) {
+    const float4 p0 = rec(e0), p1 = rec(e1);
+    uint32_t f0 = 0, f1 = 0;
+    if (k + 8 < n) f0 = li[nl_at(k + 8)];
+    if (k + 12 < n) f1 = li[nl_at(k + 12)];
+    pair(e0, p0, t);
+    ordered_add<4>(acc, t);
+    pair(e1, p1, t);
+    ordered_add<4>(acc, t);
+    e0 = f0;
+    e1 = f1;
   }
-  for (; k < n; ++k) {
-    const uint32_t e = li[nl_at(k)];
-    pair(e, pos[e >> kNlShift]);
+  if (k < n) {
+    pair(e0, rec(e0), t);
+    ordered_add<4>(acc, t);
+  }
+  if (k + 4 < n) {
+    pair(e1, rec(e1), t);
+    ordered_add<4>(acc, t);
   }
 }
 

@@ -182,6 +182,7 @@ struct tsph_engine {
     a.ccap = ccap;
     a.stride = cap;
     a.nl_cap = nl_cap;
+    a.nl_pad = (uint32_t)(cap - kTileAlign) << kNlShift;  // the null particle
     return a;
   }
   int nblocks_tiles(int block) const { return (tiles_alloc * 64 + block - 1) / block; }
@@ -213,6 +214,15 @@ int alloc_state(tsph_engine* E, PState& s) {
   return TSPH_OK;
 }
 
+// The null particle: all fields zero (m_V = 0, no type), density 1 so that
+// the soil terms divide by it; no scene range covers it.
+int init_null_particle(tsph_engine* E) {
+  const float4 v = make_float4(0.f, 0.f, 0.f, 1.f);
+  for (PState& s : E->buf)
+    HIP_TRY(hipMemcpy(s.vtmp + (E->cap - kTileAlign), &v, sizeof(v), hipMemcpyHostToDevice));
+  return TSPH_OK;
+}
+
 void free_state(PState& s) {
   void* ptrs[] = {s.cell, s.pos, s.vel, s.vtmp, s.mass, s.type, s.id0, s.obj, s.sig_f, s.sig_d,
                   s.seq, s.seqp, s.flag};
@@ -238,7 +248,8 @@ int alloc_work(tsph_engine* E) {
       (r = dalloc(&w.status, 2 * (size_t)E->max_scenes, b)) ||
       (r = dalloc(&w.gpart, 4 * (size_t)E->tiles_alloc, b)) ||
       (r = dalloc(&w.gout, 4 * (size_t)E->max_scenes, b)) ||
-      (r = dalloc(&w.nlc, n, b)) || (r = dalloc(&w.nl, (size_t)E->nl_cap * 64 * (size_t)E->tiles_alloc, b)))
+      (r = dalloc(&w.nlc, n, b)) || (r = dalloc(&w.nl, (size_t)E->nl_cap * 64 * (size_t)E->tiles_alloc, b)) ||
+      (r = dalloc(&w.tflag, E->tiles_alloc, b)))
     return r;
   if (E->method != kWC) {
     if ((r = dalloc(&w.sigt_f, n6, b)) || (r = dalloc(&w.dseq, n, b))) return r;
@@ -254,7 +265,7 @@ int alloc_work(tsph_engine* E) {
 void free_work(PWork& w) {
   void* ptrs[] = {w.key, w.slot, w.tmp, w.sid, w.p, w.vp, w.Lc, w.cspm, w.drho, w.dv, w.sigt_f, w.sigt_d,
                   w.dsig_d, w.dseq, w.dseqp, w.xs, w.drho_rk, w.dv_rk, w.dsig_rk, w.count,
-                  w.start, w.bsum, w.status, w.gpart, w.gout, w.nl, w.nlc, w.cflow,
+                  w.start, w.bsum, w.status, w.gpart, w.gout, w.nl, w.nlc, w.tflag, w.cflow,
                   w.val, w.rgb, w.x0, w.c0, w.crange, w.rigpart, w.rigout};
   for (void* p : ptrs)
     if (p) hipFree(p);
@@ -354,6 +365,7 @@ struct Seq {
   Launcher& L;
   int tb() const { return E->nblocks_tiles(E->elem_block); }
   int pb() const { return E->nblocks_tiles(E->pair_block); }
+  int lb() const { return pb() * kLanes; }  // of a list pass
 
   // update_grid_id + prefix sum + counting_sort; with fuse_init the move
   // also performs init_real2tmp and the first EOS of the step.
@@ -390,24 +402,20 @@ struct Seq {
     if (E->use_nl) {
       const int cf = E->cflow_valid ? 1 : 0, cull = E->fresh_sort ? 1 : 0;
       if (E->nl_lds) {
-        const KArgs a = E->args();
-        if (E->nl_stage == 128)
-          L.go("nl_build", k_nl_build_lds<DIM, 128>, E->tiles_alloc, 64, a, cf, cull);
-        else if (E->nl_stage == 512)
-          L.go("nl_build", k_nl_build_lds<DIM, 512>, E->tiles_alloc, 64, a, cf, cull);
-        else
-          L.go("nl_build", k_nl_build_lds<DIM, 256>, E->tiles_alloc, 64, a, cf, cull);
+        auto k = E->nl_stage == 128 ? k_nl_build_lds<DIM, 128>
+                                    : (E->nl_stage == 512 ? k_nl_build_lds<DIM, 512> : k_nl_build_lds<DIM, 256>);
+        L.go("nl_build", k, E->tiles_alloc, 64 * kBuildWaves, E->args(), cf);
       } else
         L.go("nl_build", k_nl_build<DIM>, pb(), E->pair_block, E->args(), cf, cull);
       E->nl_valid = true;
       if (!skip_all)
-        L.go("shepard", k_shepard_list<DIM>, pb(), E->pair_block, E->args(), skip_fluid ? 1 : 0);
+        L.go("shepard", k_shepard_list<DIM>, lb(), E->pair_block, E->args(), skip_fluid ? 1 : 0);
     } else if (!skip_all) {
       L.go("shepard", k_shepard<DIM>, pb(), E->pair_block, E->args(), skip_fluid ? 1 : 0);
     }
     // calc_kernel_corr (solver_sph_base.py:363-368): CSPM_L after CSPM_f
     if (step_flags(E).kcorr) {
-      if (E->nl_valid) L.go("cspm_L", k_cspm_L<DIM, true>, pb(), E->pair_block, E->args());
+      if (E->nl_valid) L.go("cspm_L", k_cspm_L<DIM, true>, lb(), E->pair_block, E->args());
       else L.go("cspm_L", k_cspm_L<DIM, false>, pb(), E->pair_block, E->args());
     }
   }
@@ -415,33 +423,38 @@ struct Seq {
   // one_step of the method; with_eos=false when the EOS was fused into the
   // kernel before (the move of the sort, or lf_half); shep: the WC fluid
   // pass also forms the fluid particles' Shepard factors.
-  void one_step(bool with_eos = true, bool shep = false) {
-    if (E->nl_valid) one_step_t<true>(with_eos, shep);
-    else one_step_t<false>(with_eos, shep);
+  // again: a later one_step of a fused step (what the first stored for
+  // particles without pairs still holds).
+  void one_step(bool with_eos = true, bool shep = false, bool again = false) {
+    if (E->nl_valid) one_step_t<true>(with_eos, shep, again ? 1 : 0);
+    else one_step_t<false>(with_eos, shep, again ? 1 : 0);
   }
   template <bool NL>
-  void one_step_t(bool with_eos, bool shep) {
+  void one_step_t(bool with_eos, bool shep, int again) {
     KArgs a = E->args();
-    const int B = E->pair_block;
+    const int B = E->pair_block, G = NL ? lb() : pb();
+    // kernel-corrected scenes run kernels that hold the correction's branch
+    const bool kc = step_flags(E).kcorr;
     if (E->method == kWC) {
       if (with_eos) L.go("wc_eos", k_wc_eos, tb(), E->elem_block, a);
-      if (shep) L.go("wc_bdy", k_wc_bdy<DIM, NL, true>, pb(), B, a);
-      else L.go("wc_bdy", k_wc_bdy<DIM, NL, false>, pb(), B, a);
-      if (shep) L.go("wc_fluid", k_wc_fluid<DIM, NL, true>, pb(), B, a);
-      else L.go("wc_fluid", k_wc_fluid<DIM, NL, false>, pb(), B, a);
+      L.go("wc_bdy", shep ? k_wc_bdy<DIM, NL, true> : k_wc_bdy<DIM, NL, false>, G, B, a, again);
+      L.go("wc_fluid",
+           shep ? (kc ? k_wc_fluid<DIM, NL, true, true> : k_wc_fluid<DIM, NL, true, false>)
+                : (kc ? k_wc_fluid<DIM, NL, false, true> : k_wc_fluid<DIM, NL, false, false>),
+           G, B, a, again);
     } else if (E->method == kMUI) {
-      L.go("mui_soil1", k_mui_soil1<DIM, NL>, pb(), B, a);
-      L.go("soil_bdy", k_soil_bdy<DIM, true, NL>, pb(), B, a);
-      L.go("mui_soil3", k_mui_soil3<DIM, NL>, pb(), B, a);
+      L.go("mui_soil1", kc ? k_mui_soil1<DIM, NL, true> : k_mui_soil1<DIM, NL, false>, G, B, a, again);
+      L.go("soil_bdy", k_soil_bdy<DIM, true, NL>, G, B, a, again);
+      L.go("mui_soil3", kc ? k_mui_soil3<DIM, NL, true> : k_mui_soil3<DIM, NL, false>, G, B, a, again);
     } else {
       L.go("dp_adapt", k_dp_adapt, tb(), E->elem_block, a);
-      L.go("soil_bdy", k_soil_bdy<DIM, false, NL>, pb(), B, a);
-      L.go("dp_soil", k_dp_soil<DIM, NL>, pb(), B, a);
+      L.go("soil_bdy", k_soil_bdy<DIM, false, NL>, G, B, a, again);
+      L.go("dp_soil", kc ? k_dp_soil<DIM, NL, true> : k_dp_soil<DIM, NL, false>, G, B, a, again);
     }
   }
   void lf_half(bool eos = false) { L.go("lf_half", k_lf_half, tb(), E->elem_block, E->args(), eos ? 1 : 0); }
   void lf_full() { L.go("lf_full", k_lf_full, tb(), E->elem_block, E->args()); }
-  void substep(int ti, bool shep_first = false) {
+  void substep(int ti, bool shep_first = false, bool fused = false) {
     if (ti == 1) {
       one_step(true, shep_first);
       lf_full();
@@ -455,7 +468,7 @@ struct Seq {
       L.go("rk", k_rk_init, tb(), E->elem_block, a);
       const int m[4] = {1, 2, 2, 1};
       for (int k = 0; k < 4; ++k) {
-        one_step(true, shep_first && k == 0);
+        one_step(true, shep_first && k == 0, fused && k > 0);
         L.go("rk", k_rk_update, tb(), E->elem_block, a, m[k]);
         if (k < 3) L.go("rk", k_rk_advect4, tb(), E->elem_block, a);
       }
@@ -466,7 +479,7 @@ struct Seq {
     E->fresh_sort = false;
     KArgs a = E->args();
     if (xsph) {
-      if (E->nl_valid) L.go("xsph", k_xsph<DIM, true>, pb(), E->pair_block, a);
+      if (E->nl_valid) L.go("xsph", k_xsph<DIM, true>, lb(), E->pair_block, a);
       else L.go("xsph", k_xsph<DIM, false>, pb(), E->pair_block, a);
     }
     L.go("advect_pos", k_advect_pos, tb(), E->elem_block, a, xsph ? 1 : 0);
@@ -520,17 +533,17 @@ struct Seq {
     if (ti == 2) {
       one_step(false, shep);
       lf_half(true);
-      one_step(false);
+      one_step(false, false, true);
     } else if (ti == 1) {
       one_step(false, shep);
     } else {
-      substep(4, shep);
+      substep(4, shep, true);
     }
     const bool lf_in_finish = ti != 4 && !xsph;
     KArgs a = E->args();
     if (xsph) {
       if (ti != 4) lf_full();
-      if (E->nl_valid) L.go("xsph", k_xsph<DIM, true>, pb(), E->pair_block, a);
+      if (E->nl_valid) L.go("xsph", k_xsph<DIM, true>, lb(), E->pair_block, a);
       else L.go("xsph", k_xsph<DIM, false>, pb(), E->pair_block, a);
     }
     L.go("finish", k_finish, tb(), E->elem_block, a, lf_in_finish ? 1 : 0, xsph ? 1 : 0);
@@ -1092,7 +1105,7 @@ int tsph_engine_create(int method, int dim, int64_t particle_capacity, int64_t c
       return rs;
     }
   }
-  E->cap = (int32_t)pc;
+  E->cap = (int32_t)pc + kTileAlign;  // the last tile holds the null particle of padded lists
   E->ccap = (int32_t)cell_capacity;
   // 3D lattice: 92 neighbours (+30 exactly at r_s); 2D: 24 (+4).  Denser
   // particles fall back to the stencil walk.
@@ -1112,6 +1125,7 @@ int tsph_engine_create(int method, int dim, int64_t particle_capacity, int64_t c
   if (!r) r = alloc_work(E);
   if (!r) r = dalloc(&E->d_scenes, max_scenes, E->bytes);
   if (!r) r = dalloc(&E->d_tiles, E->tiles_alloc, E->bytes);
+  if (!r) r = init_null_particle(E);
   if (!r) r = upload_tables(E);
   if (r) {
     tsph_engine_destroy(E);
@@ -1588,7 +1602,7 @@ int tsph_neighbor_lists(void* engine, int slot, int32_t* count, int32_t* ids, in
       continue;
     }
     count[i] = c;
-    const int64_t lb = (i >> 6) * per_tile + ((i & 63) << 4);
+    const int64_t lb = (int64_t)nl_base((int)i, E->nl_cap);
     for (int32_t k = 0; k < c; ++k) {
       const uint32_t e = nl[lb + (int64_t)nl_at(k)];
       const int64_t j = (int64_t)(e >> kNlShift) - base;

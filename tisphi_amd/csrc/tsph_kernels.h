@@ -35,12 +35,12 @@ __device__ __forceinline__ int xcd_block() {
     const int q = nb / kXcds, r = nb % kXcds, x = b % kXcds;
     return x * q + (x < r ? x : r) + b / kXcds;
   }
-  const int S = max(1, nb / (kXcds * kXcdStretches));  // blocks per stretch
-  const int nmain = nb - nb % (kXcds * S);
+  // blocks per stretch S = 2^sh: shifts instead of divisions
+  const int sh = max(0, 31 - __clz(nb / (kXcds * kXcdStretches)));
+  const int nmain = nb & ~((kXcds << sh) - 1);
   if (b >= nmain) return b;
   const int x = b % kXcds, i = b / kXcds;
-  const int j = i / S, o = i - j * S;
-  return (j * kXcds + x) * S + o;
+  return ((((i >> sh) * kXcds) + x) << sh) + (i & ((1 << sh) - 1));
 }
 __device__ __forceinline__ int wave_id() {
   return __builtin_amdgcn_readfirstlane((int)((xcd_block() * blockDim.x + threadIdx.x) >> 6));
@@ -55,6 +55,71 @@ __device__ __forceinline__ bool tile_thread(const KArgs& a, int& s, int& p) {
   p = t.y + (int)(threadIdx.x & 63);
   const SceneDev S = a.scenes[s];
   return p < S.pbase + S.n;
+}
+
+// What a tile holds, set by the list build: solid particles with pairs (or
+// rigid ones), boundary particles without, and flow or rigid particles.
+constexpr int kTileWall = 1, kTileBare = 2, kTileFlow = 4;
+
+// Particle p with the start of its list (any p below the capacity).
+template <bool NL>
+__device__ __forceinline__ Own own_of(const KArgs& a, int p) {
+  Own o;
+  o.P = a.cur.pos[p];
+  o.n = 0;
+  o.e0 = o.e1 = 0;
+  if (NL) {
+    o.n = a.w.nlc[p];
+    const uint32_t* __restrict__ li = a.w.nl + nl_base(p, a.nl_cap) + (threadIdx.x & 3);
+    o.e0 = li[0];
+    o.e1 = li[nl_at(4)];
+  }
+  return o;
+}
+
+// Work distribution of the pair passes: four waves per tile, a quad of lanes
+// per particle.  pred(s, p) says whether particle p has pairs to sum and, if
+// not, stores what it gets instead.  Tiles without any of `flags` are left
+// at once (the chain tile -> scene -> types of an idle wave costs more than
+// its work: 26 k of the 3D dam break's 71 k tiles are wall).  PACK: the
+// tile's particles with pairs are packed into groups of 16 first (boundary
+// tiles: 26 % of their particles have any).  Without lists (NL false) a lane
+// walks the stencil of its own particle.
+template <bool NL, bool PACK, class Pred, class Body>
+__device__ __forceinline__ void for_work(const KArgs& a, int flags, Pred&& pred, Body&& body) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int w = wave_id();
+  const int tile = NL ? w >> 2 : w, sub = w & 3;
+  const int2 t = a.tiles[tile];
+  if (NL && (a.w.tflag[tile] & flags) == 0) return;
+  if (t.x < 0) return;
+  const int s = __builtin_amdgcn_readfirstlane(t.x);
+  const int end = a.scenes[s].pbase + a.scenes[s].n;
+  if (!NL || !PACK) {
+    const int p = t.y + (NL ? sub * 16 + (lane >> 2) : lane);
+    if (p < end && pred(s, p, !NL || (lane & 3) == 0)) body(s, p, own_of<NL>(a, p));
+    return;
+  }
+  const int p = t.y + lane;
+  const bool work = p < end && pred(s, p, (lane >> 4) == sub);
+  const unsigned long long mask = __ballot(work);
+  const int cnt = __popcll(mask), g = sub * 16 + (lane >> 2);
+  if (sub * 16 >= cnt) return;
+  __shared__ uint8_t packed[kMaxBlock / 64][64];
+  uint8_t* __restrict__ pk = packed[threadIdx.x >> 6];
+  if (work)
+    pk[__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0))] =
+        (uint8_t)lane;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (g < cnt) {
+    const int q = t.y + (int)pk[g];
+    body(s, q, own_of<NL>(a, q));
+  }
+}
+// The lane that stores a particle's results.
+template <int L>
+__device__ __forceinline__ bool group_head() {
+  return L == 1 || threadIdx.x % L == 0;
 }
 
 __device__ __forceinline__ int32_t scene_shift(const KArgs& a, const SceneDev& S) {
@@ -406,44 +471,69 @@ __global__ __launch_bounds__(256) void k_rank_move(KArgs a, int move_vtmp, int m
 }
 
 // ============================================================ pair helpers
-struct Centre {
-  int cx, cy, cz;
-  float4 P;
-  int32_t shift;
-};
-__device__ __forceinline__ Centre centre_of(const KArgs& a, const SceneDev& S, int p) {
-  Centre c;
-  decode_cell(S, a.cur.cell[p], c.cx, c.cy, c.cz);
-  c.P = a.cur.pos[p];
-  c.shift = scene_shift(a, S);
-  return c;
-}
 // Walk the stencil around particle p's own (renormalised) cell.
 template <int DIM, class Fn>
-__device__ __forceinline__ void walk_c(const SceneDev& S, const KArgs& a, int p, const Centre& C,
+__device__ __forceinline__ void walk_c(const SceneDev& S, const KArgs& a, int p, const float4& P,
                                        Fn&& fn) {
-  walk<DIM>(S, a.w.start, a.cur.pos, C.shift, p, C.cx, C.cy, C.cz, C.cx, C.cy, C.cz, C.P.x, C.P.y,
-            C.P.z, fn);
+  int cx, cy, cz;
+  decode_cell(S, a.cur.cell[p], cx, cy, cz);
+  walk<DIM>(S, a.w.start, a.cur.pos, scene_shift(a, S), p, cx, cy, cz, cx, cy, cz, P.x, P.y, P.z, fn);
 }
 
-// Neighbours of p: the stored list when it is valid for this step, else the
-// stencil walk.  Both visit the same pairs in the same order.
-template <int DIM, bool NL, class Fn>
-__device__ __forceinline__ void neighbours(const SceneDev& S, const KArgs& a, int p,
-                                           const Centre& C, Fn&& fn) {
-  if (NL) {
-    const int n = a.w.nlc[p];
-    if (n <= a.nl_cap) {
-      for_list<DIM>(S, a.w.nl, n, a.nl_cap, a.cur.pos, p, C.P.x, C.P.y, C.P.z, fn);
-      return;
+// The stencil walk by a quad of lanes: lane q tests every fourth candidate
+// and the hits' terms are added in walk order, as in sum_list().
+template <int DIM, int NT, class Fn>
+__device__ __forceinline__ void walk_quad(const SceneDev& S, const KArgs& a, int i, const float4& P,
+                                          float (&acc)[NT], Fn&& fn) {
+  int cx, cy, cz;
+  decode_cell(S, a.cur.cell[i], cx, cy, cz);
+  const int32_t shift = scene_shift(a, S);
+  const int q = (int)threadIdx.x & 3;
+#pragma unroll 1
+  for (int k = 0; k < (DIM == 3 ? 27 : 9); ++k) {
+    const int dx = k / (DIM == 3 ? 9 : 3) - 1, dy = (DIM == 3 ? k / 3 : k) % 3 - 1, dz = DIM == 3 ? k % 3 - 1 : 0;
+    const int nx = cx + dx, ny = cy + dy, nz = cz + dz;
+    if (nx < 0 || nx >= S.gn[0] || ny < 0 || ny >= S.gn[1] || nz < 0 || nz >= S.gn[2]) continue;
+    const float bx = P.x + (float)(-dx) * S.g, by = P.y + (float)(-dy) * S.g;
+    const float bz = DIM == 3 ? P.z + (float)(-dz) * S.g : 0.0f;
+    const int32_t key = S.cbase + (nx * S.gn[1] + ny) * S.gn[2] + nz;
+    const int32_t je = a.w.start[key + 1] + shift;
+    for (int32_t j0 = a.w.start[key] + shift; j0 < je; j0 += 4) {
+      const int32_t j = j0 + q;
+      const float4 pj = a.cur.pos[min(j, je - 1)];
+      const float x = bx - pj.x, y = by - pj.y, z = DIM == 3 ? bz - pj.z : 0.0f;
+      const float r2 = fmaf(z, z, fmaf(y, y, x * x));
+      const bool hit = j < je && r2 < S.rs2 && j != i;
+      if (!__any(hit)) continue;
+      float t[NT];
+#pragma unroll
+      for (int c = 0; c < NT; ++c) t[c] = 0.0f;
+      if (hit) fn(j, x, y, z, r2, pj.w, t);
+      ordered_add<4>(acc, t);
     }
   }
-  walk_c<DIM>(S, a, p, C, fn);
 }
 
-// Appends of one particle's list, four entries per 16-byte store (a
-// lane's entries k..k+3, k % 4 == 0, are contiguous and 16-byte aligned):
-// a quarter of the write transactions of one store per entry.
+// acc[c] += term c of every neighbour of p: over the stored list when the
+// step has lists, by the stencil walk when p's is longer than nl_cap or there
+// are none.  All visit the same pairs in the same order.
+template <int DIM, bool NL, int L, int NT, class Fn>
+__device__ __forceinline__ void sum_pairs(const SceneDev& S, const KArgs& a, int p, const Own& o,
+                                          float (&acc)[NT], Fn&& fn) {
+  if (NL) {
+    if (o.n <= a.nl_cap) sum_list<DIM>(S, a.w.nl, a.nl_cap, a.cur.pos, p, o, acc, fn);
+    else walk_quad<DIM>(S, a, p, o.P, acc, fn);
+    return;
+  }
+  walk_c<DIM>(S, a, p, o.P, [&](int j, float x, float y, float z, float r2, float mVj, int) {
+    float t[NT];
+    fn(j, x, y, z, r2, mVj, t);
+    ordered_add<1>(acc, t);
+  });
+}
+
+// Appends of one particle's list, four entries per 16-byte store: a quarter
+// of the write transactions of one store per entry.
 struct ListAppender {
   uint32_t* __restrict__ li;
   int cap, n = 0;
@@ -451,46 +541,53 @@ struct ListAppender {
   // compare picks the slot)
   uint32_t b0 = 0, b1 = 0, b2 = 0;
   __device__ __forceinline__ void add(uint32_t e) {
-    // entries n-3..n go to nl_at(n - 3) = (n >> 4) * 1024 + (n & 12): a
-    // 32-bit byte offset (lists stay far below 4 GiB per particle)
-    if ((n & 3) == 3 && n < cap) {
-      const uint32_t off = (((uint32_t)n >> 4) << 12) | (((uint32_t)n << 2) & 48u);
-      *reinterpret_cast<uint4*>(reinterpret_cast<char*>(li) + off) = make_uint4(b0, b1, b2, e);
-    }
+    if ((n & 3) == 3 && n < cap) *reinterpret_cast<uint4*>(li + nl_at(n - 3)) = make_uint4(b0, b1, b2, e);
     b0 = b1;
     b1 = b2;
     b2 = e;
     ++n;
   }
-  // the last 1-3 entries
-  __device__ __forceinline__ int finish() {
+  // the last 1-3 entries, padded with the null particle's
+  __device__ __forceinline__ int finish(uint32_t pad) {
     const int r = n & 3;
     if (n <= cap && r > 0) {
-      const int k = n - r;
-      if (r == 3) li[nl_at(k)] = b0;
-      if (r >= 2) li[nl_at(n - 2)] = b1;
-      li[nl_at(n - 1)] = b2;
+      const uint4 v = r == 3 ? make_uint4(b0, b1, b2, pad)
+                             : (r == 2 ? make_uint4(b1, b2, pad, pad) : make_uint4(b2, pad, pad, pad));
+      *reinterpret_cast<uint4*>(li + nl_at(n - r)) = v;
     }
     return n;
   }
 };
 
-// neighbours() with the scene's kernel type as a compile-time tag: fn gets
+// sum_pairs() with the scene's kernel type as a compile-time tag: fn gets
 // KTag<1> (Wendland C2) or KTag<0> (cubic) first, so its kernel values
 // come from kernel_W_t / kernel_gradfac_t (straight-line code).
 template <int K>
 struct KTag {
   static constexpr int v = K;
 };
-template <int DIM, bool NL, class Fn>
-__device__ __forceinline__ void neighbours_k(const SceneDev& S, const KArgs& a, int p,
-                                             const Centre& C, Fn&& fn) {
+template <int DIM, bool NL, int L, int NT, class Fn>
+__device__ __forceinline__ void sum_pairs_k(const SceneDev& S, const KArgs& a, int p,
+                                            const Own& o, float (&acc)[NT], Fn&& fn) {
   if (S.kernel == 1)
-    neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj,
-                                        int code) { fn(KTag<1>{}, j, x, y, z, r2, mVj, code); });
+    sum_pairs<DIM, NL, L>(S, a, p, o, acc, [&](int j, float x, float y, float z, float r2, float mVj,
+                                               float (&t)[NT]) { fn(KTag<1>{}, j, x, y, z, r2, mVj, t); });
   else
-    neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj,
-                                        int code) { fn(KTag<0>{}, j, x, y, z, r2, mVj, code); });
+    sum_pairs<DIM, NL, L>(S, a, p, o, acc, [&](int j, float x, float y, float z, float r2, float mVj,
+                                               float (&t)[NT]) { fn(KTag<0>{}, j, x, y, z, r2, mVj, t); });
+}
+// on ? x : +0 as a select (the guard keeps the compiler from forming x in a
+// branch, which also keeps the quad's additions from reading it through
+// their DPP operand).
+__device__ __forceinline__ float term_if(bool on, float x) {
+  asm("" : "+v"(x));
+  return on ? x : 0.0f;
+}
+// A term that no neighbour of another kind adds: +0 leaves a sum's bits.
+template <int NT>
+__device__ __forceinline__ void no_terms(float (&t)[NT]) {
+#pragma unroll
+  for (int c = 0; c < NT; ++c) t[c] = 0.0f;
 }
 
 // Whether any of the 3^DIM stencil cells around (cx, cy, cz) holds a flow
@@ -516,247 +613,358 @@ __device__ __forceinline__ bool flow_in_reach(const SceneDev& S, const uint8_t* 
   return false;
 }
 
+// The tile's flags (every lane of the wave that owns it; n: list length, < 0
+// for a lane without a particle).
+__device__ __forceinline__ void set_tile_flags(const KArgs& a, int tile, int n, bool bdy, bool rig) {
+  const bool some = n >= 0;
+  const int f = (__any(some && (rig || (bdy && n > 0))) ? kTileWall : 0) |
+                (__any(some && bdy && n == 0) ? kTileBare : 0) | (__any(some && !bdy) ? kTileFlow : 0);
+  if ((threadIdx.x & 63) == 0) a.w.tflag[tile] = f;
+}
+
 // Neighbour-list build: one stencil walk per particle per step, recording
 // (j << 6 | stencil code) for every neighbour; boundary particles keep only
 // their flow neighbours (the only ones their passes read).  The candidate
 // loop does nothing else, so the rarely taken append is the only divergent
 // work in it.
 template <int DIM>
-__global__ __launch_bounds__(256) void k_nl_build(KArgs a, int use_cflow, int cull) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
+__device__ __forceinline__ int nl_build_one(const KArgs& a, int s, int p, bool bdy, bool rig, int use_cflow,
+                                            int cull) {
   const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+  const float4 P = a.cur.pos[p];
   const int8_t* __restrict__ type = a.cur.type;
-  // Boundary particles record flow neighbours only; rigid ones flow and
-  // rigid neighbours (the XSPH sum of a rigid particle runs over rigid
-  // ones); flow particles record all.
-  const bool bdy = is_bdy(type[p]), rig = type[p] == kRigid;
   const int cap = a.nl_cap;
   uint32_t* __restrict__ li = a.w.nl + nl_base(p, cap);
+  int cx, cy, cz;
+  decode_cell(S, a.cur.cell[p], cx, cy, cz);
   // A boundary particle only records flow neighbours: none can exist if
   // no stencil cell holds a flow particle.
-  if (bdy && use_cflow && !flow_in_reach<DIM>(S, a.w.cflow, C.cx, C.cy, C.cz)) {
-    a.w.nlc[p] = 0;
-    return;
-  }
+  if (bdy && use_cflow && !flow_in_reach<DIM>(S, a.w.cflow, cx, cy, cz)) return 0;
   ListAppender ap{li, cap};
   auto rec = [&](int j, float x, float y, float z, float r2, float mVj, int code) {
     if ((bdy && !is_flow(type[j])) || (rig && !(is_flow(type[j]) || type[j] == kRigid))) return;
     ap.add(nl_entry(j, code));
   };
   if (cull)
-    walk<DIM, true>(S, a.w.start, a.cur.pos, C.shift, p, C.cx, C.cy, C.cz, C.cx, C.cy, C.cz, C.P.x,
-                    C.P.y, C.P.z, rec);
+    walk<DIM, true>(S, a.w.start, a.cur.pos, scene_shift(a, S), p, cx, cy, cz, cx, cy, cz, P.x, P.y,
+                    P.z, rec);
   else
-    walk_c<DIM>(S, a, p, C, rec);
-  a.w.nlc[p] = ap.finish();
+    walk_c<DIM>(S, a, p, P, rec);
+  return ap.finish(a.nl_pad);
+}
+template <int DIM>
+__global__ __launch_bounds__(256) void k_nl_build(KArgs a, int use_cflow, int cull) {
+  const int w = wave_id();
+  if (a.tiles[w].x < 0) return;
+  int s, p, n = -1;
+  bool bdy = false, rig = false;
+  if (tile_thread(a, s, p)) {
+    // Boundary particles record flow neighbours only; rigid ones flow and
+    // rigid neighbours (the XSPH sum of a rigid particle runs over rigid
+    // ones); flow particles record all.
+    bdy = is_bdy(a.cur.type[p]);
+    rig = a.cur.type[p] == kRigid;
+    n = nl_build_one<DIM>(a, s, p, bdy, rig, use_cflow, cull);
+    a.w.nlc[p] = n;
+  }
+  set_tile_flags(a, w, n, bdy, rig);
 }
 
 // ------------------------------------------------ LDS-staged list build
-// The same list build with the candidates read from LDS.  One wave per
-// workgroup owns one tile.  Cell keys run (row, fast) with the fast axis z
-// in 3D and y in 2D; a tile's particles usually share one row, so for each
-// row offset (dx, dy in 3D; dx in 2D) the neighbour cells of all its lanes
-// are consecutive keys and their particles one contiguous range.  The wave
-// copies that range (coalesced, at most STAGE particles: the cell tile) into
-// LDS and every lane walks its own three fast-axis cells there, in the order
-// of walk() (same pairs, same order, same values).  A tile spanning two
-// rows, or a larger range, reads global memory instead.  STAGE (128, 256 or
-// 512 candidates: 2, 4 or 8 KiB of LDS per wave) trades how often a window
-// fits against how many waves a CU holds; the engine's cell-tile setting
-// picks it.
+// The same lists from candidates staged in LDS.  A workgroup of three waves
+// owns one tile; wave v takes the stencil's dx = v - 1 plane for the tile's
+// 64 particles, a lane each, so a tile's work is three independent pieces
+// (a small scene has few tiles).  Cell keys run (row, fast) with the fast
+// axis z in 3D and y in 2D.  The lanes of one row (a tile holds one or two)
+// have their candidates of one row offset (dy in 3D) in one contiguous
+// particle range, which the wave copies into LDS (at most STAGE candidates,
+// the cell tile; a larger window is read from global memory).
+//
+// Test: every lane walks its own three fast-axis cells there in the order of
+// walk() and shifts one bit per candidate, hit or not, into a word per 32:
+// 8 vector instructions per candidate (6 in 2D) and nothing else in the
+// loop, so no lane waits for another's append.  Words with a hit go to LDS.
+// Record: when all three waves have counted, each knows where its hits start
+// in the list; a lane pops one hit per turn from its words, all lanes in the
+// same turn, so four turns fill one aligned quad of every list and a wave's
+// store is a contiguous kilobyte.  A quad that holds hits of two waves is
+// written by the first of them.
 constexpr int kStageDefault = 256;
+constexpr int kBuildWaves = 3;
+template <int DIM>
+constexpr int kHitWords = DIM == 3 ? 10 : 4;  // per lane and wave: a word per cell, 1 to spare
 
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_xor(v, d, 64);
-    v = u < v ? u : v;
+// Hit words of one lane in list order: rows [v NW, v NW + nw_v) of wave v.
+template <int NW>
+struct HitWords {
+  const uint2 (*__restrict__ words)[64];
+  const int32_t (*__restrict__ count)[64];  // words << 16 | hits, per wave
+  int lane, v, k, end;
+  uint32_t w = 0, eb = 0;
+  __device__ __forceinline__ HitWords(const uint2 (*wd)[64], const int32_t (*ct)[64], int ln, int wave)
+      : words(wd), count(ct), lane(ln), v(wave), k(wave * NW), end(wave * NW + (ct[wave][ln] >> 16)) {}
+  // the next hit's entry; at least one is left in this wave's words
+  __device__ __forceinline__ uint32_t pop() {
+    if (w == 0) {
+      const uint2 x = words[k++][lane];
+      w = x.x;
+      eb = x.y;
+    }
+    const int b = __builtin_clz(w);
+    w ^= 0x80000000u >> b;
+    return eb + ((uint32_t)b << kNlShift);
   }
-  return v;
-}
-__device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_xor(v, d, 64);
-    v = u > v ? u : v;
+  // as pop(), going on to the next waves' words; `pad` past the last
+  __device__ __forceinline__ uint32_t pop_on(uint32_t pad) {
+    while (w == 0 && k == end && v < kBuildWaves - 1) {
+      ++v;
+      k = v * NW;
+      end = k + (count[v][lane] >> 16);
+    }
+    return (w == 0 && k == end) ? pad : pop();
   }
-  return v;
-}
+};
 
 template <int DIM, int STAGE>
-__global__ __launch_bounds__(64) void k_nl_build_lds(KArgs a, int use_cflow, int cull) {
-  __shared__ float4 sp[STAGE];
-  const int w = __builtin_amdgcn_readfirstlane((int)xcd_block());
-  const int2 t = a.tiles[w];
+__global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build_lds(KArgs a, int use_cflow) {
+  constexpr int NW = kHitWords<DIM>;
+  __shared__ float4 stage[kBuildWaves][STAGE + 32];  // read up to 31 past the window
+  __shared__ uint2 words[kBuildWaves * NW][64];
+  __shared__ int32_t count[kBuildWaves][64];  // words << 16 | hits; < 0: more words than fit
+  __shared__ int32_t flow[kBuildWaves][64];   // a flow particle in the wave's reach of the lane
+  const int tile = __builtin_amdgcn_readfirstlane(xcd_block());
+  const int2 t = a.tiles[tile];
   if (t.x < 0) return;  // unused tile: the whole workgroup leaves
   const int s = __builtin_amdgcn_readfirstlane(t.x);
-  const int lane = (int)threadIdx.x;
-  const int p = t.y + lane;
+  const int v = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = (int)(threadIdx.x & 63), dx = v - 1;
   const SceneDev S = a.scenes[s];
   const int8_t* __restrict__ type = a.cur.type;
   const float4* __restrict__ pos = a.cur.pos;
   const int32_t* __restrict__ start = a.w.start;
-  const int cap = a.nl_cap;
   const int32_t shift = scene_shift(a, S);
-  const int gx = S.gn[0], gy = S.gn[1], gz = S.gn[2];
-  bool act = p < S.pbase + S.n;
-  int cx = 0, cy = 0, cz = 0, key = 0;
+  const int gx = S.gn[0], gy = DIM == 3 ? S.gn[1] : 1;  // rows: gx * gy
+  const int gf = DIM == 3 ? S.gn[2] : S.gn[1];          // cells of a row
+  const int p = t.y + lane;
+  const bool live = p < S.pbase + S.n;
+  int row = -1, f = 0, tp = 0;
   float4 P = make_float4(0.f, 0.f, 0.f, 0.f);
-  bool bdy = false, rig = false;
-  if (act) {
+  if (live) {
     const int32_t c = a.cur.cell[p];
-    decode_cell(S, c, cx, cy, cz);
-    key = S.cbase + c;
+    row = c / gf;
+    f = c - row * gf;
     P = pos[p];
-    bdy = is_bdy(type[p]);
-    rig = type[p] == kRigid;
+    tp = type[p];
   }
-  if (act && bdy && use_cflow && !flow_in_reach<DIM>(S, a.w.cflow, cx, cy, cz)) {
-    // as in k_nl_build: no flow cell in reach, no neighbours to record
-    a.w.nlc[p] = 0;
-    act = false;
-  }
-  uint32_t* __restrict__ li = a.w.nl + nl_base(act ? p : t.y, cap);
-  ListAppender ap{li, cap};
-  auto rec = [&](int j, float x, float y, float z, float r2, float mVj, int code) {
-    if ((bdy && !is_flow(type[j])) || (rig && !(is_flow(type[j]) || type[j] == kRigid))) return;
-    ap.add(nl_entry(j, code));
-  };
-  const float wmin = bdy ? 2.0f : (rig ? 1.0f : 0.0f);  // staged-record filter
-  const int row = DIM == 3 ? cx * gy + cy : cx;
-  const int rmin = wave_min(act ? row : INT32_MAX), rmax = wave_max(act ? row : INT32_MIN);
-  if (rmin > rmax) return;  // no lane left to walk (wave-uniform)
-  if (rmin != rmax) {
-    // two rows: each lane walks global memory
-    if (act) {
-      if (cull) walk<DIM, true>(S, start, pos, shift, p, cx, cy, cz, cx, cy, cz, P.x, P.y, P.z, rec);
-      else walk<DIM>(S, start, pos, shift, p, cx, cy, cz, cx, cy, cz, P.x, P.y, P.z, rec);
-      a.w.nlc[p] = ap.finish();
-    }
-    return;
-  }
-  // One row: rx (and ry in 3D) are the same for every active lane.  Walk
-  // order dx, dy, dz as in walk(); the row offsets (dx, dy in 3D; dx in 2D)
-  // are wave-uniform, and for each the three fast-axis neighbour cells of
-  // all lanes are one contiguous particle range, staged once.
-  const int rx = DIM == 3 ? rmin / gy : rmin;
-  const int ry = DIM == 3 ? rmin - rx * gy : 0;
-  const int f = DIM == 3 ? cz : cy;  // fast coordinate of the lane's cell
-  const int gf = DIM == 3 ? gz : gy;
-  const int flo = f > 0 ? -1 : 0, fhi = f < gf - 1 ? 1 : 0;
+  // boundary particles record flow neighbours only, rigid ones flow and rigid
+  // neighbours (the XSPH sum of a rigid particle runs over rigid ones)
+  const bool bdy = live && is_bdy(tp), rig = live && tp == kRigid;
+  const int need = bdy ? 2 : (rig ? 1 : 0);
+  float4* __restrict__ sp = stage[v];
+  uint2(*__restrict__ wd)[64] = words + v * NW;
+  int nw = 0, h = 0;
+  unsigned long long todo = __ballot(live);
 #pragma unroll 1
-  for (int dx = -1; dx <= 1; ++dx) {
-    if (rx + dx < 0 || rx + dx >= gx) continue;
+  while (todo) {
+    // the lanes of the next row; sorted by cell, so they are consecutive
+    const int l0 = __builtin_ctzll(todo);
+    const int R = __builtin_amdgcn_readlane(row, l0);
+    bool act = row == R;
+    const unsigned long long mine = __ballot(act);
+    todo &= ~mine;
+    const int l1 = 63 - __builtin_clzll(mine);
+    const int wlo = max(__builtin_amdgcn_readlane(f, l0) - 1, 0);
+    const int whi = min(__builtin_amdgcn_readlane(f, l1) + 1, gf - 1);
+    const int rx = DIM == 3 ? R / gy : R, ry = DIM == 3 ? R - rx * gy : 0;
+    const bool inx = rx + dx >= 0 && rx + dx < gx;
+    // A boundary particle records nothing if no stencil cell holds a flow
+    // particle.  The flags of a row offset's window are one load; each lane
+    // picks its three from the wave's mask.
+    if (use_cflow && __any(act && bdy)) {
+      bool reach = whi - wlo >= 64;
+      if (inx && !reach) {
+#pragma unroll
+        for (int dy = (DIM == 3 ? -1 : 0); dy <= (DIM == 3 ? 1 : 0); ++dy) {
+          if (ry + dy < 0 || ry + dy >= gy) continue;
+          const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy) * gf + wlo;
+          const unsigned long long m = __ballot(lane <= whi - wlo && a.w.cflow[nk + min(lane, whi - wlo)] != 0);
+          const int sh = act ? f - 1 - wlo : 0;  // bit of the lane's first cell
+          reach = reach || ((sh >= 0 ? m >> sh : m << 1) & 7ull) != 0;
+        }
+      }
+      flow[v][lane] = reach;
+      __syncthreads();
+      act = act && (!bdy || flow[0][lane] | flow[1][lane] | flow[2][lane]);
+      __syncthreads();  // before the next row's flags
+    }
+    if (!inx || !__any(act)) continue;
+    const bool filter = __any(act && need != 0);
     const float bx = P.x + (float)(-dx) * S.g;
-    const float ax = dx < 0 ? P.x : (dx > 0 ? S.g - P.x : 0.0f);
 #pragma unroll 1
     for (int dy0 = (DIM == 3 ? -1 : 0); dy0 <= (DIM == 3 ? 1 : 0); ++dy0) {
-      if (DIM == 3 && (ry + dy0 < 0 || ry + dy0 >= gy)) continue;
-      // key of the lane's neighbour cell at fast offset 0 in this row offset
-      const int rkey = key + (DIM == 3 ? (dx * gy + dy0) * gz : dx * gy);
-      const int klo = wave_min(act ? rkey + flo : INT32_MAX);
-      const int khi = wave_max(act ? rkey + fhi : INT32_MIN);
-      const int32_t jlo = start[klo] + shift;
-      const int32_t cnt = start[khi + 1] + shift - jlo;
-      const bool staged = cnt <= STAGE;  // wave-uniform
-      if (staged) {
-        __syncthreads();  // the previous row offset's reads are done
-        // w = 2 for a flow particle (the only neighbours a boundary lane
-        // records), 1 for a rigid one (a rigid lane records both), 0
-        // otherwise: the lane's filter is one compare, w >= wmin, and needs
-        // no global load per hit
-        for (int q = lane; q < cnt; q += 64) {
-          float4 v = pos[jlo + q];
-          const int tq = type[jlo + q];
-          v.w = is_flow(tq) ? 2.0f : (tq == kRigid ? 1.0f : 0.0f);
-          sp[q] = v;
-        }
-        __syncthreads();
+      if (ry + dy0 < 0 || ry + dy0 >= gy) continue;
+      const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy0) * gf;
+      const int32_t jlo = start[nk + wlo] + shift, cnt = start[nk + whi + 1] + shift - jlo;
+      if (cnt == 0) continue;
+      if (cnt > 4 * STAGE || __any(nw > NW)) {  // dense: walked below
+        nw = NW + 1;
+        break;
       }
-#pragma unroll 1
-      for (int df = -1; df <= 1; ++df) {
-        const int dy = DIM == 3 ? dy0 : df;
-        const int dz = DIM == 3 ? df : 0;
-        bool ok = act && f + df >= 0 && f + df < gf;
-        const float by = P.y + (float)(-dy) * S.g;
-        const float ay = dy < 0 ? P.y : (dy > 0 ? S.g - P.y : 0.0f);
-        if (ok && cull) {  // as in walk()
-          const float az = DIM == 3 ? (dz < 0 ? P.z : (dz > 0 ? S.g - P.z : 0.0f)) : 0.0f;
-          ok = !(fmaf(az, az, fmaf(ay, ay, ax * ax)) > S.rs2c);
+      // the lane's cells: candidates [c[k], c[k + 1]) at fast offset k - 1
+      int c[4] = {0, 0, 0, 0};
+      if (act) {
+        c[1] = start[nk + f] + shift - jlo;
+        c[2] = start[nk + f + 1] + shift - jlo;
+        c[0] = f > 0 ? start[nk + f - 1] + shift - jlo : c[1];
+        c[3] = f < gf - 1 ? start[nk + f + 2] + shift - jlo : c[2];
+      }
+      const bool staged = cnt <= STAGE;
+      if (staged) {
+        __builtin_amdgcn_wave_barrier();  // the last row offset's reads are done (one wave, in order)
+        for (int q = lane; q < cnt; q += 64) {
+          float4 r = pos[jlo + q];
+          const int tq = type[jlo + q];
+          r.w = is_flow(tq) ? 2.0f : (tq == kRigid ? 1.0f : 0.0f);
+          sp[q] = r;
         }
-        if (!ok) continue;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int dy = DIM == 3 ? dy0 : k - 1, dz = DIM == 3 ? k - 1 : 0;
+        const float by = P.y + (float)(-dy) * S.g;
         const float bz = DIM == 3 ? P.z + (float)(-dz) * S.g : 0.0f;
-        const int nkey = rkey + df;
-        const int code = ((dx + 1) << 4) | ((dy + 1) << 2) | (dz + 1);
-        const int32_t jb = start[nkey] + shift, je = start[nkey + 1] + shift;
-        auto cand = [&](int32_t j, const float4& pj) {
-          const float x = bx - pj.x;
-          const float y = by - pj.y;
-          const float z = DIM == 3 ? bz - pj.z : 0.0f;
-          const float r2 = fmaf(z, z, fmaf(y, y, x * x));
-          if (r2 < S.rs2 && j != p) rec(j, x, y, z, r2, pj.w, code);
+        // the sign bit of |r2| - rs2 (a NaN's is clear) is the hit
+        auto dist = [&](const float4& r) {
+          const float x = bx - r.x, y = by - r.y;
+          float r2;
+          if (DIM == 3) {
+            const float z = bz - r.z;
+            r2 = fmaf(z, z, fmaf(y, y, x * x));
+          } else {
+            r2 = fmaf(y, y, x * x);
+          }
+          return __float_as_uint(fabsf(r2) - S.rs2);
         };
-        if (staged) {
-          // One induction variable, the LDS byte offset, kept opaque so
-          // the compiler derives no second one from the own-cell test; the
-          // particle index is formed only on a hit.  p is a candidate of the
-          // own cell only (wave-uniform offset 0), so only that cell's loop
-          // carries the test, and the record is read whole (one 16-byte LDS
-          // read) so the flow flag costs no second read on the hit path:
-          // 10 vector instructions per rejected candidate instead of 12.
-          // The entry of the staged record at byte offset o (a multiple of
-          // 16) is nl_entry(jlo + o / 16, code) = (o << 2) + kbase: one
-          // shift-add on the hit path.
-          const uint32_t oend = (uint32_t)(je - jlo) * 16u;
-          const uint32_t kbase = nl_entry(jlo, code);
-          const char* __restrict__ sb = reinterpret_cast<const char*>(sp);
-          auto scan = [&](uint32_t skip, auto own) {
+        auto shift_in = [&](uint32_t w, const float4& r) {
+          return __builtin_amdgcn_alignbit(w, dist(r), 31);
+        };
+        // as shift_in, for candidates the lane records (kind >= need) only
+        auto shift_in_kind = [&](uint32_t w, const float4& r) {
+          return __builtin_amdgcn_alignbit(w, dist(r) & ~__float_as_uint(r.w - (float)need), 31);
+        };
+        int lo = c[k];
+        const int hi = c[k + 1];
 #pragma unroll 1
-            for (uint32_t o = (uint32_t)(jb - jlo) * 16u; o < oend; o += 16u) {
-              asm volatile("" : "+v"(o));
-              float4 pj = *reinterpret_cast<const float4*>(sb + o);
-              asm volatile("" : "+v"(pj.w));  // one 16-byte read per candidate
-              const float x = bx - pj.x;
-              const float y = by - pj.y;
-              const float z = DIM == 3 ? bz - pj.z : 0.0f;
-              const float r2 = fmaf(z, z, fmaf(y, y, x * x));
-              if (r2 < S.rs2 && (!decltype(own)::value || o != skip) && pj.w >= wmin)
-                ap.add((o << 2) + kbase);
+        for (; __any(lo < hi); lo += 32) {
+          const int m = min(hi - lo, 32);  // <= 0 for a lane that is done
+          uint32_t w = 0;
+          if (staged) {
+            const float4* __restrict__ q = sp + min(lo, cnt);
+            int done = 0;
+            if (!filter) {
+#pragma unroll 1
+              do {
+                const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
+                w = shift_in(shift_in(shift_in(shift_in(w, r0), r1), r2), r3);
+                done += 4;
+                q += 4;
+              } while (__any(done < m));
+            } else {
+#pragma unroll 1
+              do {
+                const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
+                w = shift_in_kind(shift_in_kind(shift_in_kind(shift_in_kind(w, r0), r1), r2), r3);
+                done += 4;
+                q += 4;
+              } while (__any(done < m));
             }
-          };
-          if (dx == 0 && dy == 0 && dz == 0)
-            scan((uint32_t)(p - jlo) * 16u, std::true_type{});
-          else
-            scan(0u, std::false_type{});
-        } else {
-          for (int32_t j = jb; j < je; ++j) cand(j, pos[j]);
+            w <<= (32 - done) & 31;
+          } else {
+            for (int i = 0; i < m; ++i) {
+              float4 r = pos[jlo + lo + i];
+              const int tj = type[jlo + lo + i];
+              r.w = is_flow(tj) ? 2.0f : (tj == kRigid ? 1.0f : 0.0f);
+              w |= shift_in_kind(0, r) << (31 - i);
+            }
+          }
+          // candidates past the lane's cell, and the particle itself
+          if (m < 32) w &= m > 0 ? ~(0xFFFFFFFFu >> m) : 0u;
+          if (dx == 0 && dy == 0 && dz == 0) {
+            const int i = p - jlo - lo;
+            if (i >= 0 && i < 32) w &= ~(0x80000000u >> i);
+          }
+          if (w) {
+            if (nw < NW)
+              wd[nw][lane] = make_uint2(w, nl_entry(jlo + lo, ((dx + 1) << 4) | ((dy + 1) << 2) | (dz + 1)));
+            ++nw;
+            h += __popc(w);
+          }
         }
       }
     }
   }
-  if (act) a.w.nlc[p] = ap.finish();
+  count[v][lane] = nw > NW ? INT32_MIN : (nw << 16 | h);
+  __syncthreads();
+  const int c0 = count[0][lane], c1 = count[1][lane], c2 = count[2][lane];
+  const int cap = a.nl_cap;
+  if (__any((c0 | c1 | c2) < 0)) {
+    // more hit words than fit (cells of over 32 particles): the first wave walks
+    if (v != 0) return;
+    int n = -1;
+    if (live) a.w.nlc[p] = n = nl_build_one<DIM>(a, s, p, bdy, rig, use_cflow, 0);
+    set_tile_flags(a, tile, n, bdy, rig);
+    return;
+  }
+  const int h0 = c0 & 0xFFFF, h1 = c1 & 0xFFFF, n = h0 + h1 + (c2 & 0xFFFF);
+  if (v == 0) {
+    if (live) a.w.nlc[p] = n;
+    set_tile_flags(a, tile, live ? n : -1, bdy, rig);
+  }
+  if (n > cap) return;  // walked by the pair passes
+  // this wave's hits are [o, o + h) of the list: the quads that start there
+  const int o = (v > 0 ? h0 : 0) + (v > 1 ? h1 : 0), skip = -o & 3;
+  if (h <= skip) return;
+  uint32_t* __restrict__ li = a.w.nl + nl_base(p, cap) + nl_at(o + skip);
+  HitWords<NW> hw(words, count, lane, v);
+  for (int i = 0; i < skip; ++i) hw.pop();
+  int left = h - skip;
+  for (; left >= 4; left -= 4) {
+    const uint32_t e0 = hw.pop(), e1 = hw.pop(), e2 = hw.pop(), e3 = hw.pop();
+    *reinterpret_cast<uint4*>(li) = make_uint4(e0, e1, e2, e3);
+    li += nl_at(4);
+  }
+  if (left > 0) {
+    const uint32_t e0 = hw.pop(), e1 = hw.pop_on(a.nl_pad), e2 = hw.pop_on(a.nl_pad), e3 = hw.pop_on(a.nl_pad);
+    *reinterpret_cast<uint4*>(li) = make_uint4(e0, e1, e2, e3);
+  }
 }
 
 // calc_CSPM_f (solver_sph_base.py:386-398) over the recorded lists.
 template <int DIM>
 __global__ __launch_bounds__(256) void k_shepard_list(KArgs a, int skip_fluid) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (skip_fluid && a.cur.type[p] == kFluid) return;  // formed by the fluid pass
-  const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
   const int8_t* __restrict__ type = a.cur.type;
-  float sum = 0.0f;
-  neighbours_k<DIM, true>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                  float mVj, int) {
-    // straight-line: a non-flow neighbour adds +0 (the sum's bits stay)
-    const bool fl = is_flow(type[j]);
-    const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
-    sum += fl ? mVj * w : 0.0f;
-  });
-  a.w.cspm[p] = sum != 0.0f ? 1.0f / sum : 1.0f;
+  for_work<true, false>(
+      a, ~0,
+      [&](int, int p, bool mine) {
+        if (skip_fluid && type[p] == kFluid) return false;  // formed by the fluid pass
+        if (a.w.nlc[p] != 0) return true;
+        if (mine) a.w.cspm[p] = 1.0f;
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        float acc[1] = {0.0f};
+        sum_pairs_k<DIM, true, kLanes>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z,
+                                                                       float r2, float mVj, float (&t)[1]) {
+          // straight-line: a non-flow neighbour adds +0 (the sum's bits stay)
+          const bool fl = is_flow(type[j]);
+          const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
+          t[0] = term_if(fl, mVj * w);
+        });
+        if (group_head<kLanes>()) a.w.cspm[p] = acc[0] != 0.0f ? 1.0f / acc[0] : 1.0f;
+      });
 }
 
 // calc_CSPM_L (solver_sph_base.py:400-423) for scenes with
@@ -769,32 +977,42 @@ __global__ __launch_bounds__(256) void k_shepard_list(KArgs a, int skip_fluid) {
 // get a zero gradient.
 template <int DIM, bool NL>
 __global__ __launch_bounds__(256) void k_cspm_L(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  const SceneDev S = a.scenes[s];
-  if (S.kcorr == 0) return;
-  const float one = S.kcorr == 1 ? 1.f : 0.f;
-  float M[9] = {one, 0.f, 0.f, 0.f, one, 0.f, 0.f, 0.f, one};
+  constexpr int L = NL ? kLanes : 1;
   const int8_t* __restrict__ type = a.cur.type;
-  const int ti = type[p];
-  if (S.kcorr == 1 && is_flow(ti)) {
-    const Centre C = centre_of(a, S, p);
-    float L[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-    neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                          float mVj, int) {
-      if (type[j] != ti) return;
-      const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
-      const float g[3] = {f * x, f * y, f * z};
-      const float c[3] = {mVj * (-x), mVj * (-y), mVj * (-z)};
+  auto store = [&](int p, const float M[9]) {
 #pragma unroll
-      for (int aa = 0; aa < 3; ++aa)
+    for (int c = 0; c < 9; ++c) a.w.Lc[(size_t)c * a.stride + p] = M[c];
+  };
+  for_work<NL, false>(
+      a, ~0,
+      [&](int s, int p, bool mine) {
+        const int kc = a.scenes[s].kcorr;
+        if (kc == 0) return false;
+        if (kc == 1 && is_flow(type[p])) return true;
+        if (!mine) return false;
+        const float one = kc == 1 ? 1.f : 0.f;
+        const float M[9] = {one, 0.f, 0.f, 0.f, one, 0.f, 0.f, 0.f, one};
+        store(p, M);
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        const int ti = type[p];
+        float M[9] = {1.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f, 0.f, 1.f};
+        float acc[9] = {};
+        sum_pairs_k<DIM, NL, L>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                                float mVj, float (&t)[9]) {
+          const bool same = type[j] == ti;
+          const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
+          const float g[3] = {f * x, f * y, f * z};
+          const float c[3] = {mVj * (-x), mVj * (-y), mVj * (-z)};
 #pragma unroll
-        for (int bb = 0; bb < 3; ++bb) L[aa][bb] += c[aa] * g[bb];
-    });
-    corr_invert<DIM>(L, S.eps, M);
-  }
-#pragma unroll
-  for (int c = 0; c < 9; ++c) a.w.Lc[(size_t)c * a.stride + p] = M[c];
+          for (int k = 0; k < 9; ++k) t[k] = term_if(same, c[k / 3] * g[k % 3]);
+        });
+        const float Lm[3][3] = {{acc[0], acc[1], acc[2]}, {acc[3], acc[4], acc[5]}, {acc[6], acc[7], acc[8]}};
+        corr_invert<DIM>(Lm, S.eps, M);
+        if (group_head<L>()) store(p, M);
+      });
 }
 
 // =================================================================== Shepard
@@ -805,10 +1023,10 @@ __global__ __launch_bounds__(256) void k_shepard(KArgs a, int skip_fluid) {
   if (!tile_thread(a, s, p)) return;
   if (skip_fluid && a.cur.type[p] == kFluid) return;  // formed by the fluid pass
   const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+  const float4 P = a.cur.pos[p];
   const int8_t* __restrict__ type = a.cur.type;
   float sum = 0.0f;
-  walk_c<DIM>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj, int) {
+  walk_c<DIM>(S, a, p, P, [&](int j, float x, float y, float z, float r2, float mVj, int) {
     if (is_flow(type[j])) sum += mVj * kernel_W(S, pair_dist(r2));
   });
   a.w.cspm[p] = sum != 0.0f ? 1.0f / sum : 1.0f;
@@ -853,57 +1071,72 @@ __global__ __launch_bounds__(256) void k_wc_eos(KArgs a) {  // solver_sph_wc.py:
 // With SHEP the same walk first forms the particle's Shepard sum
 // (calc_CSPM_f, solver_sph_base.py:386-398: flow neighbours, list order),
 // which the fused step then leaves out of the Shepard pass: bitwise equal.
-template <int DIM, bool NL, bool SHEP>
-__global__ __launch_bounds__(256) void k_wc_bdy(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (!is_solid(a.cur.type[p])) return;  // boundary and rigid (solver_sph_wc.py:90-103)
-  const SceneDev S = a.scenes[s];
-  const int8_t* __restrict__ type = a.cur.type;
-  const float4* __restrict__ vtmp = a.cur.vtmp;
-  const float* __restrict__ pr = a.w.p;
-  const float gy = S.grav[1];
-  // Most dummy particles have no flow particle in reach (an empty list):
-  // their sums stay zero, so they skip the centre and the walk and only
-  // form the extrapolation below (the same values the empty walk gives).
+// acc: sums of v (3), p and, with SHEP, W.
+template <bool SHEP>
+__device__ __forceinline__ void wc_wall_store(const KArgs& a, const SceneDev& S, int p, const float* acc) {
   const float4 v = a.cur.vel[p];
-  const float cs_in = SHEP ? 1.0f : a.w.cspm[p];
-  float svx = 0.f, svy = 0.f, svz = 0.f, sp = 0.f, shep = 0.f;
-  if (!NL || a.w.nlc[p] != 0) {
-    const Centre C = centre_of(a, S, p);
-    // Straight-line pair terms (a non-flow neighbour adds +0, which leaves
-    // every sum's bits unchanged: the sums start at +0 and never become -0
-    // in round-to-nearest), so the loads of a batch of neighbours are
-    // issued together instead of one branch at a time.
-    neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                    float mVj, int) {
-      const bool fl = is_flow(type[j]);
-      const float4 vj = vtmp[j];
-      const float prj = pr[j];
-      const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
-      if (SHEP) shep += fl ? mVj * w : 0.0f;
-      svx += fl ? mVj * vj.x * w : 0.0f;
-      svy += fl ? mVj * vj.y * w : 0.0f;
-      svz += fl ? mVj * vj.z * w : 0.0f;
-      sp += fl ? mVj * (prj + vj.w * gy * y) * w : 0.0f;
-    });
-  }
   float cs;
   if (SHEP) {
-    cs = shep != 0.0f ? 1.0f / shep : 1.0f;
+    cs = acc[4] != 0.0f ? 1.0f / acc[4] : 1.0f;
     a.w.cspm[p] = cs;
   } else {
-    cs = cs_in;
+    cs = a.w.cspm[p];
   }
-  const float4 vt = make_float4(2.0f * v.x - svx * cs, 2.0f * v.y - svy * cs,
-                                2.0f * v.z - svz * cs, S.rho0);
+  const float4 vt = make_float4(2.0f * v.x - acc[0] * cs, 2.0f * v.y - acc[1] * cs,
+                                2.0f * v.z - acc[2] * cs, S.rho0);
   a.cur.vtmp[p] = vt;
-  const float pv = sp * cs;
+  const float pv = acc[3] * cs;
   const float pc = pv > 0.0f ? pv : 0.0f;
   a.w.p[p] = pc;
   // sign bit marks the boundary particle for the fluid pass
   a.w.vp[p] = make_float4(vt.x, vt.y, vt.z,
                           __int_as_float(__float_as_int(pc / (S.rho0 * S.rho0)) | (int)0x80000000));
+}
+// again: a later one_step of the same fused step.  Most dummy particles have
+// no flow particle in reach (an empty list): their sums are +0 in every
+// one_step, so the first stores their extrapolation and the later ones skip
+// them (1.41 M of the 1.65 M dummy particles of the 3D dam break).
+template <int DIM, bool NL, bool SHEP>
+__global__ __launch_bounds__(256) void k_wc_bdy(KArgs a, int again) {
+  constexpr int L = NL ? kLanes : 1;
+  const int8_t* __restrict__ type = a.cur.type;
+  const float4* __restrict__ vtmp = a.cur.vtmp;
+  const float* __restrict__ pr = a.w.p;
+  for_work<NL, true>(
+      a, again ? kTileWall : kTileWall | kTileBare,
+      [&](int s, int p, bool mine) {
+        const int tp = type[p];
+        if (!is_solid(tp)) return false;  // boundary and rigid (solver_sph_wc.py:90-103)
+        if (!NL || a.w.nlc[p] != 0) return true;
+        if (mine && !(again && is_bdy(tp))) {
+          const float none[5] = {};
+          wc_wall_store<SHEP>(a, a.scenes[s], p, none);
+        }
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        const float gy = S.grav[1];
+        constexpr int NT = SHEP ? 5 : 4;
+        float acc[NT] = {};
+        // Straight-line pair terms (a non-flow neighbour adds +0, which leaves
+        // every sum's bits unchanged: the sums start at +0 and never become -0
+        // in round-to-nearest), so the loads of a batch of neighbours are
+        // issued together instead of one branch at a time.
+        sum_pairs_k<DIM, NL, L>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                                float mVj, float (&t)[NT]) {
+          const bool fl = is_flow(type[j]);
+          const float4 vj = vtmp[j];
+          const float prj = pr[j];
+          const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
+          t[0] = term_if(fl, mVj * vj.x * w);
+          t[1] = term_if(fl, mVj * vj.y * w);
+          t[2] = term_if(fl, mVj * vj.z * w);
+          t[3] = term_if(fl, mVj * (prj + vj.w * gy * y) * w);
+          if (SHEP) t[NT - 1] = term_if(fl, mVj * w);
+        });
+        if (group_head<L>()) wc_wall_store<SHEP>(a, S, p, acc);
+      });
 }
 
 // Fluid loop B (solver_sph_wc.py:108-123; tasks solver_sph_base.py:195-203,
@@ -912,118 +1145,75 @@ __global__ __launch_bounds__(256) void k_wc_bdy(KArgs a) {
 // solver_sph_base.py:386-398: flow neighbours, list order), which the fused
 // step then leaves out of the Shepard pass: in WC only boundary particles
 // read CSPM_f within the step, so fluid particles get it here, bitwise equal.
-// The pair terms of one fluid particle, one neighbour at a time in list
-// order: d_density (solver_sph_base.py:195-203), viscosity and pressure
-// force (solver_sph_wc.py:33-71) and, with SHEP, the Shepard sum.  q is the
-// neighbour's pair record (v_tmp, p / rho_tmp^2, sign bit set for a wall).
-template <int KT, bool SHEP>
-struct WcPairSum {
-  float vix, viy, viz, pri, c1, c2, rho0, rr;
-  float dd = 0.f, dvx = 0.f, dvy = 0.f, dvz = 0.f, shep = 0.f;
-  __device__ __forceinline__ void add(const SceneDev& S, float x, float y, float z, float r2, float mVj,
-                                      const float4& q) {
-    const float rn = pair_dist(r2);
-    const float f = kernel_gradfac_t<KT>(S, rn);
-    const float gx = f * x, gy = f * y, gz = f * z;
-    const bool bj = __float_as_int(q.w) < 0;  // boundary neighbour
-    const float ux = vix - q.x, uy = viy - q.y, uz = viz - q.z;
-    dd += (mVj * ux) * gx + (mVj * uy) * gy + (mVj * uz) * gz;
-    if (SHEP) shep += bj ? 0.0f : mVj * kernel_W_t<KT>(S, rn);
-    // viscosity_force: fluid and boundary neighbours (solver_sph_wc.py:33-45)
-    const float vx_ = ux * x + uy * y + uz * z;
-    const float mn = vx_ < 0.0f ? vx_ : 0.0f;
-    const float a0 = c1 * mVj;
-    const float aa = bj ? a0 * rr : a0;
-    const float vis = aa * mn / (r2 + c2);
-    const float pc = (-rho0 * mVj) * (pri + fabsf(q.w));
-    const float sc = vis + pc;
-    dvx += sc * gx;
-    dvy += sc * gy;
-    dvz += sc * gz;
-  }
-  __device__ __forceinline__ void store(const KArgs& a, const SceneDev& S, int p, float rho_i) const {
-    a.w.drho[p] = dd * rho_i;
-    a.w.dv[p] = make_float4(dvx + S.grav[0], dvy + S.grav[1], dvz + S.grav[2], 0.0f);
-    if (SHEP) a.w.cspm[p] = shep != 0.0f ? 1.0f / shep : 1.0f;
-  }
-};
-
-template <int DIM, bool NL, bool SHEP, int KT, bool KC>
-__device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, int p) {
-  const Centre C = centre_of(a, S, p);
-  // A WC scene holds fluid, boundary and rigid particles only (checked at
-  // upload), and rigid ones are walls to the fluid: a neighbour's pair
-  // record (written by the EOS or the boundary pass, sign bit set for a
-  // wall) says which it is, so the pass reads position + m_V and
-  // v_tmp + p/rho_tmp^2 per neighbour and nothing else.
+// The pair terms: d_density (solver_sph_base.py:195-203, by the corrected
+// gradient with KC), viscosity and pressure force (solver_sph_wc.py:33-71,
+// by the plain one) and, with SHEP, the Shepard sum.  A WC scene holds fluid,
+// boundary and rigid particles only (checked at upload), and rigid ones are
+// walls to the fluid: a neighbour's pair record q (v_tmp, p / rho_tmp^2,
+// written by the EOS or the boundary pass, sign bit set for a wall) says
+// which it is, so the pass reads position + m_V and q per neighbour and
+// nothing else.
+template <int DIM, bool NL, bool SHEP, int KT, bool KC, int L>
+__device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   const float4* __restrict__ vp = a.w.vp;
   const float4 vi = a.cur.vtmp[p];
   const float pri = vp[p].w;
   const float c1 = S.visc_c1, c2 = S.visc_c2, rho0 = S.rho0;
   const float rr = rho0 / vi.w;  // rho0 / rho_i of the boundary viscosity
-  if (!KC) {
-    WcPairSum<KT, SHEP> acc{vi.x, vi.y, vi.z, pri, c1, c2, rho0, rr};
-    neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj, int) {
-      acc.add(S, x, y, z, r2, mVj, vp[j]);
-    });
-    if (S.rep) {
-      // calc_rep_force_task (solver_sph_wc.py:74-76, 118-121): a second
-      // sweep adding the repulsive particles' force after the pair forces
-      const int8_t* __restrict__ type = a.cur.type;
-      neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float, int) {
-        if (type[j] != kRep) return;
-        const float f = rep_fac(S, sqrtf(r2));
-        acc.dvx += f * x;
-        acc.dvy += f * y;
-        acc.dvz += f * z;
-      });
-    }
-    acc.store(a, S, p, vi.w);
-    return;
-  }
   float M[9];
-  corr_load(a.w.Lc, a.stride, p, M);
-  float dd = 0.f, dvx = 0.f, dvy = 0.f, dvz = 0.f, shep = 0.f;
-  neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj, int) {
+  if (KC) corr_load(a.w.Lc, a.stride, p, M);
+  constexpr int NT = DIM + 1 + (SHEP ? 1 : 0);
+  float acc[NT] = {};  // d_density, d_vel, Shepard
+  sum_pairs<DIM, NL, L>(S, a, p, o, acc, [&](int j, float x, float y, float z, float r2, float mVj,
+                                             float (&t)[NT]) {
     const float rn = pair_dist(r2);
     const float f = kernel_gradfac_t<KT>(S, rn);
     const float gx = f * x, gy = f * y, gz = f * z;
-    const float4 q = vp[j];
+    float4 q = vp[j];
+    if (DIM == 2) asm volatile("" : "+v"(q.z));  // one 16-byte load
     const bool bj = __float_as_int(q.w) < 0;  // boundary neighbour
     const float ux = vi.x - q.x, uy = vi.y - q.y, uz = vi.z - q.z;
-    {  // d_density takes the corrected gradient, the forces do not
-      float cg[3] = {gx, gy, gz};
-      corr_apply(M, cg);
-      dd += (mVj * ux) * cg[0] + (mVj * uy) * cg[1] + (mVj * uz) * cg[2];
-    }
-    if (SHEP) shep += bj ? 0.0f : mVj * kernel_W_t<KT>(S, rn);
+    float cg[3] = {gx, gy, gz};
+    if (KC) corr_apply(M, cg);
+    // in 2D z = g_z = 0: their products are +-0 and leave the sums' bits
+    t[0] = (mVj * ux) * cg[0] + (mVj * uy) * cg[1];
+    if (DIM == 3 || KC) t[0] += (mVj * uz) * cg[2];
+    if (SHEP) t[NT - 1] = term_if(!bj, mVj * kernel_W_t<KT>(S, rn));
     // viscosity_force: fluid and boundary neighbours (solver_sph_wc.py:33-45)
-    const float vx_ = ux * x + uy * y + uz * z;
+    const float vx_ = DIM == 3 ? ux * x + uy * y + uz * z : ux * x + uy * y;
     const float mn = vx_ < 0.0f ? vx_ : 0.0f;
     const float a0 = c1 * mVj;
     const float aa = bj ? a0 * rr : a0;
     const float vis = aa * mn / (r2 + c2);
     const float pc = (-rho0 * mVj) * (pri + fabsf(q.w));
     const float sc = vis + pc;
-    dvx += sc * gx;
-    dvy += sc * gy;
-    dvz += sc * gz;
+    t[1] = sc * gx;
+    t[2] = sc * gy;
+    if (DIM == 3) t[3] = sc * gz;
   });
   if (S.rep) {
     // calc_rep_force_task (solver_sph_wc.py:74-76, 118-121): a second sweep
     // adding the repulsive particles' force after the pair forces
     const int8_t* __restrict__ type = a.cur.type;
-    neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float, int) {
-      if (type[j] != kRep) return;
+    float dv[DIM];
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) dv[c] = acc[1 + c];
+    sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int j, float x, float y, float z, float r2, float,
+                                              float (&t)[DIM]) {
+      if (type[j] != kRep) return no_terms(t);
       const float f = rep_fac(S, sqrtf(r2));
-      dvx += f * x;
-      dvy += f * y;
-      dvz += f * z;
+      t[0] = f * x;
+      t[1] = f * y;
+      if (DIM == 3) t[DIM - 1] = f * z;
     });
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) acc[1 + c] = dv[c];
   }
-  a.w.drho[p] = dd * vi.w;
-  a.w.dv[p] = make_float4(dvx + S.grav[0], dvy + S.grav[1], dvz + S.grav[2], 0.0f);
-  if (SHEP) a.w.cspm[p] = shep != 0.0f ? 1.0f / shep : 1.0f;
+  if (!group_head<L>()) return;
+  a.w.drho[p] = acc[0] * vi.w;
+  a.w.dv[p] = make_float4(acc[1] + S.grav[0], acc[2] + S.grav[1],
+                          (DIM == 3 ? acc[3] : 0.0f) + S.grav[2], 0.0f);
+  if (SHEP) a.w.cspm[p] = acc[NT - 1] != 0.0f ? 1.0f / acc[NT - 1] : 1.0f;
 }
 
 // d_vel of a dynamic rigid particle j: g (loop A, solver_sph_wc.py:105-106)
@@ -1032,19 +1222,19 @@ __device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, 
 // scatters with atomic updates in no fixed order; here j gathers the same
 // terms, formed from i's side (x_ij = x_i - x_j, i's density_tmp in the
 // wall viscosity), in its own neighbour order.
-template <int DIM, bool NL, int KT>
-__device__ __forceinline__ float4 wc_rigid_force(const KArgs& a, const SceneDev& S, int p) {
-  const Centre C = centre_of(a, S, p);
+template <int DIM, bool NL, int KT, int L>
+__device__ __forceinline__ float4 wc_rigid_force(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   const int8_t* __restrict__ type = a.cur.type;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float4* __restrict__ vp = a.w.vp;
   const float4 vj = vtmp[p];
-  const float mVj = C.P.w;
+  const float mVj = o.P.w;
   const float prj = fabsf(vp[p].w);  // p_j / rho_j^2 of the wall record
   const float c1 = S.visc_c1, c2 = S.visc_c2, rho0 = S.rho0;
-  float dvx = S.grav[0], dvy = S.grav[1], dvz = S.grav[2];
-  neighbours<DIM, NL>(S, a, p, C, [&](int i, float x, float y, float z, float r2, float, int) {
-    if (type[i] != kFluid) return;
+  float dv[3] = {S.grav[0], S.grav[1], S.grav[2]};
+  sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int i, float x, float y, float z, float r2, float,
+                                            float (&t)[3]) {
+    if (type[i] != kFluid) return no_terms(t);
     const float xi = -x, yi = -y, zi = -z;  // x_i - x_j
     const float rn = pair_dist(r2);
     const float f = kernel_gradfac_t<KT>(S, rn);
@@ -1057,78 +1247,83 @@ __device__ __forceinline__ float4 wc_rigid_force(const KArgs& a, const SceneDev&
     const float vis = ((c1 * mVj) * rr) * mn / (r2 + c2);
     const float pc = (-rho0 * mVj) * (vp[i].w + prj);
     const float sc = vis + pc;
-    dvx -= sc * gx;
-    dvy -= sc * gy;
-    dvz -= sc * gz;
+    t[0] = -(sc * gx);
+    t[1] = -(sc * gy);
+    t[2] = -(sc * gz);
   });
-  return make_float4(dvx, dvy, dvz, 0.0f);
+  return make_float4(dv[0], dv[1], dv[2], 0.0f);
 }
 
-template <int DIM, bool NL, bool SHEP>
-__global__ __launch_bounds__(256) void k_wc_fluid(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  const int tp = a.cur.type[p];
-  if (tp != kFluid) {
-    // Rates of other particles are never written by the reference: zero;
-    // a static rigid particle's d_vel is zero too (solver_sph_wc.py:125-126).
-    float4 dv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tp == kRigid) {
-      const SceneDev S = a.scenes[s];
-      if (rigid_slot(S, tp, a.cur.obj[p]) >= 0) {
-        if (S.kernel == 1) dv = wc_rigid_force<DIM, NL, 1>(a, S, p);
-        else dv = wc_rigid_force<DIM, NL, 0>(a, S, p);
-      }
-    }
-    a.w.drho[p] = 0.0f;
-    a.w.dv[p] = dv;
-    return;
-  }
-  const SceneDev S = a.scenes[s];
-  if (S.kcorr != 0) {
-    if (S.kernel == 1) wc_fluid_one<DIM, NL, SHEP, 1, true>(a, S, p);
-    else wc_fluid_one<DIM, NL, SHEP, 0, true>(a, S, p);
-  } else {
-    if (S.kernel == 1) wc_fluid_one<DIM, NL, SHEP, 1, false>(a, S, p);
-    else wc_fluid_one<DIM, NL, SHEP, 0, false>(a, S, p);
-  }
+// Rates of other particles are never written by the reference: zero (by the
+// step's first pass; again: a later one); a static rigid particle's d_vel is
+// zero too (solver_sph_wc.py:125-126).
+template <int DIM, bool NL, bool SHEP, bool KC>
+__global__ __launch_bounds__(256) void k_wc_fluid(KArgs a, int again) {
+  constexpr int L = NL ? kLanes : 1;
+  for_work<NL, false>(
+      a, again ? kTileFlow : ~0,
+      [&](int s, int p, bool mine) {
+        const int tp = a.cur.type[p];
+        if (tp == kFluid) return true;
+        if (tp == kRigid && rigid_slot(a.scenes[s], tp, a.cur.obj[p]) >= 0) return true;
+        if (mine && !again) {
+          a.w.drho[p] = 0.0f;
+          a.w.dv[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        if (a.cur.type[p] == kRigid) {
+          const float4 dv = S.kernel == 1 ? wc_rigid_force<DIM, NL, 1, L>(a, S, p, o)
+                                          : wc_rigid_force<DIM, NL, 0, L>(a, S, p, o);
+          if (!group_head<L>()) return;
+          a.w.drho[p] = 0.0f;
+          a.w.dv[p] = dv;
+          return;
+        }
+        if (KC && S.kcorr != 0) {
+          if (S.kernel == 1) wc_fluid_one<DIM, NL, SHEP, 1, true, L>(a, S, p, o);
+          else wc_fluid_one<DIM, NL, SHEP, 0, true, L>(a, S, p, o);
+        } else {
+          if (S.kernel == 1) wc_fluid_one<DIM, NL, SHEP, 1, false, L>(a, S, p, o);
+          else wc_fluid_one<DIM, NL, SHEP, 0, false, L>(a, S, p, o);
+        }
+      });
 }
 
 // ======================================================================= muI
+// Velocity gradient L and d_density terms of a soil pair (calc_v_grad_task,
+// d_density): t[0..8] = m_V (v_j - v_i) (x) grad W, t[9] = d_density.
+__device__ __forceinline__ void soil_grad_terms(const float4& vi, const float4& vj, float mVj,
+                                                const float gw[3], float* t) {
+  const float u[3] = {mVj * (vj.x - vi.x), mVj * (vj.y - vi.y), mVj * (vj.z - vi.z)};
+#pragma unroll
+  for (int k = 0; k < 9; ++k) t[k] = u[k / 3] * gw[k % 3];
+  t[9] = (mVj * (vi.x - vj.x)) * gw[0] + (mVj * (vi.y - vj.y)) * gw[1] +
+         (mVj * (vi.z - vj.z)) * gw[2];
+}
+
 // Soil loop 1 (solver_sph_muI.py:200-225).
-template <int DIM, bool NL>
-__global__ __launch_bounds__(256) void k_mui_soil1(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) {
-    a.w.drho[p] = 0.0f;
-    a.w.p[p] = 0.0f;
-    a.w.dseq[p] = 0.0;
-    return;
-  }
-  const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+template <int DIM, bool NL, bool KC>
+__device__ __forceinline__ void mui_soil1_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+  constexpr int LN = NL ? kLanes : 1;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float4 vi = vtmp[p];
-  const bool kc = S.kcorr != 0;
+  const bool kc = KC && S.kcorr != 0;
   float M[9];
   if (kc) corr_load(a.w.Lc, a.stride, p, M);
-  float L[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-  float dd = 0.f;
-  neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                  float mVj, int) {
+  float acc[10] = {};
+  sum_pairs_k<DIM, NL, LN>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                float mVj, float (&t)[10]) {
     const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
     float gw[3] = {f * x, f * y, f * z};
     if (kc) corr_apply(M, gw);
-    const float4 vj = vtmp[j];
-    const float u[3] = {mVj * (vj.x - vi.x), mVj * (vj.y - vi.y), mVj * (vj.z - vi.z)};
-#pragma unroll
-    for (int aa = 0; aa < 3; ++aa)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb) L[aa][bb] += u[aa] * gw[bb];
-    dd += (mVj * (vi.x - vj.x)) * gw[0] + (mVj * (vi.y - vj.y)) * gw[1] +
-          (mVj * (vi.z - vj.z)) * gw[2];
+    soil_grad_terms(vi, vtmp[j], mVj, gw, t);
   });
+  if (!group_head<LN>()) return;
+  const float L[3][3] = {{acc[0], acc[1], acc[2]}, {acc[3], acc[4], acc[5]}, {acc[6], acc[7], acc[8]}};
+  const float dd = acc[9];
   a.w.drho[p] = dd * vi.w;
   float pp = S.vsound2 * (a.cur.vel[p].w - S.rho0);
   pp = pp > 0.0f ? pp : 0.0f;
@@ -1162,57 +1357,86 @@ __global__ __launch_bounds__(256) void k_mui_soil1(KArgs a) {
     }
   a.w.dseq[p] = (double)sqrtf(sd * 2.0f / 3.0f);
 }
+template <int DIM, bool NL, bool KC>
+__global__ __launch_bounds__(256) void k_mui_soil1(KArgs a, int again) {
+  for_work<NL, false>(
+      a, again ? kTileFlow : ~0,
+      [&](int, int p, bool mine) {
+        if (a.cur.type[p] == kSoil) return true;
+        if (mine && !again) {
+          a.w.drho[p] = 0.0f;
+          a.w.p[p] = 0.0f;
+          a.w.dseq[p] = 0.0;
+        }
+        return false;
+      },
+      [&](int s, int p, const Own& o) { mui_soil1_one<DIM, NL, KC>(a, a.scenes[s], p, o); });
+}
 
 // Dummy loop of muI (:228-242) and DP (:220-231).
-template <int DIM, bool EXTRAP_DENSITY, bool NL>
-__global__ __launch_bounds__(256) void k_soil_bdy(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (!is_solid(a.cur.type[p])) return;  // boundary and rigid (muI :96, DP :221)
-  const SceneDev S = a.scenes[s];
-  const int8_t* __restrict__ type = a.cur.type;
-  const float4* __restrict__ vtmp = a.cur.vtmp;
-  const float* __restrict__ sgt = a.w.sigt_f;
+// acc: sums of the stress (6), v (3) and the density.
+template <bool EXTRAP_DENSITY>
+__device__ __forceinline__ void soil_wall_store(const KArgs& a, const SceneDev& S, int p, const float* acc) {
   const int st = a.stride;
-  float sv[3] = {0.f, 0.f, 0.f}, sr = 0.f, ssg[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  // as in k_wc_bdy: an empty list skips the walk (the sums stay +0), and
-  // the pair terms are straight-line (a non-flow neighbour adds +0)
-  if (!NL || a.w.nlc[p] != 0) {
-    const Centre C = centre_of(a, S, p);
-    neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                    float mVj, int) {
-      const bool fl = is_flow(type[j]);
-      const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
-      const float4 vj = vtmp[j];
-      float sj[6];
-#pragma unroll
-      for (int c = 0; c < 6; ++c) sj[c] = sgt[c * st + j];
-      sv[0] += fl ? mVj * vj.x * w : 0.0f;
-      sv[1] += fl ? mVj * vj.y * w : 0.0f;
-      sv[2] += fl ? mVj * vj.z * w : 0.0f;
-      sr += fl ? mVj * vj.w * w : 0.0f;
-      const float xr[3] = {x, y, z};
-#pragma unroll
-      for (int c = 0; c < 3; ++c) ssg[c] += fl ? mVj * (sj[c] + (vj.w * S.grav[c]) * xr[c]) * w : 0.0f;
-#pragma unroll
-      for (int c = 3; c < 6; ++c) ssg[c] += fl ? mVj * sj[c] * w : 0.0f;
-    });
-  }
   const float cs = a.w.cspm[p];
   const float4 v = a.cur.vel[p];
   float rt = S.rho0;
   if (EXTRAP_DENSITY) {
-    const float r = sr * cs;
+    const float r = acc[9] * cs;
     rt = r > S.rho0 ? r : S.rho0;
   }
-  a.cur.vtmp[p] =
-      make_float4(2.0f * v.x - sv[0] * cs, 2.0f * v.y - sv[1] * cs, 2.0f * v.z - sv[2] * cs, rt);
+  a.cur.vtmp[p] = make_float4(2.0f * v.x - acc[6] * cs, 2.0f * v.y - acc[7] * cs,
+                              2.0f * v.z - acc[8] * cs, rt);
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
-    const float val = ssg[c] * cs;
+    const float val = acc[c] * cs;
     a.w.sigt_f[c * st + p] = val;
     if (!EXTRAP_DENSITY) a.w.sigt_d[c * st + p] = (double)val;
   }
+}
+template <int DIM, bool EXTRAP_DENSITY, bool NL>
+__global__ __launch_bounds__(256) void k_soil_bdy(KArgs a, int again) {
+  constexpr int L = NL ? kLanes : 1;
+  const int8_t* __restrict__ type = a.cur.type;
+  const float4* __restrict__ vtmp = a.cur.vtmp;
+  const float* __restrict__ sgt = a.w.sigt_f;
+  const int st = a.stride;
+  for_work<NL, true>(
+      a, again ? kTileWall : kTileWall | kTileBare,
+      [&](int s, int p, bool mine) {
+        const int tp = type[p];
+        if (!is_solid(tp)) return false;  // boundary and rigid (muI :96, DP :221)
+        if (!NL || a.w.nlc[p] != 0) return true;
+        if (mine && !(again && is_bdy(tp))) {  // as in k_wc_bdy
+          const float none[10] = {};
+          soil_wall_store<EXTRAP_DENSITY>(a, a.scenes[s], p, none);
+        }
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        float acc[10] = {};
+        // straight-line pair terms, as in k_wc_bdy
+        sum_pairs_k<DIM, NL, L>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                                float mVj, float (&t)[10]) {
+          const bool fl = is_flow(type[j]);
+          const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
+          const float4 vj = vtmp[j];
+          float sj[6];
+#pragma unroll
+          for (int c = 0; c < 6; ++c) sj[c] = sgt[c * st + j];
+          const float xr[3] = {x, y, z};
+#pragma unroll
+          for (int c = 0; c < 3; ++c) t[c] = term_if(fl, mVj * (sj[c] + (vj.w * S.grav[c]) * xr[c]) * w);
+#pragma unroll
+          for (int c = 3; c < 6; ++c) t[c] = term_if(fl, mVj * sj[c] * w);
+          t[6] = term_if(fl, mVj * vj.x * w);
+          t[7] = term_if(fl, mVj * vj.y * w);
+          t[8] = term_if(fl, mVj * vj.z * w);
+          t[9] = term_if(fl, mVj * vj.w * w);
+        });
+        if (group_head<L>()) soil_wall_store<EXTRAP_DENSITY>(a, S, p, acc);
+      });
 }
 
 // Acceleration from stress (muI :248-261; DP :260-270) + viscous damping
@@ -1220,7 +1444,7 @@ __global__ __launch_bounds__(256) void k_soil_bdy(KArgs a) {
 template <int DIM>
 __device__ __forceinline__ void soil_dv_pair(const SceneDev& S, const float* __restrict__ sgt,
                                              int st, int j, const float si[6], float mVj,
-                                             float rtj, const float gw[3], float dv[3]) {
+                                             float rtj, const float gw[3], float* t) {
   const float rj2 = rtj * rtj;
   const float sc = mVj * rtj;
   float sj[6];
@@ -1234,7 +1458,7 @@ __device__ __forceinline__ void soil_dv_pair(const SceneDev& S, const float* __r
       const int c = sidx(aa, bb);
       acc += (sc * (sj[c] / rj2 + si[c])) * gw[bb];
     }
-    dv[aa] += acc;
+    t[aa] = acc;
   }
 }
 
@@ -1243,18 +1467,18 @@ __device__ __forceinline__ void soil_dv_pair(const SceneDev& S, const float* __r
 // neighbour i (muI :38-46, DP :158-165), formed from i's side (x_ip, i's
 // corrected gradient) and gathered in p's neighbour order (the reference
 // subtracts them with atomic updates in no fixed order).
-template <int DIM, bool NL, int KT>
-__device__ __forceinline__ float4 soil_rigid_force(const KArgs& a, const SceneDev& S, int p) {
-  const Centre C = centre_of(a, S, p);
+template <int DIM, bool NL, int KT, int L>
+__device__ __forceinline__ float4 soil_rigid_force(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   const int8_t* __restrict__ type = a.cur.type;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float* __restrict__ sgt = a.w.sigt_f;
   const int st = a.stride;
-  const float rtp = vtmp[p].w, mVp = C.P.w;
+  const float rtp = vtmp[p].w, mVp = o.P.w;
   const bool kc = S.kcorr != 0;
   float dv[3] = {S.grav[0], S.grav[1], S.grav[2]};
-  neighbours<DIM, NL>(S, a, p, C, [&](int i, float x, float y, float z, float r2, float, int) {
-    if (type[i] != kSoil) return;
+  sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int i, float x, float y, float z, float r2, float,
+                                            float (&t)[3]) {
+    if (type[i] != kSoil) return no_terms(t);
     const float f = kernel_gradfac_t<KT>(S, pair_dist(r2));
     float gw[3] = {f * -x, f * -y, f * -z};
     if (kc) {
@@ -1266,24 +1490,23 @@ __device__ __forceinline__ float4 soil_rigid_force(const KArgs& a, const SceneDe
     float si[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + i] / ri2;
-    float t[3] = {0.f, 0.f, 0.f};
     soil_dv_pair<DIM>(S, sgt, st, p, si, mVp, rtp, gw, t);
-    dv[0] -= t[0];
-    dv[1] -= t[1];
-    dv[2] -= t[2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) t[c] = -t[c];
   });
   return make_float4(dv[0], dv[1], dv[2], 0.0f);
 }
-// The non-soil branch of the soil force passes: zero rates, or the
-// gathered force of a dynamic rigid particle (a static one keeps 0,
-// muI :130-132, DP :272-274).
-template <int DIM, bool NL>
-__device__ __forceinline__ float4 soil_nonsoil_dv(const KArgs& a, int s, int p) {
+// The other particles of the soil force passes: zero rates, or the gathered
+// force of a dynamic rigid particle (a static one keeps 0, muI :130-132, DP
+// :272-274).
+__device__ __forceinline__ bool soil_has_force(const KArgs& a, int s, int p) {
   const int tp = a.cur.type[p];
-  if (tp != kRigid) return make_float4(0.f, 0.f, 0.f, 0.f);
-  const SceneDev S = a.scenes[s];
-  if (rigid_slot(S, tp, a.cur.obj[p]) < 0) return make_float4(0.f, 0.f, 0.f, 0.f);
-  return S.kernel == 1 ? soil_rigid_force<DIM, NL, 1>(a, S, p) : soil_rigid_force<DIM, NL, 0>(a, S, p);
+  return tp == kSoil || (tp == kRigid && rigid_slot(a.scenes[s], tp, a.cur.obj[p]) >= 0);
+}
+template <int DIM, bool NL, int L>
+__device__ __forceinline__ float4 soil_nonsoil_dv(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+  return S.kernel == 1 ? soil_rigid_force<DIM, NL, 1, L>(a, S, p, o)
+                       : soil_rigid_force<DIM, NL, 0, L>(a, S, p, o);
 }
 
 __device__ __forceinline__ float4 soil_dv_finish(const SceneDev& S, const float dv[3], float4 vi) {
@@ -1292,16 +1515,9 @@ __device__ __forceinline__ float4 soil_dv_finish(const SceneDev& S, const float 
                      dv[2] + S.grav[2] + damp * vi.z, 0.0f);
 }
 
-template <int DIM, bool NL>
-__global__ __launch_bounds__(256) void k_mui_soil3(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) {
-    a.w.dv[p] = soil_nonsoil_dv<DIM, NL>(a, s, p);
-    return;
-  }
-  const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+template <int DIM, bool NL, bool KC>
+__device__ __forceinline__ void mui_soil3_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+  constexpr int L = NL ? kLanes : 1;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float* __restrict__ sgt = a.w.sigt_f;
   const int st = a.stride;
@@ -1310,30 +1526,48 @@ __global__ __launch_bounds__(256) void k_mui_soil3(KArgs a) {
   float si[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + p] / ri2;
-  float dv[3] = {0.f, 0.f, 0.f};
-  const bool kc = S.kcorr != 0;
+  float dv[3] = {};
+  const bool kc = KC && S.kcorr != 0;
   float M[9];
   if (kc) corr_load(a.w.Lc, a.stride, p, M);
-  neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                  float mVj, int) {
+  sum_pairs_k<DIM, NL, L>(S, a, p, o, dv, [&](auto kt, int j, float x, float y, float z, float r2,
+                                              float mVj, float (&t)[3]) {
     const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
     float gw[3] = {f * x, f * y, f * z};
     if (kc) corr_apply(M, gw);
-    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vtmp[j].w, gw, dv);
+    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vtmp[j].w, gw, t);
   });
   if (S.rep) {
     // calc_rep_force_task (solver_sph_muI.py:34-36, 121-123), after the
     // stress forces and before gravity and damping
     const int8_t* __restrict__ type = a.cur.type;
-    neighbours<DIM, NL>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float, int) {
-      if (type[j] != kRep) return;
+    sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int j, float x, float y, float z, float r2, float,
+                                              float (&t)[3]) {
+      if (type[j] != kRep) return no_terms(t);
       const float f = rep_fac(S, sqrtf(r2));
-      dv[0] += f * x;
-      dv[1] += f * y;
-      dv[2] += f * z;
+      t[0] = f * x;
+      t[1] = f * y;
+      t[2] = f * z;
     });
   }
-  a.w.dv[p] = soil_dv_finish(S, dv, vi);
+  if (group_head<L>()) a.w.dv[p] = soil_dv_finish(S, dv, vi);
+}
+template <int DIM, bool NL, bool KC>
+__global__ __launch_bounds__(256) void k_mui_soil3(KArgs a, int again) {
+  constexpr int L = NL ? kLanes : 1;
+  for_work<NL, false>(
+      a, again ? kTileFlow : ~0,
+      [&](int s, int p, bool mine) {
+        if (soil_has_force(a, s, p)) return true;
+        if (mine && !again) a.w.dv[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        if (a.cur.type[p] == kSoil) return mui_soil3_one<DIM, NL, KC>(a, S, p, o);
+        const float4 d = soil_nonsoil_dv<DIM, NL, L>(a, S, p, o);
+        if (group_head<L>()) a.w.dv[p] = d;
+      });
 }
 
 // advect_something_func, muI (:267-289), phase 1 of D2.
@@ -1362,9 +1596,11 @@ __global__ __launch_bounds__(256) void k_mui_regu(KArgs a) {
   if (!tile_thread(a, s, p)) return;
   if (a.cur.type[p] != kSoil) return;
   const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
-  int sx = C.cx, sy = C.cy, sz = C.cz;
-  float tx = C.P.x, ty = C.P.y, tz = C.P.z;
+  const float4 P = a.cur.pos[p];
+  int cx, cy, cz;
+  decode_cell(S, a.cur.cell[p], cx, cy, cz);
+  int sx = cx, sy = cy, sz = cz;
+  float tx = P.x, ty = P.y, tz = P.z;
   renorm(sx, tx, S.grid);
   renorm(sy, ty, S.grid);
   if (DIM == 3) renorm(sz, tz, S.grid);
@@ -1373,8 +1609,8 @@ __global__ __launch_bounds__(256) void k_mui_regu(KArgs a) {
   const int st = a.stride;
   const int ti = type[p];
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  walk<DIM>(S, a.w.start, a.cur.pos, C.shift, p, sx, sy, sz, C.cx, C.cy, C.cz, C.P.x, C.P.y,
-            C.P.z, [&](int j, float x, float y, float z, float r2, float mVj, int) {
+  walk<DIM>(S, a.w.start, a.cur.pos, scene_shift(a, S), p, sx, sy, sz, cx, cy, cz, P.x, P.y, P.z,
+            [&](int j, float x, float y, float z, float r2, float mVj, int) {
               if (type[j] != ti) return;
               const float w = kernel_W(S, pair_dist(r2));
 #pragma unroll
@@ -1529,22 +1765,9 @@ __device__ void dp_bui2008(const SceneDev& S, const double L[3][3], const double
 
 // DP soil loop (solver_sph_dp.py:237-270): velocity gradient, d_density
 // and the stress acceleration in one walk, then the FP64 stress rate.
-template <int DIM, bool NL>
-__global__ __launch_bounds__(256) void k_dp_soil(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) {
-    const int st = a.stride;
-    a.w.drho[p] = 0.0f;
-    a.w.dv[p] = soil_nonsoil_dv<DIM, NL>(a, s, p);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) a.w.dsig_d[c * st + p] = 0.0;
-    a.w.dseq[p] = 0.0;
-    a.w.dseqp[p] = 0.0;
-    return;
-  }
-  const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+template <int DIM, bool NL, bool KC>
+__device__ __forceinline__ void dp_soil_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+  constexpr int LN = NL ? kLanes : 1;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float* __restrict__ sgt = a.w.sigt_f;
   const int st = a.stride;
@@ -1553,26 +1776,22 @@ __global__ __launch_bounds__(256) void k_dp_soil(KArgs a) {
   float si[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + p] / ri2;
-  float L[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-  float dd = 0.f, dv[3] = {0.f, 0.f, 0.f};
-  const bool kc = S.kcorr != 0;
+  const bool kc = KC && S.kcorr != 0;
   float M[9];
   if (kc) corr_load(a.w.Lc, a.stride, p, M);
-  neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                  float mVj, int) {
+  float acc[13] = {};  // velocity gradient (9), d_density, d_vel (3)
+  sum_pairs_k<DIM, NL, LN>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                float mVj, float (&t)[13]) {
     const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
     float gw[3] = {f * x, f * y, f * z};
     if (kc) corr_apply(M, gw);
     const float4 vj = vtmp[j];
-    const float u[3] = {mVj * (vj.x - vi.x), mVj * (vj.y - vi.y), mVj * (vj.z - vi.z)};
-#pragma unroll
-    for (int aa = 0; aa < 3; ++aa)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb) L[aa][bb] += u[aa] * gw[bb];
-    dd += (mVj * (vi.x - vj.x)) * gw[0] + (mVj * (vi.y - vj.y)) * gw[1] +
-          (mVj * (vi.z - vj.z)) * gw[2];
-    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vj.w, gw, dv);
+    soil_grad_terms(vi, vj, mVj, gw, t);
+    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vj.w, gw, t + 10);
   });
+  if (!group_head<LN>()) return;
+  const float L[3][3] = {{acc[0], acc[1], acc[2]}, {acc[3], acc[4], acc[5]}, {acc[6], acc[7], acc[8]}};
+  const float dd = acc[9], dv[3] = {acc[10], acc[11], acc[12]};
   a.w.drho[p] = dd * vi.w;
   double Ld[3][3], sd[6], ds[6], dq, dqp;
 #pragma unroll
@@ -1587,6 +1806,32 @@ __global__ __launch_bounds__(256) void k_dp_soil(KArgs a) {
   a.w.dseq[p] = dq;
   a.w.dseqp[p] = dqp;
   a.w.dv[p] = soil_dv_finish(S, dv, vi);
+}
+template <int DIM, bool NL, bool KC>
+__global__ __launch_bounds__(256) void k_dp_soil(KArgs a, int again) {
+  constexpr int L = NL ? kLanes : 1;
+  const int st = a.stride;
+  auto other = [&](int p, const float4& d) {
+    a.w.drho[p] = 0.0f;
+    a.w.dv[p] = d;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) a.w.dsig_d[c * st + p] = 0.0;
+    a.w.dseq[p] = 0.0;
+    a.w.dseqp[p] = 0.0;
+  };
+  for_work<NL, false>(
+      a, again ? kTileFlow : ~0,
+      [&](int s, int p, bool mine) {
+        if (soil_has_force(a, s, p)) return true;
+        if (mine && !again) other(p, make_float4(0.f, 0.f, 0.f, 0.f));
+        return false;
+      },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        if (a.cur.type[p] == kSoil) return dp_soil_one<DIM, NL, KC>(a, S, p, o);
+        const float4 d = soil_nonsoil_dv<DIM, NL, L>(a, S, p, o);
+        if (group_head<L>()) other(p, d);
+      });
 }
 
 // advect_something_func, DP (:276-296).
@@ -1739,26 +1984,28 @@ __global__ __launch_bounds__(256) void k_finish(KArgs a, int do_lf, int use_xsph
 // XSPH sum (solver_sph_base.py:223-226), from pre-advect positions (D3).
 template <int DIM, bool NL>
 __global__ __launch_bounds__(256) void k_xsph(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  const int ti = a.cur.type[p];
-  if (!is_real(ti)) return;
-  const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+  constexpr int L = NL ? kLanes : 1;
   const int8_t* __restrict__ type = a.cur.type;
   const float4* __restrict__ vel = a.cur.vel;
-  const float4 vi = vel[p];
-  float sx = 0.f, sy = 0.f, sz = 0.f;
-  neighbours_k<DIM, NL>(S, a, p, C, [&](auto kt, int j, float x, float y, float z, float r2,
-                                                  float mVj, int) {
-    if (type[j] != ti) return;
-    const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
-    const float4 vj = vel[j];
-    sx += mVj * (vj.x - vi.x) * w;
-    sy += mVj * (vj.y - vi.y) * w;
-    sz += mVj * (vj.z - vi.z) * w;
-  });
-  a.w.xs[p] = make_float4(sx, sy, sz, 0.f);
+  for_work<NL, false>(
+      a, kTileFlow, [&](int, int p, bool) { return is_real(type[p]); },
+      [&](int s, int p, const Own& o) {
+        const SceneDev S = a.scenes[s];
+        const int ti = type[p];
+        const float4 vi = vel[p];
+        float acc[3] = {};
+        sum_pairs_k<DIM, NL, L>(S, a, p, o, acc, [&](auto kt, int j, float x, float y, float z, float r2,
+                                                                float mVj, float (&t)[3]) {
+          // straight-line: a neighbour of another type adds +0
+          const bool same = type[j] == ti;
+          const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
+          const float4 vj = vel[j];
+          t[0] = term_if(same, mVj * (vj.x - vi.x) * w);
+          t[1] = term_if(same, mVj * (vj.y - vi.y) * w);
+          t[2] = term_if(same, mVj * (vj.z - vi.z) * w);
+        });
+        if (group_head<L>()) a.w.xs[p] = make_float4(acc[0], acc[1], acc[2], 0.f);
+      });
 }
 
 // advect_pos (solver_sph_base.py:228-238): offsets move, cells are
@@ -1933,11 +2180,11 @@ __global__ __launch_bounds__(256) void k_neighbor_stats(KArgs a, int32_t* __rest
   if (!tile_thread(a, s, p)) return;
   if (only_slot >= 0 && s != only_slot) return;
   const SceneDev S = a.scenes[s];
-  const Centre C = centre_of(a, S, p);
+  const float4 P = a.cur.pos[p];
   const int32_t* __restrict__ id0 = a.cur.id0;
   int n = 0;
   long long a1 = 0, a2 = 0;
-  walk_c<DIM>(S, a, p, C, [&](int j, float x, float y, float z, float r2, float mVj, int) {
+  walk_c<DIM>(S, a, p, P, [&](int j, float x, float y, float z, float r2, float mVj, int) {
     const long long id = id0[j];
     ++n;
     a1 += id;
