@@ -56,7 +56,7 @@ def test_sort_route_of_small_scenes(dim, block):
 
 
 def uneven(method, dim, nan, seed=3):
-    """A scene whose flow particles lie from far apart to ~80 per cell (lists
+    """A scene whose flow particles lie from far apart to 80 per cell (lists
     longer than the engine keeps, cells of more than 32 particles, windows
     wider than a cell tile), in any order; ``nan``: one offset is not a
     number and one is infinite."""
@@ -67,7 +67,7 @@ def uneven(method, dim, nan, seed=3):
     flow = np.flatnonzero((sc.mat_type == 1) | (sc.mat_type == 2))
     n = flow.size
     # x crowds towards 0: the density falls off exponentially along x
-    x = np.stack([rng.exponential(0.05, n) % 0.9, rng.uniform(0.02, 0.5, n), rng.uniform(0.02, 0.2, n)], 1)
+    x = np.stack([rng.exponential(0.025 if dim == 2 else 0.05, n) % 0.9, rng.uniform(0.02, 0.5, n), rng.uniform(0.02, 0.2, n)], 1)
     sc.pos[flow, :dim] = (x + 0.02)[:, :dim]
     sc.vel[flow, :dim] = rng.uniform(-0.1, 0.1, (n, dim))
     bad = {int(flow[5]): np.nan, int(flow[70]): np.inf} if nan else {}

@@ -677,8 +677,8 @@ __global__ __launch_bounds__(256) void k_nl_build(KArgs a, int use_cflow, int cu
 // (a small scene has few tiles).  Cell keys run (row, fast) with the fast
 // axis z in 3D and y in 2D.  The lanes of one row (a tile holds one or two)
 // have their candidates of one row offset (dy in 3D) in one contiguous
-// particle range, which the wave copies into LDS (at most STAGE candidates,
-// the cell tile; a larger window is read from global memory).
+// particle range, which the wave copies into LDS (STAGE candidates, the cell
+// tile, at a time).
 //
 // Test: every lane walks its own three fast-axis cells there in the order of
 // walk() and shifts one bit per candidate, hit or not, into a word per 32:
@@ -688,11 +688,15 @@ __global__ __launch_bounds__(256) void k_nl_build(KArgs a, int use_cflow, int cu
 // in the list; a lane pops one hit per turn from its words, all lanes in the
 // same turn, so four turns fill one aligned quad of every list and a wave's
 // store is a contiguous kilobyte.  A quad that holds hits of two waves is
-// written by the first of them.
+// written by the first of them.  A tile with a lane whose words do not fit
+// (many cells of over 32 particles) is tested a second time and records its
+// hits one by one; the counts, and so the places, are known by then.
 constexpr int kStageDefault = 256;
 constexpr int kBuildWaves = 3;
+// per lane and wave: a word per cell and 1 to spare (30 KiB of LDS in 3D with
+// 256 candidates staged: five workgroups per CU)
 template <int DIM>
-constexpr int kHitWords = DIM == 3 ? 10 : 4;  // per lane and wave: a word per cell, 1 to spare
+constexpr int kHitWords = DIM == 3 ? 10 : 5;
 
 // Hit words of one lane in list order: rows [v NW, v NW + nw_v) of wave v.
 template <int NW>
@@ -730,7 +734,7 @@ __global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build_lds(KArgs a, int 
   constexpr int NW = kHitWords<DIM>;
   __shared__ float4 stage[kBuildWaves][STAGE + 32];  // read up to 31 past the window
   __shared__ uint2 words[kBuildWaves * NW][64];
-  __shared__ int32_t count[kBuildWaves][64];  // words << 16 | hits; < 0: more words than fit
+  __shared__ int32_t count[kBuildWaves][64];  // words (at most NW + 1) << 16 | hits
   __shared__ int32_t flow[kBuildWaves][64];   // a flow particle in the wave's reach of the lane
   const int tile = __builtin_amdgcn_readfirstlane(xcd_block());
   const int2 t = a.tiles[tile];
@@ -762,169 +766,171 @@ __global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build_lds(KArgs a, int 
   const int need = bdy ? 2 : (rig ? 1 : 0);
   float4* __restrict__ sp = stage[v];
   uint2(*__restrict__ wd)[64] = words + v * NW;
+  // found(w, eb): hit bits (from the top) of up to 32 consecutive candidates,
+  // the first of which has entry eb, in list order
+  auto scan = [&](auto&& found) {
+    unsigned long long todo = __ballot(live);
+#pragma unroll 1
+    while (todo) {
+      // the lanes of the next row; sorted by cell, so they are consecutive
+      const int l0 = __builtin_ctzll(todo);
+      const int R = __builtin_amdgcn_readlane(row, l0);
+      bool act = row == R;
+      const unsigned long long mine = __ballot(act);
+      todo &= ~mine;
+      const int l1 = 63 - __builtin_clzll(mine);
+      const int wlo = max(__builtin_amdgcn_readlane(f, l0) - 1, 0);
+      const int whi = min(__builtin_amdgcn_readlane(f, l1) + 1, gf - 1);
+      const int rx = DIM == 3 ? R / gy : R, ry = DIM == 3 ? R - rx * gy : 0;
+      const bool inx = rx + dx >= 0 && rx + dx < gx;
+      // A boundary particle records nothing if no stencil cell holds a flow
+      // particle.  The flags of a row offset's window are one load; each lane
+      // picks its three from the wave's mask.
+      if (use_cflow && __any(act && bdy)) {
+        bool reach = whi - wlo >= 64;
+        if (inx && !reach) {
+#pragma unroll
+          for (int dy = (DIM == 3 ? -1 : 0); dy <= (DIM == 3 ? 1 : 0); ++dy) {
+            if (ry + dy < 0 || ry + dy >= gy) continue;
+            const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy) * gf + wlo;
+            const unsigned long long m = __ballot(lane <= whi - wlo && a.w.cflow[nk + min(lane, whi - wlo)] != 0);
+            const int sh = act ? f - 1 - wlo : 0;  // bit of the lane's first cell
+            reach = reach || ((sh >= 0 ? m >> sh : m << 1) & 7ull) != 0;
+          }
+        }
+        flow[v][lane] = reach;
+        __syncthreads();
+        act = act && (!bdy || flow[0][lane] | flow[1][lane] | flow[2][lane]);
+        __syncthreads();  // before the next row's flags
+      }
+      if (!inx || !__any(act)) continue;
+      const bool filter = __any(act && need != 0);
+      const float bx = P.x + (float)(-dx) * S.g;
+#pragma unroll 1
+      for (int dy0 = (DIM == 3 ? -1 : 0); dy0 <= (DIM == 3 ? 1 : 0); ++dy0) {
+        if (ry + dy0 < 0 || ry + dy0 >= gy) continue;
+        const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy0) * gf;
+        const int32_t jlo = start[nk + wlo] + shift, cnt = start[nk + whi + 1] + shift - jlo;
+        // the lane's cells: candidates [c[k], c[k + 1]) at fast offset k - 1
+        int c[4] = {0, 0, 0, 0};
+        if (act) {
+          c[1] = start[nk + f] + shift - jlo;
+          c[2] = start[nk + f + 1] + shift - jlo;
+          c[0] = f > 0 ? start[nk + f - 1] + shift - jlo : c[1];
+          c[3] = f < gf - 1 ? start[nk + f + 2] + shift - jlo : c[2];
+        }
+#pragma unroll 1
+        for (int w0 = 0; w0 < cnt; w0 += STAGE) {
+          const int wn = min(cnt - w0, STAGE);
+          __builtin_amdgcn_wave_barrier();  // the last window's reads are done (one wave, in order)
+          for (int q = lane; q < wn; q += 64) {
+            float4 r = pos[jlo + w0 + q];
+            const int tq = type[jlo + w0 + q];
+            r.w = is_flow(tq) ? 2.0f : (tq == kRigid ? 1.0f : 0.0f);
+            sp[q] = r;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const int dy = DIM == 3 ? dy0 : k - 1, dz = DIM == 3 ? k - 1 : 0;
+            const float by = P.y + (float)(-dy) * S.g;
+            const float bz = DIM == 3 ? P.z + (float)(-dz) * S.g : 0.0f;
+            // the sign bit of |r2| - rs2 (a NaN's is clear) is the hit
+            auto dist = [&](const float4& r) {
+              const float x = bx - r.x, y = by - r.y;
+              float r2;
+              if (DIM == 3) {
+                const float z = bz - r.z;
+                r2 = fmaf(z, z, fmaf(y, y, x * x));
+              } else {
+                r2 = fmaf(y, y, x * x);
+              }
+              return __float_as_uint(fabsf(r2) - S.rs2);
+            };
+            auto shift_in = [&](uint32_t w, const float4& r) {
+              return __builtin_amdgcn_alignbit(w, dist(r), 31);
+            };
+            // as shift_in, for candidates the lane records (kind >= need) only
+            auto shift_in_kind = [&](uint32_t w, const float4& r) {
+              return __builtin_amdgcn_alignbit(w, dist(r) & ~__float_as_uint(r.w - (float)need), 31);
+            };
+            int lo = max(c[k] - w0, 0);
+            const int hi = min(c[k + 1] - w0, wn);
+#pragma unroll 1
+            for (; __any(lo < hi); lo += 32) {
+              const int m = min(hi - lo, 32);  // <= 0 for a lane that is done
+              uint32_t w = 0;
+              const float4* __restrict__ q = sp + min(lo, wn);
+              int done = 0;
+              if (!filter) {
+#pragma unroll 1
+                do {
+                  const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
+                  w = shift_in(shift_in(shift_in(shift_in(w, r0), r1), r2), r3);
+                  done += 4;
+                  q += 4;
+                } while (__any(done < m));
+              } else {
+#pragma unroll 1
+                do {
+                  const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
+                  w = shift_in_kind(shift_in_kind(shift_in_kind(shift_in_kind(w, r0), r1), r2), r3);
+                  done += 4;
+                  q += 4;
+                } while (__any(done < m));
+              }
+              w <<= (32 - done) & 31;
+              // candidates past the lane's cell, and the particle itself
+              if (m < 32) w &= m > 0 ? ~(0xFFFFFFFFu >> m) : 0u;
+              const int32_t j = jlo + w0 + lo;
+              if (dx == 0 && dy == 0 && dz == 0) {
+                const int i = p - j;
+                if (i >= 0 && i < 32) w &= ~(0x80000000u >> i);
+              }
+              if (w) found(w, nl_entry(j, ((dx + 1) << 4) | ((dy + 1) << 2) | (dz + 1)));
+            }
+          }
+        }
+      }
+    }
+  };
   int nw = 0, h = 0;
-  unsigned long long todo = __ballot(live);
-#pragma unroll 1
-  while (todo) {
-    // the lanes of the next row; sorted by cell, so they are consecutive
-    const int l0 = __builtin_ctzll(todo);
-    const int R = __builtin_amdgcn_readlane(row, l0);
-    bool act = row == R;
-    const unsigned long long mine = __ballot(act);
-    todo &= ~mine;
-    const int l1 = 63 - __builtin_clzll(mine);
-    const int wlo = max(__builtin_amdgcn_readlane(f, l0) - 1, 0);
-    const int whi = min(__builtin_amdgcn_readlane(f, l1) + 1, gf - 1);
-    const int rx = DIM == 3 ? R / gy : R, ry = DIM == 3 ? R - rx * gy : 0;
-    const bool inx = rx + dx >= 0 && rx + dx < gx;
-    // A boundary particle records nothing if no stencil cell holds a flow
-    // particle.  The flags of a row offset's window are one load; each lane
-    // picks its three from the wave's mask.
-    if (use_cflow && __any(act && bdy)) {
-      bool reach = whi - wlo >= 64;
-      if (inx && !reach) {
-#pragma unroll
-        for (int dy = (DIM == 3 ? -1 : 0); dy <= (DIM == 3 ? 1 : 0); ++dy) {
-          if (ry + dy < 0 || ry + dy >= gy) continue;
-          const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy) * gf + wlo;
-          const unsigned long long m = __ballot(lane <= whi - wlo && a.w.cflow[nk + min(lane, whi - wlo)] != 0);
-          const int sh = act ? f - 1 - wlo : 0;  // bit of the lane's first cell
-          reach = reach || ((sh >= 0 ? m >> sh : m << 1) & 7ull) != 0;
-        }
-      }
-      flow[v][lane] = reach;
-      __syncthreads();
-      act = act && (!bdy || flow[0][lane] | flow[1][lane] | flow[2][lane]);
-      __syncthreads();  // before the next row's flags
-    }
-    if (!inx || !__any(act)) continue;
-    const bool filter = __any(act && need != 0);
-    const float bx = P.x + (float)(-dx) * S.g;
-#pragma unroll 1
-    for (int dy0 = (DIM == 3 ? -1 : 0); dy0 <= (DIM == 3 ? 1 : 0); ++dy0) {
-      if (ry + dy0 < 0 || ry + dy0 >= gy) continue;
-      const int32_t nk = S.cbase + ((rx + dx) * gy + ry + dy0) * gf;
-      const int32_t jlo = start[nk + wlo] + shift, cnt = start[nk + whi + 1] + shift - jlo;
-      if (cnt == 0) continue;
-      if (cnt > 4 * STAGE || __any(nw > NW)) {  // dense: walked below
-        nw = NW + 1;
-        break;
-      }
-      // the lane's cells: candidates [c[k], c[k + 1]) at fast offset k - 1
-      int c[4] = {0, 0, 0, 0};
-      if (act) {
-        c[1] = start[nk + f] + shift - jlo;
-        c[2] = start[nk + f + 1] + shift - jlo;
-        c[0] = f > 0 ? start[nk + f - 1] + shift - jlo : c[1];
-        c[3] = f < gf - 1 ? start[nk + f + 2] + shift - jlo : c[2];
-      }
-      const bool staged = cnt <= STAGE;
-      if (staged) {
-        __builtin_amdgcn_wave_barrier();  // the last row offset's reads are done (one wave, in order)
-        for (int q = lane; q < cnt; q += 64) {
-          float4 r = pos[jlo + q];
-          const int tq = type[jlo + q];
-          r.w = is_flow(tq) ? 2.0f : (tq == kRigid ? 1.0f : 0.0f);
-          sp[q] = r;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int dy = DIM == 3 ? dy0 : k - 1, dz = DIM == 3 ? k - 1 : 0;
-        const float by = P.y + (float)(-dy) * S.g;
-        const float bz = DIM == 3 ? P.z + (float)(-dz) * S.g : 0.0f;
-        // the sign bit of |r2| - rs2 (a NaN's is clear) is the hit
-        auto dist = [&](const float4& r) {
-          const float x = bx - r.x, y = by - r.y;
-          float r2;
-          if (DIM == 3) {
-            const float z = bz - r.z;
-            r2 = fmaf(z, z, fmaf(y, y, x * x));
-          } else {
-            r2 = fmaf(y, y, x * x);
-          }
-          return __float_as_uint(fabsf(r2) - S.rs2);
-        };
-        auto shift_in = [&](uint32_t w, const float4& r) {
-          return __builtin_amdgcn_alignbit(w, dist(r), 31);
-        };
-        // as shift_in, for candidates the lane records (kind >= need) only
-        auto shift_in_kind = [&](uint32_t w, const float4& r) {
-          return __builtin_amdgcn_alignbit(w, dist(r) & ~__float_as_uint(r.w - (float)need), 31);
-        };
-        int lo = c[k];
-        const int hi = c[k + 1];
-#pragma unroll 1
-        for (; __any(lo < hi); lo += 32) {
-          const int m = min(hi - lo, 32);  // <= 0 for a lane that is done
-          uint32_t w = 0;
-          if (staged) {
-            const float4* __restrict__ q = sp + min(lo, cnt);
-            int done = 0;
-            if (!filter) {
-#pragma unroll 1
-              do {
-                const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
-                w = shift_in(shift_in(shift_in(shift_in(w, r0), r1), r2), r3);
-                done += 4;
-                q += 4;
-              } while (__any(done < m));
-            } else {
-#pragma unroll 1
-              do {
-                const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
-                w = shift_in_kind(shift_in_kind(shift_in_kind(shift_in_kind(w, r0), r1), r2), r3);
-                done += 4;
-                q += 4;
-              } while (__any(done < m));
-            }
-            w <<= (32 - done) & 31;
-          } else {
-            for (int i = 0; i < m; ++i) {
-              float4 r = pos[jlo + lo + i];
-              const int tj = type[jlo + lo + i];
-              r.w = is_flow(tj) ? 2.0f : (tj == kRigid ? 1.0f : 0.0f);
-              w |= shift_in_kind(0, r) << (31 - i);
-            }
-          }
-          // candidates past the lane's cell, and the particle itself
-          if (m < 32) w &= m > 0 ? ~(0xFFFFFFFFu >> m) : 0u;
-          if (dx == 0 && dy == 0 && dz == 0) {
-            const int i = p - jlo - lo;
-            if (i >= 0 && i < 32) w &= ~(0x80000000u >> i);
-          }
-          if (w) {
-            if (nw < NW)
-              wd[nw][lane] = make_uint2(w, nl_entry(jlo + lo, ((dx + 1) << 4) | ((dy + 1) << 2) | (dz + 1)));
-            ++nw;
-            h += __popc(w);
-          }
-        }
-      }
-    }
-  }
-  count[v][lane] = nw > NW ? INT32_MIN : (nw << 16 | h);
+  scan([&](uint32_t w, uint32_t eb) {
+    if (nw < NW) wd[nw][lane] = make_uint2(w, eb);
+    ++nw;
+    h += __popc(w);
+  });
+  // at most 2^16 - 1 hits can be recorded, and a list is far shorter
+  count[v][lane] = min(nw, NW + 1) << 16 | min(h, 0xFFFF);
   __syncthreads();
   const int c0 = count[0][lane], c1 = count[1][lane], c2 = count[2][lane];
   const int cap = a.nl_cap;
-  if (__any((c0 | c1 | c2) < 0)) {
-    // more hit words than fit (cells of over 32 particles): the first wave walks
-    if (v != 0) return;
-    int n = -1;
-    if (live) a.w.nlc[p] = n = nl_build_one<DIM>(a, s, p, bdy, rig, use_cflow, 0);
-    set_tile_flags(a, tile, n, bdy, rig);
-    return;
-  }
   const int h0 = c0 & 0xFFFF, h1 = c1 & 0xFFFF, n = h0 + h1 + (c2 & 0xFFFF);
   if (v == 0) {
     if (live) a.w.nlc[p] = n;
     set_tile_flags(a, tile, live ? n : -1, bdy, rig);
   }
+  // this wave's hits are [o, o + h) of the list
+  const int o = (v > 0 ? h0 : 0) + (v > 1 ? h1 : 0);
+  if (__any(max(c0, max(c1, c2)) >> 16 > NW)) {  // workgroup-uniform
+    int k = o;
+    uint32_t* __restrict__ li = a.w.nl + nl_base(live ? p : t.y, cap);
+    scan([&](uint32_t w, uint32_t eb) {
+      while (w) {
+        const int b = __builtin_clz(w);
+        w ^= 0x80000000u >> b;
+        if (n <= cap) li[nl_at(k)] = eb + ((uint32_t)b << kNlShift);
+        ++k;
+      }
+    });
+    if (v == 2 && live && n <= cap)
+      for (; k & (kNlPad - 1); ++k) li[nl_at(k)] = a.nl_pad;
+    return;
+  }
   if (n > cap) return;  // walked by the pair passes
-  // this wave's hits are [o, o + h) of the list: the quads that start there
-  const int o = (v > 0 ? h0 : 0) + (v > 1 ? h1 : 0), skip = -o & 3;
+  // the quads that start in it
+  const int skip = -o & 3;
   if (h <= skip) return;
   uint32_t* __restrict__ li = a.w.nl + nl_base(p, cap) + nl_at(o + skip);
   HitWords<NW> hw(words, count, lane, v);
