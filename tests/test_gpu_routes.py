@@ -1,9 +1,12 @@
 """Launch routes chosen by size: a scene gets the same bits whichever route
 its engine takes (every resident scene small enough for the one-workgroup
 sort, or not)."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
+from oracle.sph_numpy import NumpySPH
 from tests.common import tiny_cfg
 from tisphi_amd import _lib as L
 from tisphi_amd.scene import build_scene
@@ -105,3 +108,47 @@ def test_list_modes_agree_on_uneven_scenes(method, dim, nan):
             ref = out
         for f in fields:
             np.testing.assert_array_equal(out[f], ref[f], err_msg=f"mode {mode} tile {tile}: {f}")
+
+
+@pytest.mark.parametrize("dim,kernel", [(2, 0), (2, 1), (3, 1)])
+def test_stress_regularisation_sums(dim, kernel):
+    """The regularised stress of uneven scenes in motion (0 to hundreds of
+    pairs per particle, particles that have left their cell) against the sums
+    in float64 over the same stencil."""
+    sc, _ = uneven(2, dim, False)
+    sc.kernel = kernel
+    soil = sc.mat_type == 2
+    rng = np.random.default_rng(5)
+    step = 0.2 * sc.geo.grid_size / sc.dt  # at most a fifth of a cell
+    sc.vel[soil, :dim] = rng.uniform(-step, step, (int(soil.sum()), dim))
+    eng = L.Engine(sc.method, dim, sc.n, sc.geo.grid_num_total, 1)
+    slot = eng.add_scene(sc.desc())
+    L.upload_scene(eng, slot, sc)
+    eng.upload(slot, "stress", rng.uniform(-1e4, 1e4, (sc.n, 6)))
+    for what in ("sort", "shepard", "init_tmp", "advect_pos", "advect_something"):
+        eng.run(what)
+    off, cell, mv, ty, cs, tmp, out = (eng.download(slot, f) for f in
+                                       ("offset", "cell", "m_V", "type", "cspm_f", "stress_tmp", "stress"))
+    eng.close()
+    gn, g, rs = sc.geo.grid_num, sc.geo.grid_size, sc.geo.support_radius
+    c = np.stack(np.unravel_index(cell.astype(np.int64), gn), 1)[:, :dim]
+    new = c + np.floor(off[:, :dim] / g).astype(np.int64)
+    x = off[:, :dim] + c * g
+    flow = np.flatnonzero(ty == 2)
+    like = SimpleNamespace(h=sc.geo.smoothing_len, dim=dim, d={"kernel": kernel})
+    moved, longest = 0, 0
+    for i in flow[:: max(1, flow.size // 400)]:
+        d = x[i] - x[flow]
+        r = np.sqrt((d * d).sum(1))
+        ok = (np.abs(c[flow] - new[i]).max(1) <= 1) & (r < rs) & (flow != i)
+        j, w = flow[ok], NumpySPH.W(like, r[ok])
+        t = mv[j, None] * tmp[j] * w[:, None]
+        ref = t.sum(0) * cs[i]
+        # float32 sums of n terms of a few roundings, and the distance's
+        # error (2^-22 of the cell size, from the offsets) through W
+        tol = abs(cs[i]) * ((j.size + 16) * 2.0 ** -24 * np.abs(t).sum(0)
+                            + 2.0 ** -19 * (mv[j, None] * np.abs(tmp[j])).sum(0) * float(NumpySPH.W(like, 1e-3 * rs)))
+        assert (np.abs(out[i] - ref) <= tol).all(), (i, j.size, out[i], ref, tol)
+        moved += bool((new[i] != c[i]).any())
+        longest = max(longest, j.size)
+    assert moved > 0 and longest > 64

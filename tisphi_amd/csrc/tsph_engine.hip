@@ -490,8 +490,7 @@ struct Seq {
       L.go("chk_density", k_chk_density, tb(), E->elem_block, a);
     } else if (E->method == kMUI) {
       L.go("mui_adv", k_mui_adv1, tb(), E->elem_block, a);
-      L.go("mui_regu", k_mui_regu<DIM>, pb(), E->pair_block, a);
-      L.go("mui_adv", k_mui_adv2, tb(), E->elem_block, a);
+      L.go("mui_regu", k_mui_regu<DIM>, lb(), E->pair_block, a, E->nl_valid ? 1 : 0);
     } else {
       L.go("dp_adv", k_dp_adv, tb(), E->elem_block, a);
     }
@@ -549,8 +548,7 @@ struct Seq {
     L.go("finish", k_finish, tb(), E->elem_block, a, lf_in_finish ? 1 : 0, xsph ? 1 : 0);
     E->fresh_sort = false;
     if (E->method == kMUI) {
-      L.go("mui_regu", k_mui_regu<DIM>, pb(), E->pair_block, a);
-      L.go("mui_adv", k_mui_adv2, tb(), E->elem_block, a);
+      L.go("mui_regu", k_mui_regu<DIM>, lb(), E->pair_block, a, E->nl_valid ? 1 : 0);
     }
     if (rigid) solve_rigid();
     if (collide || rigid) enforce_boundary();

@@ -1576,7 +1576,8 @@ __global__ __launch_bounds__(256) void k_mui_soil3(KArgs a, int again) {
       });
 }
 
-// advect_something_func, muI (:267-289), phase 1 of D2.
+// advect_something_func, muI (:267-289), phase 1 of D2.  The stress it sets
+// to stress_tmp is read there by phase 2, which writes every soil particle's.
 __global__ __launch_bounds__(256) void k_mui_adv1(KArgs a) {
   int s, p;
   if (!tile_thread(a, s, p)) return;
@@ -1587,22 +1588,47 @@ __global__ __launch_bounds__(256) void k_mui_adv1(KArgs a) {
   a.cur.vel[p] = v;
   a.cur.pos[p].w = a.cur.mass[p] / v.w;
   a.cur.seq[p] = (double)((float)a.cur.seq[p] + S.dt * (float)a.w.dseq[p]);
-  const int st = a.stride;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) a.cur.sig_f[c * st + p] = a.w.sigt_f[c * st + p];
 }
 
 // Phase 2 of D2: stress regularisation from the post-advect positions; the
 // stencil centre is the cell of the new position, the pair vectors use the
-// stored (pre-advect) cells.  The result is parked in the other state
-// buffer's stress, which is dead until the next counting sort refills it.
-template <int DIM>
-__global__ __launch_bounds__(256) void k_mui_regu(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) return;
-  const SceneDev S = a.scenes[s];
+// stored (pre-advect) cells.  The step's lists hold the pairs of the
+// positions before, so the stencil is walked again: a quad of lanes per
+// particle tests four candidates of a stencil column at a time (the cells of
+// a column are adjacent in the particle order) and queues the hits in LDS,
+// and the terms are formed from the queue, four entries at a time, in walk
+// order.  (Formed where a candidate hits, they cost every candidate of the
+// wave their time: one of sixteen particles' hits nearly always.)  It reads
+// stress_tmp, which phase 1 makes the stress, and writes the stress.
+// Bound: vector issue (64 % busy) and L1 data return (70 %), of ~730
+// candidates per particle in 3D.  120 k soil particles in 3D (307 k with
+// walls): 278 -> 207 us, 85 k in 2D: 41 -> 27 us, against a
+// lane per particle with the terms where a candidate hits and a copy after.
+// A queue of 16: 220 and 27 us; one quad of candidates per turn: 225 and 24.
+constexpr int kReguQueue = 32;  // hits held per particle, a multiple of 4
+struct ReguHit {
+  int j;
+  float r2;
+};
+// rows an odd number of entries apart: the quads' rows start in different banks
+__device__ __forceinline__ ReguHit* regu_queue() {
+  __shared__ ReguHit queue[kMaxBlock / 4 * (kReguQueue + 1)];
+  return queue;
+}
+template <int DIM, int KT>
+__device__ __forceinline__ void mui_regu_one(const KArgs& a, const SceneDev& S, int p) {
+  ReguHit* __restrict__ queue = regu_queue() + (threadIdx.x >> 2) * (kReguQueue + 1);
   const float4 P = a.cur.pos[p];
+  const float4* __restrict__ pos = a.cur.pos;
+  const int32_t* __restrict__ start = a.w.start;
+  const int8_t* __restrict__ type = a.cur.type;
+  const float* __restrict__ sgt = a.w.sigt_f;
+  const int st = a.stride;
+  const int lane = (int)(threadIdx.x & 63), q = lane & 3, quad = lane & 28;
+  const bool upper = lane >= 32;
+  const float rs2 = S.rs2;
+  const uint32_t below = (1u << q) - 1u;
+  const int32_t shift = scene_shift(a, S);
   int cx, cy, cz;
   decode_cell(S, a.cur.cell[p], cx, cy, cz);
   int sx = cx, sy = cy, sz = cz;
@@ -1610,30 +1636,96 @@ __global__ __launch_bounds__(256) void k_mui_regu(KArgs a) {
   renorm(sx, tx, S.grid);
   renorm(sy, ty, S.grid);
   if (DIM == 3) renorm(sz, tz, S.grid);
-  const int8_t* __restrict__ type = a.cur.type;
-  const float* __restrict__ sg = a.cur.sig_f;
-  const int st = a.stride;
-  const int ti = type[p];
-  float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  walk<DIM>(S, a.w.start, a.cur.pos, scene_shift(a, S), p, sx, sy, sz, cx, cy, cz, P.x, P.y, P.z,
-            [&](int j, float x, float y, float z, float r2, float mVj, int) {
-              if (type[j] != ti) return;
-              const float w = kernel_W(S, pair_dist(r2));
+  // the column's axis: z in 3D, y in 2D (one cell in z)
+  const int cf = DIM == 3 ? cz : cy, gf = DIM == 3 ? S.gn[2] : S.gn[1];
+  const int f0 = max((DIM == 3 ? sz : sy) - 1, 0), f1 = min((DIM == 3 ? sz : sy) + 1, gf - 1);
+  const float of = DIM == 3 ? P.z : P.y;
+  float b0 = of + (float)(cf - f0) * S.g;
+  float b1 = of + (float)(cf - (f0 + 1)) * S.g;
+  float b2 = of + (float)(cf - (f0 + 2)) * S.g;
+  // kept, or they are formed again for every candidate
+  asm("" : "+v"(b0), "+v"(b1), "+v"(b2));
+  constexpr int U = DIM == 3 ? 2 : 1;  // quads of candidates per turn
+  float acc[6] = {};
+  int cnt = 0;
+  // the terms of the first `n` queued hits (a multiple of 4, or all)
+  auto drain = [&](int n) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int k = 0; k < n; k += 4) {
+      const bool in = k + q < n;
+      ReguHit h = queue[in ? k + q : 0];
+      const bool same = in && h.j != p && type[h.j] == kSoil;
+      const float mVj = pos[h.j].w;
+      const float w = kernel_W_t<KT>(S, pair_dist(h.r2));
+      float t[6];
 #pragma unroll
-              for (int c = 0; c < 6; ++c) acc[c] += mVj * sg[c * st + j] * w;
-            });
+      for (int c = 0; c < 6; ++c) t[c] = term_if(same, mVj * sgt[c * st + h.j] * w);
+      ordered_add<4>(acc, t);
+    }
+  };
+  if (f0 <= f1) {
+#pragma unroll 1
+    for (int k = 0; k < (DIM == 3 ? 9 : 3); ++k) {
+      const int nx = sx + (DIM == 3 ? k / 3 : k) - 1, ny = DIM == 3 ? sy + k % 3 - 1 : 0;
+      if (nx < 0 || nx >= S.gn[0] || (DIM == 3 && (ny < 0 || ny >= S.gn[1]))) continue;
+      const float bx = P.x + (float)(cx - nx) * S.g;
+      const float by = P.y + (float)(cy - ny) * S.g;  // 3D
+      const int32_t* __restrict__ sk = start + S.cbase + (DIM == 3 ? (nx * S.gn[1] + ny) : nx) * gf + f0;
+      const int nf = f1 - f0 + 1;
+      const int32_t e1 = sk[1] + shift, e2 = sk[min(2, nf)] + shift, je = sk[nf] + shift;
+      // up to seven records past the column are read (the state ends in a
+      // tile of null particles)
+      for (int32_t j = sk[0] + shift + q; j - q < je; j += 4 * U) {
+        float4 pj[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) pj[u] = pos[j + 4 * u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int32_t ju = j + 4 * u;
+          float bf = b2;
+          bf = ju < e2 ? b1 : bf;
+          bf = ju < e1 ? b0 : bf;
+          const float x = bx - pj[u].x;
+          const float y = DIM == 3 ? by - pj[u].y : bf - pj[u].y;
+          const float z = DIM == 3 ? bf - pj[u].z : 0.0f;
+          const float r2 = fmaf(z, z, fmaf(y, y, x * x));
+          const bool hit = ju < je && r2 < rs2;
+          const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+          const uint32_t half = upper ? (uint32_t)(m >> 32) : (uint32_t)m;
+          const uint32_t four = (half >> quad) & 15u;
+          if (hit) queue[cnt + __popc(four & below)] = {ju, r2};
+          cnt += __popc(four);
+        }
+        if (__any(cnt > kReguQueue - 4 * U)) {
+          const int full = cnt & ~3, rest = cnt & 3;
+          drain(full);
+          const ReguHit h = queue[min(full + q, kReguQueue)];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          if (q < rest) queue[q] = h;
+          cnt = rest;
+        }
+      }
+    }
+  }
+  drain(cnt);
+  if (q != 0) return;
   const float cs = a.w.cspm[p];
 #pragma unroll
-  for (int c = 0; c < 6; ++c) a.alt.sig_f[c * st + p] = acc[c] * cs;
+  for (int c = 0; c < 6; ++c) a.cur.sig_f[c * st + p] = acc[c] * cs;
 }
-
-__global__ __launch_bounds__(256) void k_mui_adv2(KArgs a) {
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) return;
-  const int st = a.stride;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) a.cur.sig_f[c * st + p] = a.alt.sig_f[c * st + p];
+// Four waves per tile; `flagged`: the tiles' flags are those of this step.
+template <int DIM>
+__global__ __launch_bounds__(256) void k_mui_regu(KArgs a, int flagged) {
+  const int w = wave_id(), tile = w >> 2;
+  if (flagged && (a.w.tflag[tile] & kTileFlow) == 0) return;
+  const int2 t = a.tiles[tile];
+  if (t.x < 0) return;
+  const int s = __builtin_amdgcn_readfirstlane(t.x);
+  const SceneDev& S = a.scenes[s];
+  const int p = t.y + (w & 3) * 16 + (int)((threadIdx.x & 63) >> 2);
+  if (p >= S.pbase + S.n || a.cur.type[p] != kSoil) return;
+  if (S.kernel == 1) mui_regu_one<DIM, 1>(a, S, p);
+  else mui_regu_one<DIM, 0>(a, S, p);
 }
 
 // ======================================================================== DP
@@ -1972,8 +2064,6 @@ __global__ __launch_bounds__(256) void k_finish(KArgs a, int do_lf, int use_xsph
   if (t != kSoil) return;
   if (S.method == kMUI) {
     a.cur.seq[p] = (double)((float)a.cur.seq[p] + S.dt * (float)a.w.dseq[p]);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) a.cur.sig_f[c * st + p] = a.w.sigt_f[c * st + p];
   } else if (S.method == kDP) {
     double q[6];
 #pragma unroll
