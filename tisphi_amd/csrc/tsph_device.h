@@ -103,7 +103,8 @@ struct PWork {
   float* cspm;       // Shepard factor
   float* drho;       // d_density
   float4* dv;        // d_vel
-  float* sigt_f;     // 6 x cap, stress_tmp in float (muI; DP mirror)
+  float* sigt_f;     // stress_tmp in float (muI; DP mirror), one record (rec6) per particle
+  float* sigq;       // records: stress_tmp / density_tmp^2, density_tmp
   double* sigt_d;    // 6 x cap, DP stress_tmp
   double* dsig_d;    // 6 x cap, DP d_stress
   double* dseq;      // d_strain_equ
@@ -495,6 +496,36 @@ __device__ __forceinline__ float2* xy_table() {
 __device__ __forceinline__ float* z_table() {
   __shared__ float tab[3 * kTabCols];
   return tab;
+}
+
+// A record of six floats (and one more) per particle, padded to 32 bytes: a
+// pair pass gathers a neighbour's in two loads, where six arrays took six.
+constexpr int kRec = 8;
+__device__ __forceinline__ void rec6_load(const float* __restrict__ r, int i, float (&s)[6]) {
+  const float4 a = *reinterpret_cast<const float4*>(r + (size_t)i * kRec);
+  const float2 b = *reinterpret_cast<const float2*>(r + (size_t)i * kRec + 4);
+  s[0] = a.x;
+  s[1] = a.y;
+  s[2] = a.z;
+  s[3] = a.w;
+  s[4] = b.x;
+  s[5] = b.y;
+}
+__device__ __forceinline__ float rec7_load(const float* __restrict__ r, int i, float (&s)[6]) {
+  const float4 a = *reinterpret_cast<const float4*>(r + (size_t)i * kRec);
+  const float4 b = *reinterpret_cast<const float4*>(r + (size_t)i * kRec + 4);
+  s[0] = a.x;
+  s[1] = a.y;
+  s[2] = a.z;
+  s[3] = a.w;
+  s[4] = b.x;
+  s[5] = b.y;
+  return b.z;
+}
+__device__ __forceinline__ void rec6_store(float* __restrict__ r, int i, const float (&s)[6], float e = 0.0f) {
+  float4* __restrict__ o = reinterpret_cast<float4*>(r + (size_t)i * kRec);
+  o[0] = make_float4(s[0], s[1], s[2], s[3]);
+  o[1] = make_float4(s[4], s[5], e, 0.0f);
 }
 
 // A particle with the start of its list.

@@ -252,7 +252,7 @@ int alloc_work(tsph_engine* E) {
       (r = dalloc(&w.tflag, E->tiles_alloc, b)))
     return r;
   if (E->method != kWC) {
-    if ((r = dalloc(&w.sigt_f, n6, b)) || (r = dalloc(&w.dseq, n, b))) return r;
+    if ((r = dalloc(&w.sigt_f, kRec * n, b)) || (r = dalloc(&w.sigq, kRec * n, b)) || (r = dalloc(&w.dseq, n, b))) return r;
   }
   if (E->method == kDP) {
     if ((r = dalloc(&w.sigt_d, n6, b)) || (r = dalloc(&w.dsig_d, n6, b)) ||
@@ -263,7 +263,7 @@ int alloc_work(tsph_engine* E) {
 }
 
 void free_work(PWork& w) {
-  void* ptrs[] = {w.key, w.slot, w.tmp, w.sid, w.p, w.vp, w.Lc, w.cspm, w.drho, w.dv, w.sigt_f, w.sigt_d,
+  void* ptrs[] = {w.key, w.slot, w.tmp, w.sid, w.p, w.vp, w.Lc, w.cspm, w.drho, w.dv, w.sigt_f, w.sigq, w.sigt_d,
                   w.dsig_d, w.dseq, w.dseqp, w.xs, w.drho_rk, w.dv_rk, w.dsig_rk, w.count,
                   w.start, w.bsum, w.status, w.gpart, w.gout, w.nl, w.nlc, w.tflag, w.cflow,
                   w.val, w.rgb, w.x0, w.c0, w.crange, w.rigpart, w.rigout};
@@ -905,7 +905,21 @@ int transfer(tsph_engine* E, int slot, int field, void* host, size_t bytes, bool
     return TSPH_OK;
   };
   // 6-component stress: float (muI) or double (DP), component-major.
-  auto s6 = [&](float* af, double* ad, bool mirror_f) -> int {
+  // records of six floats per particle
+  auto rec6 = [&](float* rec) -> int {
+    std::vector<float> v;
+    if (up) {
+      v.assign(kRec * n, 0.0f);
+      for (int64_t i = 0; i < n; ++i)
+        for (int c = 0; c < 6; ++c) v[kRec * i + c] = (float)hd[6 * i + c];
+      return h2d(E, rec, kRec * off, v);
+    }
+    if ((r = d2h(E, (const float*)rec, kRec * off, kRec * n, v))) return r;
+    for (int64_t i = 0; i < n; ++i)
+      for (int c = 0; c < 6; ++c) hd[6 * i + c] = v[kRec * i + c];
+    return TSPH_OK;
+  };
+  auto s6 = [&](float* af, double* ad) -> int {
     for (int c = 0; c < 6; ++c) {
       if (ad) {
         std::vector<double> v;
@@ -913,11 +927,6 @@ int transfer(tsph_engine* E, int slot, int field, void* host, size_t bytes, bool
           v.resize(n);
           for (int64_t i = 0; i < n; ++i) v[i] = hd[6 * i + c];
           if ((r = h2d(E, ad, off + c * st, v))) return r;
-          if (mirror_f && af) {
-            std::vector<float> vf(n);
-            for (int64_t i = 0; i < n; ++i) vf[i] = (float)v[i];
-            if ((r = h2d(E, af, off + c * st, vf))) return r;
-          }
         } else {
           if ((r = d2h(E, (const double*)ad, off + c * st, n, v))) return r;
           for (int64_t i = 0; i < n; ++i) hd[6 * i + c] = v[i];
@@ -1007,9 +1016,11 @@ int transfer(tsph_engine* E, int slot, int field, void* host, size_t bytes, bool
         return TSPH_OK;
       }
       return i1(cur.flag);
-    case TSPH_F_STRESS: return s6(mui ? cur.sig_f : nullptr, dp ? cur.sig_d : nullptr, false);
-    case TSPH_F_STRESS_TMP: return s6(w.sigt_f, dp ? w.sigt_d : nullptr, true);
-    case TSPH_F_D_STRESS: return s6(nullptr, dp ? w.dsig_d : nullptr, false);
+    case TSPH_F_STRESS: return s6(mui ? cur.sig_f : nullptr, dp ? cur.sig_d : nullptr);
+    case TSPH_F_STRESS_TMP:
+      if (up && dp && (r = rec6(w.sigt_f))) return r;
+      return dp || !w.sigt_f ? s6(nullptr, dp ? w.sigt_d : nullptr) : rec6(w.sigt_f);
+    case TSPH_F_D_STRESS: return s6(nullptr, dp ? w.dsig_d : nullptr);
     case TSPH_F_STRAIN_EQU:
       if (!cur.seq) { if (!up) std::memset(hd, 0, n * 8); return TSPH_OK; }
       if (mui && up) {

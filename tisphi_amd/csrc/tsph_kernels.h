@@ -432,8 +432,11 @@ __global__ __launch_bounds__(256) void k_rank_move(KArgs a, int move_vtmp, int m
   if (move_vtmp) a.alt.vtmp[d] = a.cur.vtmp[p];
   const int st = a.stride;
   if (move_mui) {
+    // a soil particle's stress is not read in a step, whose regularisation
+    // writes it anew
+    if (!(fuse_init && a.cur.type[p] == kSoil))
 #pragma unroll
-    for (int c = 0; c < 6; ++c) a.alt.sig_f[c * st + d] = a.cur.sig_f[c * st + p];
+      for (int c = 0; c < 6; ++c) a.alt.sig_f[c * st + d] = a.cur.sig_f[c * st + p];
     a.alt.seq[d] = a.cur.seq[p];
   }
   if (move_dp) {
@@ -456,16 +459,11 @@ __global__ __launch_bounds__(256) void k_rank_move(KArgs a, int move_vtmp, int m
         a.w.vp[d] = make_float4(v.x, v.y, v.z, pv / (v.w * v.w));
       }
     }
-    if (t == kSoil && S.method == kMUI) {
+    // (muI: stress_tmp is formed by the first soil loop; the float records of
+    // DP by the return mapping that starts a one_step)
+    if (t == kSoil && S.method == kDP) {
 #pragma unroll
-      for (int c = 0; c < 6; ++c) a.w.sigt_f[c * st + d] = a.cur.sig_f[c * st + p];
-    } else if (t == kSoil && S.method == kDP) {
-#pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        const double v = a.cur.sig_d[c * st + p];
-        a.w.sigt_d[c * st + d] = v;
-        a.w.sigt_f[c * st + d] = (float)v;
-      }
+      for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + d] = a.cur.sig_d[c * st + p];
     }
   }
 }
@@ -1048,15 +1046,13 @@ __global__ __launch_bounds__(256) void k_init_tmp(KArgs a) {
   if (t == kSoil) {
     const int st = a.stride;
     if (S.method == kMUI) {
+      float q[6];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) a.w.sigt_f[c * st + p] = a.cur.sig_f[c * st + p];
+      for (int c = 0; c < 6; ++c) q[c] = a.cur.sig_f[c * st + p];
+      rec6_store(a.w.sigt_f, p, q);
     } else if (S.method == kDP) {
 #pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        const double v = a.cur.sig_d[c * st + p];
-        a.w.sigt_d[c * st + p] = v;
-        a.w.sigt_f[c * st + p] = (float)v;
-      }
+      for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + p] = a.cur.sig_d[c * st + p];
     }
   }
 }
@@ -1310,6 +1306,21 @@ __device__ __forceinline__ void soil_grad_terms(const float4& vi, const float4& 
          (mVj * (vi.z - vj.z)) * gw[2];
 }
 
+// stress_tmp of particle p and what the force pass takes from it, the
+// quotients by density_tmp^2: formed here once per particle, not once per
+// pair (six divisions each; the same quotients).  Both as records, two loads
+// per neighbour instead of six or seven.  muI force pass: 108 -> 54 us at
+// 120 k soil particles in 3D (wall pass 33 -> 26), 22 -> 14 us at 85 k in 2D;
+// DP pass 35 -> 28 us at 85 k in 2D.
+__device__ __forceinline__ void soil_stress_store(const KArgs& a, int p, const float (&sg)[6], float rt) {
+  const float rt2 = rt * rt;
+  float q[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) q[c] = sg[c] / rt2;
+  rec6_store(a.w.sigt_f, p, sg);
+  rec6_store(a.w.sigq, p, q, rt);
+}
+
 // Soil loop 1 (solver_sph_muI.py:200-225).
 template <int DIM, bool NL, bool KC>
 __device__ __forceinline__ void mui_soil1_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
@@ -1346,12 +1357,12 @@ __device__ __forceinline__ void mui_soil1_one(const KArgs& a, const SceneDev& S,
     for (int bb = 0; bb < 3; ++bb) ss += e[aa][bb] * e[aa][bb];
   const float en = sqrtf(0.5f * ss) + S.eps;
   const float fac = 0.0f + (S.coh + pp * S.mu) / en;
-  const int st = a.stride;
+  float sg[6];
 #pragma unroll
   for (int aa = 0; aa < 3; ++aa)
 #pragma unroll
-    for (int bb = aa; bb < 3; ++bb)
-      a.w.sigt_f[sidx(aa, bb) * st + p] = fac * e[aa][bb] - (aa == bb ? pp : 0.0f);
+    for (int bb = aa; bb < 3; ++bb) sg[sidx(aa, bb)] = fac * e[aa][bb] - (aa == bb ? pp : 0.0f);
+  soil_stress_store(a, p, sg, vi.w);
   const float tr3 = (e[0][0] + e[1][1] + e[2][2]) / 3.0f;
   float sd = 0.f;
 #pragma unroll
@@ -1393,12 +1404,13 @@ __device__ __forceinline__ void soil_wall_store(const KArgs& a, const SceneDev& 
   }
   a.cur.vtmp[p] = make_float4(2.0f * v.x - acc[6] * cs, 2.0f * v.y - acc[7] * cs,
                               2.0f * v.z - acc[8] * cs, rt);
+  float sg[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
-    const float val = acc[c] * cs;
-    a.w.sigt_f[c * st + p] = val;
-    if (!EXTRAP_DENSITY) a.w.sigt_d[c * st + p] = (double)val;
+    sg[c] = acc[c] * cs;
+    if (!EXTRAP_DENSITY) a.w.sigt_d[c * st + p] = (double)sg[c];
   }
+  soil_stress_store(a, p, sg, rt);
 }
 template <int DIM, bool EXTRAP_DENSITY, bool NL>
 __global__ __launch_bounds__(256) void k_soil_bdy(KArgs a, int again) {
@@ -1406,7 +1418,6 @@ __global__ __launch_bounds__(256) void k_soil_bdy(KArgs a, int again) {
   const int8_t* __restrict__ type = a.cur.type;
   const float4* __restrict__ vtmp = a.cur.vtmp;
   const float* __restrict__ sgt = a.w.sigt_f;
-  const int st = a.stride;
   for_work<NL, true>(
       a, again ? kTileWall : kTileWall | kTileBare,
       [&](int s, int p, bool mine) {
@@ -1429,8 +1440,7 @@ __global__ __launch_bounds__(256) void k_soil_bdy(KArgs a, int again) {
           const float w = kernel_W_t<decltype(kt)::v>(S, pair_dist(r2));
           const float4 vj = vtmp[j];
           float sj[6];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) sj[c] = sgt[c * st + j];
+          rec6_load(sgt, j, sj);
           const float xr[3] = {x, y, z};
 #pragma unroll
           for (int c = 0; c < 3; ++c) t[c] = term_if(fl, mVj * (sj[c] + (vj.w * S.grav[c]) * xr[c]) * w);
@@ -1447,22 +1457,17 @@ __global__ __launch_bounds__(256) void k_soil_bdy(KArgs a, int again) {
 
 // Acceleration from stress (muI :248-261; DP :260-270) + viscous damping
 // (solver_sph_base.py:713-715).
-template <int DIM>
-__device__ __forceinline__ void soil_dv_pair(const SceneDev& S, const float* __restrict__ sgt,
-                                             int st, int j, const float si[6], float mVj,
+// qi, qj: the stresses over their density_tmp^2; rtj: j's density_tmp.
+__device__ __forceinline__ void soil_dv_pair(const float (&qi)[6], const float (&qj)[6], float mVj,
                                              float rtj, const float gw[3], float* t) {
-  const float rj2 = rtj * rtj;
   const float sc = mVj * rtj;
-  float sj[6];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) sj[c] = sgt[c * st + j];
 #pragma unroll
   for (int aa = 0; aa < 3; ++aa) {
     float acc = 0.f;
 #pragma unroll
     for (int bb = 0; bb < 3; ++bb) {
       const int c = sidx(aa, bb);
-      acc += (sc * (sj[c] / rj2 + si[c])) * gw[bb];
+      acc += (sc * (qj[c] + qi[c])) * gw[bb];
     }
     t[aa] = acc;
   }
@@ -1476,10 +1481,10 @@ __device__ __forceinline__ void soil_dv_pair(const SceneDev& S, const float* __r
 template <int DIM, bool NL, int KT, int L>
 __device__ __forceinline__ float4 soil_rigid_force(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   const int8_t* __restrict__ type = a.cur.type;
-  const float4* __restrict__ vtmp = a.cur.vtmp;
-  const float* __restrict__ sgt = a.w.sigt_f;
+  const float* __restrict__ sgq = a.w.sigq;
   const int st = a.stride;
-  const float rtp = vtmp[p].w, mVp = o.P.w;
+  float qp[6];
+  const float rtp = rec7_load(sgq, p, qp), mVp = o.P.w;
   const bool kc = S.kcorr != 0;
   float dv[3] = {S.grav[0], S.grav[1], S.grav[2]};
   sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int i, float x, float y, float z, float r2, float,
@@ -1492,11 +1497,9 @@ __device__ __forceinline__ float4 soil_rigid_force(const KArgs& a, const SceneDe
       corr_load(a.w.Lc, st, i, M);
       corr_apply(M, gw);
     }
-    const float ri2 = vtmp[i].w * vtmp[i].w;
-    float si[6];
-#pragma unroll
-    for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + i] / ri2;
-    soil_dv_pair<DIM>(S, sgt, st, p, si, mVp, rtp, gw, t);
+    float qi[6];
+    rec6_load(sgq, i, qi);
+    soil_dv_pair(qi, qp, mVp, rtp, gw, t);
 #pragma unroll
     for (int c = 0; c < 3; ++c) t[c] = -t[c];
   });
@@ -1524,14 +1527,10 @@ __device__ __forceinline__ float4 soil_dv_finish(const SceneDev& S, const float 
 template <int DIM, bool NL, bool KC>
 __device__ __forceinline__ void mui_soil3_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   constexpr int L = NL ? kLanes : 1;
-  const float4* __restrict__ vtmp = a.cur.vtmp;
-  const float* __restrict__ sgt = a.w.sigt_f;
-  const int st = a.stride;
-  const float4 vi = vtmp[p];
-  const float ri2 = vi.w * vi.w;
-  float si[6];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + p] / ri2;
+  const float* __restrict__ sgq = a.w.sigq;
+  const float4 vi = a.cur.vtmp[p];
+  float qi[6];
+  rec6_load(sgq, p, qi);
   float dv[3] = {};
   const bool kc = KC && S.kcorr != 0;
   float M[9];
@@ -1541,7 +1540,9 @@ __device__ __forceinline__ void mui_soil3_one(const KArgs& a, const SceneDev& S,
     const float f = kernel_gradfac_t<decltype(kt)::v>(S, pair_dist(r2));
     float gw[3] = {f * x, f * y, f * z};
     if (kc) corr_apply(M, gw);
-    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vtmp[j].w, gw, t);
+    float qj[6];
+    const float rtj = rec7_load(sgq, j, qj);
+    soil_dv_pair(qi, qj, mVj, rtj, gw, t);
   });
   if (S.rep) {
     // calc_rep_force_task (solver_sph_muI.py:34-36, 121-123), after the
@@ -1602,7 +1603,7 @@ __global__ __launch_bounds__(256) void k_mui_adv1(KArgs a) {
 // stress_tmp, which phase 1 makes the stress, and writes the stress.
 // Bound: vector issue (64 % busy) and L1 data return (70 %), of ~730
 // candidates per particle in 3D.  120 k soil particles in 3D (307 k with
-// walls): 278 -> 207 us, 85 k in 2D: 41 -> 27 us, against a
+// walls): 278 -> 193 us, 85 k in 2D: 41 -> 24 us, against a
 // lane per particle with the terms where a candidate hits and a copy after.
 // A queue of 16: 220 and 27 us; one quad of candidates per turn: 225 and 24.
 constexpr int kReguQueue = 32;  // hits held per particle, a multiple of 4
@@ -1658,8 +1659,9 @@ __device__ __forceinline__ void mui_regu_one(const KArgs& a, const SceneDev& S, 
       const float mVj = pos[h.j].w;
       const float w = kernel_W_t<KT>(S, pair_dist(h.r2));
       float t[6];
+      rec6_load(sgt, h.j, t);
 #pragma unroll
-      for (int c = 0; c < 6; ++c) t[c] = term_if(same, mVj * sgt[c * st + h.j] * w);
+      for (int c = 0; c < 6; ++c) t[c] = term_if(same, mVj * t[c] * w);
       ordered_add<4>(acc, t);
     }
   };
@@ -1779,11 +1781,13 @@ __global__ __launch_bounds__(256) void k_dp_adapt(KArgs a) {  // one_step loop 1
 #pragma unroll
   for (int c = 0; c < 6; ++c) t[c] = a.w.sigt_d[c * st + p];
   dp_adapt(S, t);
+  float sg[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
     a.w.sigt_d[c * st + p] = t[c];
-    a.w.sigt_f[c * st + p] = (float)t[c];
+    sg[c] = (float)t[c];
   }
+  soil_stress_store(a, p, sg, a.cur.vtmp[p].w);
 }
 
 // calc_d_stress_Bui2008 (solver_sph_dp.py:171-208), FP64.
@@ -1867,13 +1871,11 @@ template <int DIM, bool NL, bool KC>
 __device__ __forceinline__ void dp_soil_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
   constexpr int LN = NL ? kLanes : 1;
   const float4* __restrict__ vtmp = a.cur.vtmp;
-  const float* __restrict__ sgt = a.w.sigt_f;
+  const float* __restrict__ sgq = a.w.sigq;
   const int st = a.stride;
   const float4 vi = vtmp[p];
-  const float ri2 = vi.w * vi.w;
-  float si[6];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) si[c] = sgt[c * st + p] / ri2;
+  float qi[6];
+  rec6_load(sgq, p, qi);
   const bool kc = KC && S.kcorr != 0;
   float M[9];
   if (kc) corr_load(a.w.Lc, a.stride, p, M);
@@ -1885,7 +1887,9 @@ __device__ __forceinline__ void dp_soil_one(const KArgs& a, const SceneDev& S, i
     if (kc) corr_apply(M, gw);
     const float4 vj = vtmp[j];
     soil_grad_terms(vi, vj, mVj, gw, t);
-    soil_dv_pair<DIM>(S, sgt, st, j, si, mVj, vj.w, gw, t + 10);
+    float qj[6];
+    rec6_load(sgq, j, qj);
+    soil_dv_pair(qi, qj, mVj, vj.w, gw, t + 10);
   });
   if (!group_head<LN>()) return;
   const float L[3][3] = {{acc[0], acc[1], acc[2]}, {acc[3], acc[4], acc[5]}, {acc[6], acc[7], acc[8]}};
@@ -1981,11 +1985,7 @@ __global__ __launch_bounds__(256) void k_lf_half(KArgs a, int eos) {
     const int st = a.stride;
     const double h = 0.5 * S.dt_d;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-      const double v = a.w.sigt_d[c * st + p] + h * a.w.dsig_d[c * st + p];
-      a.w.sigt_d[c * st + p] = v;
-      a.w.sigt_f[c * st + p] = (float)v;
-    }
+    for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + p] += h * a.w.dsig_d[c * st + p];
   }
 }
 
@@ -2232,11 +2232,8 @@ __global__ __launch_bounds__(256) void k_rk_advect4(KArgs a) {
   }
   if (t == kSoil && S.method == kDP) {
     const int st = a.stride;
-    for (int c = 0; c < 6; ++c) {
-      const double v = 0.5 * S.dt_d * a.w.dsig_d[c * st + p] + a.cur.sig_d[c * st + p];
-      a.w.sigt_d[c * st + p] = v;
-      a.w.sigt_f[c * st + p] = (float)v;
-    }
+    for (int c = 0; c < 6; ++c)
+      a.w.sigt_d[c * st + p] = 0.5 * S.dt_d * a.w.dsig_d[c * st + p] + a.cur.sig_d[c * st + p];
   }
 }
 __global__ __launch_bounds__(256) void k_rk_advect(KArgs a) {
