@@ -107,6 +107,7 @@ struct PWork {
   float* sigq;       // records: stress_tmp / density_tmp^2, density_tmp
   double* sigt_d;    // 6 x cap, DP stress_tmp
   double* dsig_d;    // 6 x cap, DP d_stress
+  float* gradv;      // 9 x cap, velocity gradient of a DP soil particle
   double* dseq;      // d_strain_equ
   double* dseqp;     // d_strain_equ_p
   float4* xs;        // XSPH sums

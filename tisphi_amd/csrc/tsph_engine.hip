@@ -256,14 +256,14 @@ int alloc_work(tsph_engine* E) {
   }
   if (E->method == kDP) {
     if ((r = dalloc(&w.sigt_d, n6, b)) || (r = dalloc(&w.dsig_d, n6, b)) ||
-        (r = dalloc(&w.dseqp, n, b)) || (r = dalloc(&w.dsig_rk, n6, b)))
+        (r = dalloc(&w.dseqp, n, b)) || (r = dalloc(&w.gradv, 9 * n, b)) || (r = dalloc(&w.dsig_rk, n6, b)))
       return r;
   }
   return TSPH_OK;
 }
 
 void free_work(PWork& w) {
-  void* ptrs[] = {w.key, w.slot, w.tmp, w.sid, w.p, w.vp, w.Lc, w.cspm, w.drho, w.dv, w.sigt_f, w.sigq, w.sigt_d,
+  void* ptrs[] = {w.key, w.slot, w.tmp, w.sid, w.p, w.vp, w.Lc, w.cspm, w.drho, w.dv, w.sigt_f, w.sigq, w.gradv, w.sigt_d,
                   w.dsig_d, w.dseq, w.dseqp, w.xs, w.drho_rk, w.dv_rk, w.dsig_rk, w.count,
                   w.start, w.bsum, w.status, w.gpart, w.gout, w.nl, w.nlc, w.tflag, w.cflow,
                   w.val, w.rgb, w.x0, w.c0, w.crange, w.rigpart, w.rigout};
@@ -385,7 +385,7 @@ struct Seq {
            E->w.cflow, n);
       L.go("scatter", k_scatter, tb(), eb, a);
     }
-    L.go("rank_move", k_rank_move, (E->cap + eb - 1) / eb, eb, a, 1, E->method == kMUI ? 1 : 0,
+    L.go("rank_move", E->method == kDP ? k_rank_move<true> : k_rank_move<false>, (E->cap + eb - 1) / eb, eb, a, 1, E->method == kMUI ? 1 : 0,
          E->method == kDP ? 1 : 0, fuse_init ? 1 : 0);
     E->parity ^= 1;
     E->nl_valid = false;
@@ -425,12 +425,15 @@ struct Seq {
   // pass also forms the fluid particles' Shepard factors.
   // again: a later one_step of a fused step (what the first stored for
   // particles without pairs still holds).
-  void one_step(bool with_eos = true, bool shep = false, bool again = false) {
-    if (E->nl_valid) one_step_t<true>(with_eos, shep, again ? 1 : 0);
-    else one_step_t<false>(with_eos, shep, again ? 1 : 0);
+  // DP: mapped: the pass before has mapped stress_tmp back already;
+  // rate_later: the pass after forms the stress rate.
+  void one_step(bool with_eos = true, bool shep = false, bool again = false, bool mapped = false,
+                bool rate_later = false) {
+    if (E->nl_valid) one_step_t<true>(with_eos, shep, again ? 1 : 0, mapped, rate_later);
+    else one_step_t<false>(with_eos, shep, again ? 1 : 0, mapped, rate_later);
   }
   template <bool NL>
-  void one_step_t(bool with_eos, bool shep, int again) {
+  void one_step_t(bool with_eos, bool shep, int again, bool mapped, bool rate_later) {
     KArgs a = E->args();
     const int B = E->pair_block, G = NL ? lb() : pb();
     // kernel-corrected scenes run kernels that hold the correction's branch
@@ -447,13 +450,19 @@ struct Seq {
       L.go("soil_bdy", k_soil_bdy<DIM, true, NL>, G, B, a, again);
       L.go("mui_soil3", kc ? k_mui_soil3<DIM, NL, true> : k_mui_soil3<DIM, NL, false>, G, B, a, again);
     } else {
-      L.go("dp_adapt", k_dp_adapt, tb(), E->elem_block, a);
+      if (!mapped) L.go("dp_adapt", k_dp_adapt, tb(), E->elem_block, a);
       L.go("soil_bdy", k_soil_bdy<DIM, false, NL>, G, B, a, again);
       L.go("dp_soil", kc ? k_dp_soil<DIM, NL, true> : k_dp_soil<DIM, NL, false>, G, B, a, again);
+      if (!rate_later) L.go("dp_rate", k_dp_rate, tb(), E->elem_block, a);
     }
   }
-  void lf_half(bool eos = false) { L.go("lf_half", k_lf_half, tb(), E->elem_block, E->args(), eos ? 1 : 0); }
-  void lf_full() { L.go("lf_full", k_lf_full, tb(), E->elem_block, E->args()); }
+  // dp: of a fused step's DP
+  void lf_half(bool eos = false, bool dp = false) {
+    L.go("lf_half", dp ? k_lf_half<true> : k_lf_half<false>, tb(), E->elem_block, E->args(), eos ? 1 : 0);
+  }
+  void lf_full(bool dp = false) {
+    L.go("lf_full", dp ? k_lf_full<true> : k_lf_full<false>, tb(), E->elem_block, E->args());
+  }
   void substep(int ti, bool shep_first = false, bool fused = false) {
     if (ti == 1) {
       one_step(true, shep_first);
@@ -468,7 +477,7 @@ struct Seq {
       L.go("rk", k_rk_init, tb(), E->elem_block, a);
       const int m[4] = {1, 2, 2, 1};
       for (int k = 0; k < 4; ++k) {
-        one_step(true, shep_first && k == 0, fused && k > 0);
+        one_step(true, shep_first && k == 0, fused && k > 0, fused && k == 0);
         L.go("rk", k_rk_update, tb(), E->elem_block, a, m[k]);
         if (k < 3) L.go("rk", k_rk_advect4, tb(), E->elem_block, a);
       }
@@ -529,23 +538,25 @@ struct Seq {
     // fluid passes (the boundary pass runs first and reads it right away)
     const bool shep = E->method == kWC;
     shepard(shep, shep);
+    const bool dp = E->method == kDP;
     if (ti == 2) {
-      one_step(false, shep);
-      lf_half(true);
-      one_step(false, false, true);
+      one_step(false, shep, false, true, true);
+      lf_half(true, dp);
+      one_step(false, false, true, true, true);
     } else if (ti == 1) {
-      one_step(false, shep);
+      one_step(false, shep, false, true, true);
     } else {
       substep(4, shep, true);
     }
     const bool lf_in_finish = ti != 4 && !xsph;
     KArgs a = E->args();
     if (xsph) {
-      if (ti != 4) lf_full();
+      if (ti != 4) lf_full(dp);
       if (E->nl_valid) L.go("xsph", k_xsph<DIM, true>, lb(), E->pair_block, a);
       else L.go("xsph", k_xsph<DIM, false>, pb(), E->pair_block, a);
     }
-    L.go("finish", k_finish, tb(), E->elem_block, a, lf_in_finish ? 1 : 0, xsph ? 1 : 0);
+    L.go("finish", dp && lf_in_finish ? k_finish<true> : k_finish<false>, tb(), E->elem_block, a,
+         lf_in_finish ? 1 : 0, xsph ? 1 : 0);
     E->fresh_sort = false;
     if (E->method == kMUI) {
       L.go("mui_regu", k_mui_regu<DIM>, lb(), E->pair_block, a, E->nl_valid ? 1 : 0);

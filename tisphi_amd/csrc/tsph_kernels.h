@@ -384,6 +384,8 @@ __global__ __launch_bounds__(256) void k_scatter(KArgs a) {
 // of the texture path (the global-memory count kept the TD unit ~94 % busy).
 constexpr int kRankStage = 1024;
 __device__ __forceinline__ float wc_eos(const SceneDev& S, float rt);
+__device__ __forceinline__ void dp_adapt_store(const KArgs& a, const SceneDev& S, int p, double (&t)[6], float rt);
+template <bool DPN>
 __global__ __launch_bounds__(256) void k_rank_move(KArgs a, int move_vtmp, int move_mui,
                                                    int move_dp, int fuse_init) {
   __shared__ int32_t win[kRankStage];
@@ -459,11 +461,13 @@ __global__ __launch_bounds__(256) void k_rank_move(KArgs a, int move_vtmp, int m
         a.w.vp[d] = make_float4(v.x, v.y, v.z, pv / (v.w * v.w));
       }
     }
-    // (muI: stress_tmp is formed by the first soil loop; the float records of
-    // DP by the return mapping that starts a one_step)
-    if (t == kSoil && S.method == kDP) {
+    // muI: stress_tmp is formed by the first soil loop.  DP: with the return
+    // mapping that starts the first one_step.
+    if (DPN && t == kSoil) {
+      double q[6];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + d] = a.cur.sig_d[c * st + p];
+      for (int c = 0; c < 6; ++c) q[c] = a.cur.sig_d[c * st + p];
+      dp_adapt_store(a, S, d, q, a.cur.vel[p].w);
     }
   }
 }
@@ -1771,23 +1775,26 @@ __device__ __forceinline__ int dp_flag(const SceneDev& S, const double st[6]) {
   return 1;
 }
 
-__global__ __launch_bounds__(256) void k_dp_adapt(KArgs a) {  // one_step loop 1
-  int s, p;
-  if (!tile_thread(a, s, p)) return;
-  if (a.cur.type[p] != kSoil) return;
-  const SceneDev S = a.scenes[s];
-  const int st = a.stride;
-  double t[6];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) t[c] = a.w.sigt_d[c * st + p];
+// one_step loop 1 of particle p: stress_tmp t mapped back and stored; rt: its
+// density_tmp.
+__device__ __forceinline__ void dp_adapt_store(const KArgs& a, const SceneDev& S, int p, double (&t)[6], float rt) {
   dp_adapt(S, t);
   float sg[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
-    a.w.sigt_d[c * st + p] = t[c];
+    a.w.sigt_d[c * a.stride + p] = t[c];
     sg[c] = (float)t[c];
   }
-  soil_stress_store(a, p, sg, a.cur.vtmp[p].w);
+  soil_stress_store(a, p, sg, rt);
+}
+__global__ __launch_bounds__(256) void k_dp_adapt(KArgs a) {
+  int s, p;
+  if (!tile_thread(a, s, p)) return;
+  if (a.cur.type[p] != kSoil) return;
+  double t[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) t[c] = a.w.sigt_d[c * a.stride + p];
+  dp_adapt_store(a, a.scenes[s], p, t, a.cur.vtmp[p].w);
 }
 
 // calc_d_stress_Bui2008 (solver_sph_dp.py:171-208), FP64.
@@ -1892,14 +1899,23 @@ __device__ __forceinline__ void dp_soil_one(const KArgs& a, const SceneDev& S, i
     soil_dv_pair(qi, qj, mVj, vj.w, gw, t + 10);
   });
   if (!group_head<LN>()) return;
-  const float L[3][3] = {{acc[0], acc[1], acc[2]}, {acc[3], acc[4], acc[5]}, {acc[6], acc[7], acc[8]}};
-  const float dd = acc[9], dv[3] = {acc[10], acc[11], acc[12]};
-  a.w.drho[p] = dd * vi.w;
-  double Ld[3][3], sd[6], ds[6], dq, dqp;
+  const float dv[3] = {acc[10], acc[11], acc[12]};
 #pragma unroll
-  for (int aa = 0; aa < 3; ++aa)
+  for (int c = 0; c < 9; ++c) a.w.gradv[c * a.stride + p] = acc[c];
+  a.w.drho[p] = acc[9] * vi.w;
+  a.w.dv[p] = soil_dv_finish(S, dv, vi);
+}
+// The stress rate of the velocity gradient that dp_soil_one() left, by a
+// pass (or part of one) of a lane per particle: as the pair pass's epilogue a
+// quarter of its lanes ran these ~500 FP64 instructions, at the registers
+// they take (128, four waves per SIMD).  85 k in 2D: the pass 28 -> 21 us; in
+// a fused step the rate joins the half step and the last update (3 us each)
+// and the return mapping before it (8 us, twice) the pass ahead of it.
+__device__ __forceinline__ void dp_rate(const KArgs& a, const SceneDev& S, int p, double (&ds)[6]) {
+  const int st = a.stride;
+  double Ld[3][3], sd[6], dq, dqp;
 #pragma unroll
-    for (int bb = 0; bb < 3; ++bb) Ld[aa][bb] = (double)L[aa][bb];
+  for (int c = 0; c < 9; ++c) Ld[c / 3][c % 3] = (double)a.w.gradv[c * st + p];
 #pragma unroll
   for (int c = 0; c < 6; ++c) sd[c] = a.w.sigt_d[c * st + p];
   dp_bui2008(S, Ld, sd, ds, dq, dqp);
@@ -1907,7 +1923,13 @@ __device__ __forceinline__ void dp_soil_one(const KArgs& a, const SceneDev& S, i
   for (int c = 0; c < 6; ++c) a.w.dsig_d[c * st + p] = ds[c];
   a.w.dseq[p] = dq;
   a.w.dseqp[p] = dqp;
-  a.w.dv[p] = soil_dv_finish(S, dv, vi);
+}
+__global__ __launch_bounds__(256) void k_dp_rate(KArgs a) {
+  int s, p;
+  if (!tile_thread(a, s, p)) return;
+  if (a.cur.type[p] != kSoil) return;
+  double ds[6];
+  dp_rate(a, a.scenes[s], p, ds);
 }
 template <int DIM, bool NL, bool KC>
 __global__ __launch_bounds__(256) void k_dp_soil(KArgs a, int again) {
@@ -1960,11 +1982,15 @@ __global__ __launch_bounds__(256) void k_dp_adv(KArgs a) {
 
 // =============================================================== integrators
 // advect_LF_half (solver_sph_base.py:96-104).
+// DPN: in a fused DP step, with the stress rate before and the return mapping
+// of the next one_step after.
+template <bool DPN>
 __global__ __launch_bounds__(256) void k_lf_half(KArgs a, int eos) {
   int s, p;
   if (!tile_thread(a, s, p)) return;
   const SceneDev S = a.scenes[s];
   const int t = a.cur.type[p];
+  float rt = 0.0f;
   if (is_real(t)) {
     float4 vt = a.cur.vtmp[p];
     const float4 d = a.w.dv[p];
@@ -1974,6 +2000,7 @@ __global__ __launch_bounds__(256) void k_lf_half(KArgs a, int eos) {
     vt.y += S.half_dt * d.y;
     vt.z += S.half_dt * d.z;
     a.cur.vtmp[p] = vt;
+    rt = vt.w;
     // the EOS of the next one_step (solver_sph_wc.py:88), fused
     if (eos && S.method == kWC && t == kFluid) {
       const float pv = wc_eos(S, vt.w);
@@ -1984,12 +2011,20 @@ __global__ __launch_bounds__(256) void k_lf_half(KArgs a, int eos) {
   if (t == kSoil && S.method == kDP) {
     const int st = a.stride;
     const double h = 0.5 * S.dt_d;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + p] += h * a.w.dsig_d[c * st + p];
+    if (DPN) {
+      double ds[6], q[6];
+      dp_rate(a, S, p, ds);
+      for (int c = 0; c < 6; ++c) q[c] = a.w.sigt_d[c * st + p] + h * ds[c];
+      dp_adapt_store(a, S, p, q, rt);
+    } else {
+      for (int c = 0; c < 6; ++c) a.w.sigt_d[c * st + p] += h * a.w.dsig_d[c * st + p];
+    }
   }
 }
 
 // advect_LF (:106-114); advect_SE (:79-87) is the same update.
+// DPN: in a fused DP step, with the stress rate before.
+template <bool DPN>
 __global__ __launch_bounds__(256) void k_lf_full(KArgs a) {
   int s, p;
   if (!tile_thread(a, s, p)) return;
@@ -2008,8 +2043,10 @@ __global__ __launch_bounds__(256) void k_lf_full(KArgs a) {
   }
   if (t == kSoil && S.method == kDP) {
     const int st = a.stride;
+    double ds[6];
+    if (DPN) dp_rate(a, S, p, ds);
 #pragma unroll
-    for (int c = 0; c < 6; ++c) a.cur.sig_d[c * st + p] += S.dt_d * a.w.dsig_d[c * st + p];
+    for (int c = 0; c < 6; ++c) a.cur.sig_d[c * st + p] += S.dt_d * (DPN ? ds[c] : a.w.dsig_d[c * st + p]);
   }
 }
 
@@ -2017,6 +2054,8 @@ __global__ __launch_bounds__(256) void k_lf_full(KArgs a) {
 // advect_pos -> the elementwise part of advect_something (WC chk_density,
 // DP return mapping, muI phase 1).  Same per-particle arithmetic as the
 // separate passes.
+// DPN: in a fused DP step, with the stress rate before.
+template <bool DPN>
 __global__ __launch_bounds__(256) void k_finish(KArgs a, int do_lf, int use_xsph) {
   int s, p;
   if (!tile_thread(a, s, p)) return;
@@ -2036,8 +2075,10 @@ __global__ __launch_bounds__(256) void k_finish(KArgs a, int do_lf, int use_xsph
       if (isnan(v.x) || isnan(v.y) || isnan(v.z) || isnan(v.w)) atomicAdd(&a.w.status[2 * s + 1], 1ull);
     }
     if (t == kSoil && S.method == kDP) {
+      double ds[6];
+      if (DPN) dp_rate(a, S, p, ds);
 #pragma unroll
-      for (int c = 0; c < 6; ++c) a.cur.sig_d[c * st + p] += S.dt_d * a.w.dsig_d[c * st + p];
+      for (int c = 0; c < 6; ++c) a.cur.sig_d[c * st + p] += S.dt_d * (DPN ? ds[c] : a.w.dsig_d[c * st + p]);
     }
   }
   float4 P = a.cur.pos[p];
