@@ -152,3 +152,32 @@ def test_stress_regularisation_sums(dim, kernel):
         moved += bool((new[i] != c[i]).any())
         longest = max(longest, j.size)
     assert moved > 0 and longest > 64
+
+
+def test_read_outs_of_several_stages():
+    """Fields of every row size come back as they were sent, also where a
+    read-out takes several turns of its staging memory and the last is short."""
+    sc = build_scene(tiny_cfg(method=2, dim=2, r=0.001, domain=(0.6, 0.6, 0.1), block=(0.5, 0.5, 0.0)))
+    assert sc.n * 24 > 2.5 * 2 ** 19 and (sc.n * 4) % 2 ** 19
+    rng = np.random.default_rng(1)
+    eng = L.Engine(2, 2, sc.n, sc.geo.grid_num_total, 1)
+    slot = eng.add_scene(sc.desc())
+    L.upload_scene(eng, slot, sc)
+    sent = {"vel": rng.normal(size=(sc.n, 3)), "density": rng.uniform(900, 1100, sc.n),
+            "stress": rng.normal(size=(sc.n, 6)), "stress_tmp": rng.normal(size=(sc.n, 6))}
+    ints = {"id0": rng.permutation(sc.n), "obj_id": rng.integers(0, 3, sc.n), "type": sc.mat_type}
+    for f, v in list(sent.items()) + list(ints.items()):
+        eng.upload(slot, f, v)
+    for f, v in sent.items():
+        np.testing.assert_array_equal(eng.download(slot, f), v.astype(np.float32).astype(np.float64), err_msg=f)
+    for f, v in ints.items():
+        np.testing.assert_array_equal(eng.download(slot, f), v, err_msg=f)
+    eng.run("sort")
+    cell, start = eng.download(slot, "cell"), eng.download(slot, "cell_start")
+    np.testing.assert_array_equal(np.diff(start), np.bincount(cell, minlength=start.size - 1))
+    off, pos = eng.download(slot, "offset"), eng.download(slot, "pos")
+    gn, g = sc.geo.grid_num, sc.geo.grid_size
+    c = np.stack(np.unravel_index(cell, gn), 1)
+    want = sc.geo.vdomain_start[None] + c * g + off
+    np.testing.assert_array_equal(pos[:, :2], want[:, :2])
+    eng.close()

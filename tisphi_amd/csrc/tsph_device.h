@@ -120,7 +120,6 @@ struct PWork {
   int32_t* bsum;     // scan block sums
   unsigned long long* status;  // per slot: escaped, NaN
   double* gpart;     // globals partials per tile (4 each)
-  double* gout;      // globals per slot (4 each)
   uint32_t* nl;      // neighbour lists, blocked per 64-particle tile (nl_base / nl_at)
   int32_t* nlc;      // neighbour count per particle (> nl_cap: walk instead)
   int32_t* tflag;    // per tile: what the pair passes find there (kTile*)

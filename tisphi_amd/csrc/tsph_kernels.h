@@ -2363,13 +2363,12 @@ __device__ __forceinline__ double wave_max(double v) {
   for (int d = 32; d >= 1; d >>= 1) v = fmax(v, __shfl_xor(v, d, 64));
   return v;
 }
-__global__ __launch_bounds__(256) void k_globals_tile(KArgs a) {
-  const int w = wave_id();
-  const int2 t = a.tiles[w];
-  if (t.x < 0) return;
-  const int s = t.x;
-  const SceneDev S = a.scenes[s];
-  const int p = t.y + (int)(threadIdx.x & 63);
+__global__ __launch_bounds__(256) void k_globals_tile(KArgs a, int slot) {
+  const SceneDev S = a.scenes[slot];
+  const int k = wave_id();
+  if (k >= S.n_tiles) return;
+  const int w = S.tile_first + k;
+  const int p = a.tiles[w].y + (int)(threadIdx.x & 63);
   double fr = -INFINITY, pe = 0.0, ke = 0.0, m = 0.0;
   if (p < S.pbase + S.n && is_flow(a.cur.type[p])) {
     int cc[3];
@@ -2397,11 +2396,9 @@ __global__ __launch_bounds__(256) void k_globals_tile(KArgs a) {
     o[3] = m;
   }
 }
-__global__ __launch_bounds__(256) void k_globals_scene(KArgs a, int nslots) {
-  const int s = blockIdx.x;
-  if (s >= nslots) return;
-  const SceneDev S = a.scenes[s];
-  if (!S.active) return;
+// out: the four, in pinned host memory.
+__global__ __launch_bounds__(256) void k_globals_scene(KArgs a, int slot, double* __restrict__ out) {
+  const SceneDev S = a.scenes[slot];
   double fr = -INFINITY, pe = 0.0, ke = 0.0, m = 0.0;
   for (int k = threadIdx.x; k < S.n_tiles; k += blockDim.x) {
     const double* o = a.w.gpart + 4 * (size_t)(S.tile_first + k);
@@ -2430,11 +2427,10 @@ __global__ __launch_bounds__(256) void k_globals_scene(KArgs a, int nslots) {
       ke += red[2][k];
       m += red[3][k];
     }
-    double* o = a.w.gout + 4 * s;
-    o[0] = fr;
-    o[1] = pe;
-    o[2] = ke;
-    o[3] = m;
+    out[0] = fr;
+    out[1] = pe;
+    out[2] = ke;
+    out[3] = m;
   }
 }
 
@@ -2717,7 +2713,7 @@ __global__ __launch_bounds__(256) void k_color_range_tile(KArgs a, int slot) {
 }
 __global__ __launch_bounds__(256) void k_color_range_scene(KArgs a, int slot, double given_max,
                                                            double given_min, int fix_max,
-                                                           int fix_min) {
+                                                           int fix_min, double* __restrict__ out) {
   const SceneDev S = a.scenes[slot];
   double hi = -INFINITY, lo = INFINITY;
   for (int k = threadIdx.x; k < S.n_tiles; k += blockDim.x) {
@@ -2740,8 +2736,10 @@ __global__ __launch_bounds__(256) void k_color_range_scene(KArgs a, int slot, do
       lo = fmin(lo, red[1][k]);
     }
     // vmax if givenmax == -1 or (vmax < givenmax and not fixmax) else givenmax
-    a.w.crange[2 * slot] = (given_max == -1.0 || (hi < given_max && !fix_max)) ? hi : given_max;
-    a.w.crange[2 * slot + 1] = (given_min == -1.0 || (lo > given_min && !fix_min)) ? lo : given_min;
+    const double vmax = (given_max == -1.0 || (hi < given_max && !fix_max)) ? hi : given_max;
+    const double vmin = (given_min == -1.0 || (lo > given_min && !fix_min)) ? lo : given_min;
+    a.w.crange[2 * slot] = out[0] = vmax;
+    a.w.crange[2 * slot + 1] = out[1] = vmin;
   }
 }
 
@@ -2773,6 +2771,46 @@ __global__ __launch_bounds__(256) void k_set_color(KArgs a, int slot, int group,
     c = a.w.c0[(size_t)S.pbase + (size_t)a.cur.id0[p]];
   }
   a.w.rgb[p] = c;
+}
+
+// ================================================================= read-out
+// A field of one scene in the layout its caller reads: `comps` values per
+// particle, double or int32.  Written straight into pinned host memory, in
+// whole lines; the reads are of the engine's own layout.
+enum PackKind { kPackF4, kPackPos, kPackF, kPackD, kPackI, kPackB, kPackRec, kPackStart };
+struct Pack {
+  const void* src;      // the scene's first entry
+  const int32_t* cell;  // kPackPos
+  int kind, comps;
+  int lane0;            // kPackF4: first of the float4's
+  int64_t st;           // kPackF, kPackD: stride between the components
+  int dim, gn1, gn2;    // kPackPos
+  double vds[3], grid;
+};
+__global__ __launch_bounds__(256) void k_pack(Pack k, int64_t first, int m, void* __restrict__ out) {
+  const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (e >= m) return;
+  const int q = e / k.comps, c = e - q * k.comps;
+  const int64_t i = first + q;
+  double v = 0.0;
+  switch (k.kind) {
+    case kPackF4: v = (double)((const float*)k.src)[4 * i + k.lane0 + c]; break;
+    case kPackPos: {
+      const int32_t key = k.cell[i];
+      const int yz = k.gn1 * k.gn2;
+      const int x = key / yz, y = (key - x * yz) / k.gn2, z = key - x * yz - y * k.gn2;
+      const int cc = c == 0 ? x : (c == 1 ? y : z);
+      if (!(c == 2 && k.dim == 2)) v = k.vds[c] + (double)cc * k.grid + (double)((const float*)k.src)[4 * i + c];
+      break;
+    }
+    case kPackF: v = (double)((const float*)k.src)[c * k.st + i]; break;
+    case kPackD: v = ((const double*)k.src)[c * k.st + i]; break;
+    case kPackRec: v = (double)((const float*)k.src)[kRec * i + c]; break;
+    case kPackI: ((int32_t*)out)[e] = ((const int32_t*)k.src)[i]; return;
+    case kPackB: ((int32_t*)out)[e] = ((const int8_t*)k.src)[i]; return;
+    case kPackStart: ((int32_t*)out)[e] = ((const int32_t*)k.src)[i] - ((const int32_t*)k.src)[0]; return;
+  }
+  ((double*)out)[e] = v;
 }
 
 }  // namespace tsph
