@@ -181,3 +181,32 @@ def test_read_outs_of_several_stages():
     want = sc.geo.vdomain_start[None] + c * g + off
     np.testing.assert_array_equal(pos[:, :2], want[:, :2])
     eng.close()
+
+
+@pytest.mark.parametrize("method,dim,ti,xsph", [(1, 2, 4, False), (1, 3, 4, True), (2, 2, 4, True), (2, 3, 1, False),
+                                                (3, 2, 4, True), (3, 2, 2, False), (3, 3, 2, True), (3, 2, 1, False)])
+def test_fused_integrators_equal_the_passes(method, dim, ti, xsph):
+    """The fused step's launches (stages of RK4, DP's rate and mapping within
+    their neighbours) give the bits of the passes run one by one."""
+    sc = build_scene(tiny_cfg(method=method, dim=dim, xsph=xsph, ti=ti, domain=(0.4, 0.3, 0.08),
+                              block=(0.2, 0.15, 0.06)))
+    rng = np.random.default_rng(7)
+    flow = sc.mat_type > 0
+    sc.vel[flow, :dim] = rng.uniform(-1.0, 1.0, (int(flow.sum()), dim))
+    fields = STATE + ["density_tmp", "v_tmp", "m_V", "d_density"]
+    if method != 1:
+        fields += ["stress", "stress_tmp", "strain_equ", "d_strain_equ"]
+    if method == 3:
+        fields += ["strain_equ_p", "flag_retmap", "d_stress", "d_strain_equ_p"]
+    out = []
+    for fused in (False, True):
+        eng = L.Engine(method, dim, sc.n, sc.geo.grid_num_total, 1)
+        slot = eng.add_scene(sc.desc())
+        L.upload_scene(eng, slot, sc)
+        for _ in range(1 if fused else 4):
+            eng.step(4) if fused else eng.run("step")
+        out.append({f: eng.download(slot, f) for f in fields})
+        eng.close()
+    for f in fields:
+        np.testing.assert_array_equal(out[1][f], out[0][f], err_msg=f)
+    assert np.isfinite(out[0]["vel"]).all()

@@ -467,12 +467,12 @@ struct Seq {
   void lf_full(bool dp = false) {
     L.go("lf_full", dp ? k_lf_full<true> : k_lf_full<false>, tb(), E->elem_block, E->args());
   }
-  void substep(int ti, bool shep_first = false, bool fused = false) {
+  void substep(int ti) {
     if (ti == 1) {
-      one_step(true, shep_first);
+      one_step();
       lf_full();
     } else if (ti == 2) {
-      one_step(true, shep_first);
+      one_step();
       lf_half();
       one_step();
       lf_full();
@@ -481,7 +481,7 @@ struct Seq {
       L.go("rk", k_rk_init, tb(), E->elem_block, a);
       const int m[4] = {1, 2, 2, 1};
       for (int k = 0; k < 4; ++k) {
-        one_step(true, shep_first && k == 0, fused && k > 0, fused && k == 0);
+        one_step();
         L.go("rk", k_rk_update, tb(), E->elem_block, a, m[k]);
         if (k < 3) L.go("rk", k_rk_advect4, tb(), E->elem_block, a);
       }
@@ -550,7 +550,10 @@ struct Seq {
     } else if (ti == 1) {
       one_step(false, shep, false, true, true);
     } else {
-      substep(4, shep, true);
+      for (int k = 0; k < 4; ++k) {
+        one_step(false, shep && k == 0, k > 0, true, true);
+        L.go("rk", dp ? k_rk_stage<true> : k_rk_stage<false>, tb(), E->elem_block, E->args(), k);
+      }
     }
     const bool lf_in_finish = ti != 4 && !xsph;
     KArgs a = E->args();

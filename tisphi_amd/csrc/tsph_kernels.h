@@ -2230,7 +2230,7 @@ __global__ __launch_bounds__(256) void k_rk_init(KArgs a) {
     a.w.drho_rk[p] = 0.f;
     a.w.dv_rk[p] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  if (t == kSoil) {
+  if (t == kSoil && a.w.dsig_rk) {  // DP
     const int st = a.stride;
     for (int c = 0; c < 6; ++c) a.w.dsig_rk[c * st + p] = 0.0;
   }
@@ -2298,6 +2298,77 @@ __global__ __launch_bounds__(256) void k_rk_advect(KArgs a) {
     const int st = a.stride;
     for (int c = 0; c < 6; ++c)
       a.cur.sig_d[c * st + p] += S.dt_d / 6.0 * a.w.dsig_rk[c * st + p];
+  }
+}
+// In a fused step, all that lies between one_step k (0..3) and the next: the
+// update of the sums (0 + the first rates, as the passes one by one form it),
+// the advance of v_tmp or, last, of v, and the EOS (DPN: the stress rate and
+// the return mapping) around them.  Bound by launches at the sizes RK4 is
+// used at: 4 of these in place of 13 launches (1 + 4 + 3 + 1 here, 4 EOS),
+// 25 k particles in 2D 132 -> 113 us per step.
+template <bool DPN>
+__global__ __launch_bounds__(256) void k_rk_stage(KArgs a, int k) {
+  int s, p;
+  if (!tile_thread(a, s, p)) return;
+  const SceneDev S = a.scenes[s];
+  const int t = a.cur.type[p];
+  const int m = k == 1 || k == 2 ? 2 : 1;
+  const float mf = (float)m;
+  float rt = 0.0f;
+  if (is_real(t)) {
+    const float dr = a.w.drho[p];
+    const float4 d = a.w.dv[p];
+    float4 R = make_float4(0.f, 0.f, 0.f, 0.f);  // w: the density's
+    if (k > 0) {
+      R = a.w.dv_rk[p];
+      R.w = a.w.drho_rk[p];
+    }
+    R.x += d.x * mf;
+    R.y += d.y * mf;
+    R.z += d.z * mf;
+    R.w += dr * mf;
+    float4 v = a.cur.vel[p];
+    if (k < 3) {
+      a.w.drho_rk[p] = R.w;
+      a.w.dv_rk[p] = R;
+      float4 vt;
+      vt.w = S.half_dt * dr + v.w;
+      a.cur.pos[p].w = a.cur.mass[p] / vt.w;
+      vt.x = S.half_dt * d.x + v.x;
+      vt.y = S.half_dt * d.y + v.y;
+      vt.z = S.half_dt * d.z + v.z;
+      a.cur.vtmp[p] = vt;
+      rt = vt.w;
+      if (S.method == kWC && t == kFluid) {
+        const float pv = wc_eos(S, vt.w);
+        a.w.p[p] = pv;
+        a.w.vp[p] = make_float4(vt.x, vt.y, vt.z, pv / (vt.w * vt.w));
+      }
+    } else {
+      v.w += S.dt6 * R.w;
+      a.cur.pos[p].w = a.cur.mass[p] / v.w;
+      v.x += S.dt6 * R.x;
+      v.y += S.dt6 * R.y;
+      v.z += S.dt6 * R.z;
+      a.cur.vel[p] = v;
+      if (isnan(v.x) || isnan(v.y) || isnan(v.z) || isnan(v.w)) atomicAdd(&a.w.status[2 * s + 1], 1ull);
+    }
+  }
+  if (DPN && t == kSoil) {
+    const int st = a.stride;
+    double ds[6], q[6];
+    dp_rate(a, S, p, ds);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      const double r = (k > 0 ? a.w.dsig_rk[c * st + p] : 0.0) + ds[c] * m;
+      if (k < 3) {
+        a.w.dsig_rk[c * st + p] = r;
+        q[c] = 0.5 * S.dt_d * ds[c] + a.cur.sig_d[c * st + p];
+      } else {
+        a.cur.sig_d[c * st + p] += S.dt_d / 6.0 * r;
+      }
+    }
+    if (k < 3) dp_adapt_store(a, S, p, q, rt);
   }
 }
 
