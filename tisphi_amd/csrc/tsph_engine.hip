@@ -389,7 +389,11 @@ struct Seq {
            E->w.cflow, n);
       L.go("scatter", k_scatter, tb(), eb, a);
     }
-    L.go("rank_move", E->method == kDP ? k_rank_move<true> : k_rank_move<false>, (E->cap + eb - 1) / eb, eb, a, 1, E->method == kMUI ? 1 : 0,
+    // v_tmp of real particles is set by the fused init, and of walls by the
+    // first pass of a WC or DP step (muI's first reads the walls' last)
+    const int move_vtmp = fuse_init && E->method != kMUI ? 0 : 1;
+    L.go("rank_move", E->method == kDP ? k_rank_move<true> : k_rank_move<false>, (E->cap + eb - 1) / eb, eb, a,
+         move_vtmp, E->method == kMUI ? 1 : 0,
          E->method == kDP ? 1 : 0, fuse_init ? 1 : 0);
     E->parity ^= 1;
     E->nl_valid = false;
