@@ -251,7 +251,7 @@ class Engine:
         check(load().tsph_set_block(self.h, int(pair), int(elem)))
 
     def set_cell_tile(self, stage):
-        """Candidates one wave stages in LDS per row offset in the mode-2
+        """Candidates one wave stages in LDS at a time in the mode-2
         list build: 128, 256 (default) or 512."""
         check(load().tsph_set_cell_tile(self.h, int(stage)))
 

@@ -4,7 +4,7 @@ The reference runs one scene per process (run_simulation.py:23).  Here an
 engine holds up to thousands of resident scenes of one method and
 dimension; every kernel of a step covers all of them (one 64-particle tile
 per wave, tiles of every scene in one grid), so a step of 256 scenes costs
-the same ~30 launches as a step of one.  Per-scene arithmetic does not
+the same launches as a step of one.  Per-scene arithmetic does not
 depend on the other residents: each scene keeps its own particle and cell
 ranges, its own sort order and its own tile-aligned reductions, so results
 are bitwise identical alone and in a batch.

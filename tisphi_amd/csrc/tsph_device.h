@@ -458,7 +458,10 @@ __host__ __device__ __forceinline__ size_t nl_at(int k) {
 // same order as with one lane, so the sums have the same bits.
 // Lists are padded to a multiple of kNlPad entries with the null particle
 // (m_V = 0: every term it gives is +-0, which changes no sum, since a sum
-// that starts at +0 is never -0 in round-to-nearest).
+// that starts at +0 is never -0 in round-to-nearest).  Bound by vector issue
+// on large scenes, by latency on small ones.  Against a lane per particle:
+// WC fluid pass 1090 -> 925 us at 4.5 M particles in 3D, step 365 -> 200 at
+// 191 k in 3D and 94 -> 58 at 9 k in 2D (with the list build's part).
 constexpr int kMaxBlock = 256;  // largest threads per block of a pair kernel
 constexpr int kNlPad = 4;
 constexpr int kLanes = 4;
