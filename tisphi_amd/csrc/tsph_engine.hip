@@ -833,10 +833,24 @@ int alloc_read_stage(tsph_engine* E) {
   return TSPH_OK;
 }
 
+// The calling thread's device set to the engine's, as a copy on its stream
+// would not need but a launch does.
+struct OnDevice {
+  int prev = -1;
+  explicit OnDevice(int device) {
+    int d = -1;
+    if (hipGetDevice(&d) == hipSuccess && d != device && hipSetDevice(device) == hipSuccess) prev = d;
+  }
+  ~OnDevice() {
+    if (prev >= 0) (void)hipSetDevice(prev);
+  }
+};
+
 int read_out(tsph_engine* E, const Pack& k, int64_t n, void* host) {
   if (n == 0) return TSPH_OK;
   if (!k.src) return fail(TSPH_ERR_INVALID_ARG, "field not held by this engine's method");
   std::lock_guard<std::mutex> lock(E->reading);
+  const OnDevice on(E->device);
   const size_t row = (size_t)k.comps * (k.kind == kPackI || k.kind == kPackB || k.kind == kPackStart ? 4 : 8);
   const int64_t per = (int64_t)(kReadHalf / row), turns = (n + per - 1) / per;
   auto rows = [&](int64_t t) { return std::min(per, n - t * per); };
