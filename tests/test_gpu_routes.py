@@ -210,3 +210,37 @@ def test_fused_integrators_equal_the_passes(method, dim, ti, xsph):
     for f in fields:
         np.testing.assert_array_equal(out[1][f], out[0][f], err_msg=f)
     assert np.isfinite(out[0]["vel"]).all()
+
+
+@pytest.mark.parametrize("method,dim", [(1, 2), (1, 3), (2, 2), (2, 3), (3, 2), (3, 3)])
+def test_padding_adds_nothing_to_infinite_sums(method, dim):
+    """The entries that fill up a list's last quad add nothing, also where a
+    particle's own state makes its terms infinite: 0 times infinity is not a
+    number, so they may not be formed from a neighbour of no volume.  Two
+    to six flow particles in a row, the first infinitely fast."""
+    for n in range(2, 7):
+        sc = build_scene(tiny_cfg(method=method, dim=dim, domain=(0.4, 0.4, 0.4)))
+        flow = np.flatnonzero(sc.mat_type > 0)
+        # the others far from the row and from each other's reach
+        d, top = 2 * sc.geo.particle_radius, 0.3
+        sc.pos[flow, 0] = 0.3
+        sc.pos[flow[:n], :dim] = np.array([0.1, top, 0.2])[:dim] + (np.arange(n) * 0.4 * d)[:, None] / n
+        sc.vel[:] = 0.0
+        sc.vel[flow[0], 0] = -np.inf
+        out = []
+        for mode in (0, 1, 2):
+            eng = L.Engine(method, dim, sc.n, sc.geo.grid_num_total, 1)
+            eng.set_neighbor_list(mode)
+            slot = eng.add_scene(sc.desc())
+            L.upload_scene(eng, slot, sc)
+            for what in ("sort", "shepard", "init_tmp", "one_step"):
+                eng.run(what)
+            out.append({f: eng.download(slot, f) for f in ("id0", "d_density", "d_vel")})
+            if mode:
+                i = np.flatnonzero(out[-1]["id0"] == flow[0])[0]
+                assert eng.neighbor_lists(slot)[0][i] == n - 1
+            eng.close()
+        assert np.isinf(out[0]["d_density"]).any()
+        for o in out[1:]:
+            for f in o:
+                np.testing.assert_array_equal(o[f], out[0][f], err_msg=f"{n} particles: {f}")

@@ -456,9 +456,9 @@ __host__ __device__ __forceinline__ size_t nl_at(int k) {
 // entries k + q, and every lane then adds the four terms in list order, the
 // other lanes' read through DPP quad permutations: the same additions in the
 // same order as with one lane, so the sums have the same bits.
-// Lists are padded to a multiple of kNlPad entries with the null particle
-// (m_V = 0: every term it gives is +-0, which changes no sum, since a sum
-// that starts at +0 is never -0 in round-to-nearest).  Bound by vector issue
+// Lists are padded to a multiple of kNlPad entries with the null particle,
+// whose terms are replaced by +0 (which changes no sum, since a sum that
+// starts at +0 is never -0 in round-to-nearest).  Bound by vector issue
 // on large scenes, by latency on small ones.  Against a lane per particle:
 // WC fluid pass 1090 -> 925 us at 4.5 M particles in 3D, step 365 -> 200 at
 // 191 k in 3D and 94 -> 58 at 9 k in 2D (with the list build's part).
@@ -472,6 +472,13 @@ __device__ __forceinline__ float group_read(float x) {
   static_assert(L == 4, "a quad");
   constexpr int ctrl = SRC * 0x55;  // quad_perm [SRC, SRC, SRC, SRC]
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+// on ? x : +0 as a select (the guard keeps the compiler from forming x in a
+// branch, which also keeps the quad's additions from reading it through
+// their DPP operand).
+__device__ __forceinline__ float term_if(bool on, float x) {
+  asm("" : "+v"(x));
+  return on ? x : 0.0f;
 }
 // acc += the terms of the group's lanes, lane 0 first.
 template <int L, int NT>
@@ -604,14 +611,17 @@ __device__ __forceinline__ void sum_list(const SceneDev& S, const uint32_t* __re
     e0 = f0;
     e1 = f1;
   }
-  if (k < n) {
-    pair(e0, rec(e0), t);
+  // the list's end: the padding's terms are left out, which an infinite state
+  // of the particle itself would make 0 * infinity
+  auto last = [&](uint32_t e, int kq) {
+    const bool in = kq + (int)(threadIdx.x & 3) < n;
+    pair(e, rec(e), t);
+#pragma unroll
+    for (int c = 0; c < NT; ++c) t[c] = term_if(in, t[c]);
     ordered_add<4>(acc, t);
-  }
-  if (k + 4 < n) {
-    pair(e1, rec(e1), t);
-    ordered_add<4>(acc, t);
-  }
+  };
+  if (k < n) last(e0, k);
+  if (k + 4 < n) last(e1, k + 4);
 }
 
 }  // namespace tsph

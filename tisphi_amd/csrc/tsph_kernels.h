@@ -580,13 +580,6 @@ __device__ __forceinline__ void sum_pairs_k(const SceneDev& S, const KArgs& a, i
     sum_pairs<DIM, NL, L>(S, a, p, o, acc, [&](int j, float x, float y, float z, float r2, float mVj,
                                                float (&t)[NT]) { fn(KTag<0>{}, j, x, y, z, r2, mVj, t); });
 }
-// on ? x : +0 as a select (the guard keeps the compiler from forming x in a
-// branch, which also keeps the quad's additions from reading it through
-// their DPP operand).
-__device__ __forceinline__ float term_if(bool on, float x) {
-  asm("" : "+v"(x));
-  return on ? x : 0.0f;
-}
 // A term that no neighbour of another kind adds: +0 leaves a sum's bits.
 template <int NT>
 __device__ __forceinline__ void no_terms(float (&t)[NT]) {
