@@ -244,3 +244,36 @@ def test_padding_adds_nothing_to_infinite_sums(method, dim):
         for o in out[1:]:
             for f in o:
                 np.testing.assert_array_equal(o[f], out[0][f], err_msg=f"{n} particles: {f}")
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("tile", [128, 512])
+def test_lists_of_particles_out_of_cell_order(dim, tile):
+    """Positions uploaded after the sort: the particles of a tile are in any
+    order, and every list mode still walks each one's own cells."""
+    sc = build_scene(tiny_cfg(dim=dim, domain=(0.3, 0.3, 0.12), block=(0.15, 0.12, 0.06)))
+    for share in (0.02, 1.0):  # a few particles moved, and all
+        out = []
+        for mode in (0, 1, 2):
+            eng = L.Engine(sc.method, dim, sc.n, sc.geo.grid_num_total, 1)
+            eng.set_neighbor_list(mode)
+            eng.set_cell_tile(tile)
+            slot = eng.add_scene(sc.desc())
+            L.upload_scene(eng, slot, sc)
+            eng.run("sort")
+            pos, flow = eng.download(slot, "pos"), np.flatnonzero(eng.download(slot, "type") == 1)
+            rng = np.random.default_rng(4)
+            some = rng.choice(flow, max(2, int(share * flow.size)), replace=False)
+            pos[some] = pos[rng.permutation(some)]
+            eng.upload(slot, "pos", pos)
+            for what in ("shepard", "init_tmp", "one_step"):
+                eng.run(what)
+            out.append({f: eng.download(slot, f) for f in ("cspm_f", "d_density", "d_vel")})
+            if mode:
+                out[-1]["lists"] = eng.neighbor_lists(slot)
+            eng.close()
+        for m, o in enumerate(out[1:], 1):
+            for f in out[0]:
+                np.testing.assert_array_equal(o[f], out[0][f], err_msg=f"mode {m}, share {share}: {f}")
+        for a, b in zip(out[1]["lists"], out[2]["lists"]):
+            np.testing.assert_array_equal(a, b)

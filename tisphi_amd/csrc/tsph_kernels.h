@@ -773,15 +773,27 @@ __global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build_lds(KArgs a, int 
     unsigned long long todo = __ballot(live);
 #pragma unroll 1
     while (todo) {
-      // the lanes of the next row; sorted by cell, so they are consecutive
+      // the lanes of the next row (consecutive in cell order)
       const int l0 = __builtin_ctzll(todo);
       const int R = __builtin_amdgcn_readlane(row, l0);
       bool act = row == R;
       const unsigned long long mine = __ballot(act);
       todo &= ~mine;
       const int l1 = 63 - __builtin_clzll(mine);
-      const int wlo = max(__builtin_amdgcn_readlane(f, l0) - 1, 0);
-      const int whi = min(__builtin_amdgcn_readlane(f, l1) + 1, gf - 1);
+      int f0 = __builtin_amdgcn_readlane(f, l0), f1 = __builtin_amdgcn_readlane(f, l1);
+      // Uploads since the sort (no flags then) may leave particles out of cell
+      // order: the row's window is that of its outermost lanes, and a particle
+      // may stand among the candidates of another cell than its own.
+      if (!use_cflow) {
+        f0 = act ? f : INT32_MAX;
+        f1 = act ? f : -1;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          f0 = min(f0, __shfl_xor(f0, d, 64));
+          f1 = max(f1, __shfl_xor(f1, d, 64));
+        }
+      }
+      const int wlo = max(f0 - 1, 0), whi = min(f1 + 1, gf - 1);
       const int rx = DIM == 3 ? R / gy : R, ry = DIM == 3 ? R - rx * gy : 0;
       const bool inx = rx + dx >= 0 && rx + dx < gx;
       // A boundary particle records nothing if no stencil cell holds a flow
@@ -885,7 +897,7 @@ __global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build_lds(KArgs a, int 
               // candidates past the lane's cell, and the particle itself
               if (m < 32) w &= m > 0 ? ~(0xFFFFFFFFu >> m) : 0u;
               const int32_t j = jlo + w0 + lo;
-              if (dx == 0 && dy == 0 && dz == 0) {
+              if (!use_cflow || (dx == 0 && dy == 0 && dz == 0)) {
                 const int i = p - j;
                 if (i >= 0 && i < 32) w &= ~(0x80000000u >> i);
               }
