@@ -277,3 +277,39 @@ def test_lists_of_particles_out_of_cell_order(dim, tile):
                 np.testing.assert_array_equal(o[f], out[0][f], err_msg=f"mode {m}, share {share}: {f}")
         for a, b in zip(out[1]["lists"], out[2]["lists"]):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("between", [False, True])  # a step between removal and addition
+def test_scene_in_a_freed_range_is_empty_until_sorted(between):
+    """A scene that takes the cells of a removed one has no neighbours before
+    its first sort, as in a new engine, and the other scenes keep theirs."""
+    low, mid, top = (shaken(2, b, s) for s, b in enumerate([(0.3, 0.2, 0.0), (0.4, 0.3, 0.0), (0.2, 0.4, 0.0)]))
+    new = build_scene(tiny_cfg(dim=2, r=0.005, domain=(1.0, 0.6, 0.1), block=(0.2, 0.1, 0.0)))
+    eng = L.Engine(1, 2, low.n + mid.n + top.n, sum(s.geo.grid_num_total for s in (low, mid, top)), 3)
+    slots = []
+    for sc in (low, mid, top):
+        slots.append(eng.add_scene(sc.desc()))
+        L.upload_scene(eng, slots[-1], sc)
+    eng.step(3)
+    eng.remove_scene(slots[1])
+    if between:
+        eng.step(1)
+    eng.sync()
+    keep = [slots[0], slots[2]]
+    before = [eng.neighbor_stats(s) for s in keep]
+    starts = [eng.download(s, "cell_start") for s in keep]
+    slot = eng.add_scene(new.desc())
+    L.upload_scene(eng, slot, new)
+    assert not eng.download(slot, "cell_start").any()
+    assert not eng.neighbor_stats(slot)[0].any()
+    for s, b, c in zip(keep, before, starts):
+        np.testing.assert_array_equal(eng.download(s, "cell_start"), c)
+        for x, y in zip(eng.neighbor_stats(s), b):
+            np.testing.assert_array_equal(x, y)
+    eng.step(2)
+    eng.sync()
+    got = {f: eng.download(slot, f) for f in STATE}
+    eng.close()
+    alone = run([new], 2)
+    for f in STATE:
+        np.testing.assert_array_equal(got[f], alone[f], err_msg=f)

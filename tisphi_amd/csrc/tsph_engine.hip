@@ -1259,6 +1259,16 @@ int tsph_add_scene(void* engine, const tsph_scene_desc* desc, int* out_slot) {
       if (P.flag) HIP_TRY(hipMemsetAsync(P.flag + pb, 0, n * 4, E->stream));
     }
     HIP_TRY(hipMemsetAsync(E->w.status + 2 * slot, 0, 16, E->stream));
+    std::vector<int32_t> first, end;
+    if ((rr = d2h(E, (const int32_t*)E->w.start, cb, 1, first)) ||
+        (rr = d2h(E, (const int32_t*)E->w.start, cb + ncell, 1, end)))
+      return rr;
+    const int32_t delta = end[0] - first[0];
+    const int64_t last = delta ? (int64_t)E->ccap + 1 : cb + ncell;
+    const OnDevice on(E->device);
+    hipLaunchKernelGGL(k_empty_cells, dim3((unsigned)((last - cb + 255) / 256)), dim3(256), 0, E->stream, E->w.start,
+                       (int)cb, (int)(cb + ncell), (int)last, first[0], delta);
+    HIP_TRY(hipGetLastError());
     return TSPH_OK;
   }();
   if (r) {

@@ -368,6 +368,20 @@ __global__ __launch_bounds__(kSmallBlock) void k_sort_small(KArgs a) {
     if (cell[k] >= 0) a.w.tmp[cnt[cell[k]] + slot[k]] = S.pbase + k * kSmallBlock + tid;
 }
 
+// The cells [cb, ce) of a scene just added, which no sort has filled yet,
+// hold nothing: its first entry stays (the end of the scene below, if one
+// ends there), the others become v, its value, and all above move down by
+// delta = (entry ce) - v, which leaves the other scenes' ranges as they are,
+// for only differences of entries are used.  A sort of small scenes writes
+// their own entries only, so a range that a removed scene held keeps that
+// scene's counts, and a pass run before the next sort would walk them.
+__global__ __launch_bounds__(256) void k_empty_cells(int32_t* __restrict__ start, int cb, int ce, int n, int32_t v,
+                                                     int32_t delta) {
+  const int i = cb + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < ce) start[i] = v;
+  else if (i < n) start[i] -= delta;
+}
+
 __global__ __launch_bounds__(256) void k_scatter(KArgs a) {
   int s, p;
   if (!tile_thread(a, s, p)) return;
