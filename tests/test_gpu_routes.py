@@ -58,6 +58,33 @@ def test_sort_route_of_small_scenes(dim, block):
         np.testing.assert_array_equal(alone[f], beside[f], err_msg=f)
 
 
+def sorts(sc):
+    """(launches of the one-workgroup sort, of the general one) in a step."""
+    eng = L.Engine(sc.method, sc.geo.dim, sc.n, sc.geo.grid_num_total, 1)
+    L.upload_scene(eng, eng.add_scene(sc.desc()), sc)
+    eng.timing(True)
+    eng.step(1)
+    eng.sync()
+    out = eng.kernel_time("sort_small")[1], eng.kernel_time("scatter")[1]
+    eng.close()
+    return out
+
+
+# cells: more than half of what the one-workgroup sort holds (64 KiB less 16
+# words), all of it, and the next larger grid
+@pytest.mark.parametrize("domain,cells", [((2.8, 2.7), 8832), ((3.9, 3.66), 16368), ((3.81, 3.75), 16383)])
+def test_sort_route_of_many_cells(domain, cells):
+    sc = build_scene(tiny_cfg(r=0.005, domain=domain + (0.2,), block=(1.0, 0.9, 0.0)))
+    flow = sc.mat_type == 1
+    sc.vel[flow, :2] = np.random.default_rng(0).uniform(-2.0, 2.0, (int(flow.sum()), 2))
+    assert sc.geo.grid_num_total == cells and sc.n <= 16384
+    assert sorts(sc) == ((1, 0) if cells <= 16368 else (0, 1))
+    wide = build_scene(tiny_cfg(r=0.005, domain=(6.0, 3.0, 0.2), block=(0.2, 0.2, 0.0)))
+    alone, beside = run([sc], 5), run([sc, wide], 5)
+    for f in STATE:
+        np.testing.assert_array_equal(alone[f], beside[f], err_msg=f)
+
+
 def uneven(method, dim, nan, seed=3):
     """A scene whose flow particles lie from far apart to 80 per cell (lists
     longer than the engine keeps, cells of more than 32 particles, windows

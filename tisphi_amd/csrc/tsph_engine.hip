@@ -133,12 +133,10 @@ struct Timing {
 struct StepFlags {
   int ti = 2;
   bool xsph = false, collide = false, kcorr = false, rigid = false, rep = false;
-  // cells of the largest resident scene, rounded up to a power of two, if
-  // every one is small enough for k_sort_small; 0 otherwise
-  int small_cells = 0;
+  bool small = false;  // every resident scene is small enough for k_sort_small
   bool operator==(const StepFlags& o) const {
     return ti == o.ti && xsph == o.xsph && collide == o.collide && kcorr == o.kcorr &&
-           rigid == o.rigid && rep == o.rep && small_cells == o.small_cells;
+           rigid == o.rigid && rep == o.rep && small == o.small;
   }
 };
 
@@ -317,7 +315,6 @@ int ensure_rigid(tsph_engine* E) {
 struct Launcher {
   tsph_engine* E;
   int status = TSPH_OK;
-  int lds = 0;  // dynamic LDS of the next launches, bytes
   template <class K, class... Args>
   void go(const char* name, K kernel, int grid, int block, Args... args) {
     if (status != TSPH_OK || grid <= 0) return;
@@ -337,7 +334,7 @@ struct Launcher {
       T.pool.pop_back();
       hipEventRecord(rec.a, E->stream);
     }
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, E->stream, args...);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, E->stream, args...);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) status = fail(TSPH_ERR_HIP, std::string(name) + ": " + hipGetErrorString(e));
     if (timed) {
@@ -376,10 +373,8 @@ struct Seq {
   void sort(bool fuse_init = false) {
     KArgs a = E->args();
     const int eb = E->elem_block;
-    if (const int cells = step_flags(E).small_cells) {
-      L.lds = cells * (int)sizeof(int32_t);
+    if (step_flags(E).small) {
       L.go("sort_small", k_sort_small<DIM>, E->max_scenes, kSmallBlock, a);
-      L.lds = 0;
     } else {
       L.go("hash", k_hash<DIM>, tb(), eb, a);
       const int n = E->ccap;
@@ -586,11 +581,9 @@ struct Seq {
 StepFlags step_flags(tsph_engine* E) {
   StepFlags f;
   bool first = true, small = true;
-  int cells = 0;
   for (size_t s = 0; s < E->scenes.size(); ++s) {
     if (!E->scenes[s].active) continue;
     small = small && E->scenes[s].n <= kSmallParticles && E->scenes[s].ncell <= kSmallCells;
-    cells = std::max(cells, E->scenes[s].ncell);
     if (first) f.ti = E->scenes[s].ti;
     first = false;
     f.xsph = f.xsph || E->scenes[s].xsph;
@@ -599,10 +592,7 @@ StepFlags step_flags(tsph_engine* E) {
     f.rigid = f.rigid || E->scenes[s].nrig > 0;
     f.rep = f.rep || E->scenes[s].rep != 0;
   }
-  if (small && !first) {
-    f.small_cells = 64;
-    while (f.small_cells < cells) f.small_cells *= 2;
-  }
+  f.small = small && !first;
   return f;
 }
 
