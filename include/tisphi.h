@@ -289,7 +289,8 @@ int tsph_set_color(void* engine, int slot, int color_group, int show_bdy);
 int tsph_status(void* engine, int slot, int64_t out[2]);
 /* Average device time (ms) of the named kernel class over the launches
  * since the last reset, measured with HIP events on the engine stream.
- * name: "pair_fluid" etc.; returns count in *out_launches. */
+ * name: "wc_fluid" etc.; returns count in *out_launches.  "capture": the
+ * captures of the step's graphs (both parities) and their host time. */
 int tsph_kernel_time(void* engine, const char* name, double* out_ms,
                      int64_t* out_launches);
 int tsph_timing(void* engine, int enable);

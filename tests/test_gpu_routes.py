@@ -340,3 +340,37 @@ def test_scene_in_a_freed_range_is_empty_until_sorted(between):
     alone = run([new], 2)
     for f in STATE:
         np.testing.assert_array_equal(got[f], alone[f], err_msg=f)
+
+
+def test_residents_that_come_and_go_capture_once_per_route():
+    """Scenes of any size admitted and retired: the step's graphs are captured
+    once for each route of the sort."""
+    small = [shaken(2, b, s) for s, b in enumerate([(0.1, 0.1, 0.0), (0.6, 0.5, 0.0)])]
+    few = build_scene(tiny_cfg(r=0.005, domain=(0.3, 0.3, 0.2), block=(0.1, 0.1, 0.0)))
+    large = build_scene(tiny_cfg(r=0.005, domain=(6.0, 3.0, 0.2), block=(0.2, 0.2, 0.0)))
+    scenes = [few, small[0], small[1], large]
+    eng = L.Engine(1, 2, sum(s.n for s in scenes), sum(s.geo.grid_num_total for s in scenes), 4)
+
+    def add(sc):
+        slot = eng.add_scene(sc.desc())
+        L.upload_scene(eng, slot, sc)
+        eng.step(2)
+        return slot
+
+    assert eng.kernel_time("capture")[1] == 0
+    add(few)
+    a, b = add(small[0]), add(small[1])
+    eng.remove_scene(b)
+    eng.step(1)
+    assert eng.kernel_time("capture")[1] == 1
+    for _ in range(3):
+        c = add(large)
+        eng.remove_scene(c)
+        eng.step(1)
+    assert eng.kernel_time("capture")[1] == 2
+    got = {f: eng.download(a, f) for f in STATE}
+    steps = eng.steps(a)
+    eng.close()
+    alone = run([small[0]], steps)
+    for f in STATE:
+        np.testing.assert_array_equal(got[f], alone[f], err_msg=f)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -139,6 +140,12 @@ struct StepFlags {
            rigid == o.rigid && rep == o.rep && small == o.small;
   }
 };
+// A step captured for either parity of the state buffers.
+struct StepGraphs {
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  bool valid = false;
+  StepFlags flags;  // options they were captured with
+};
 
 struct tsph_engine {
   int method = 1, dim = 2, max_scenes = 1, device = 0;
@@ -154,9 +161,9 @@ struct tsph_engine {
   bool cflow_valid = false;  // per-cell flow flags match the current order
   bool fresh_sort = false;   // offsets renormalised, no motion since the sort
   int32_t nl_cap = 0;
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
-  bool graph_valid = false;
-  StepFlags graph_flags;  // options the graphs were captured with
+  // by the sort's route (StepFlags::small): residents that come and go on
+  // either side of its limits replay what was captured for it before
+  StepGraphs graphs[2];
   int parity = 0;  // which state buffer is current
   PState buf[2];
   PWork w;
@@ -274,13 +281,16 @@ void free_work(PWork& w) {
   w = PWork{};
 }
 
-void invalidate_graph(tsph_engine* E) {
-  for (auto& g : E->graph)
+void drop_graphs(StepGraphs& G) {
+  for (auto& g : G.exec)
     if (g) {
       hipGraphExecDestroy(g);
       g = nullptr;
     }
-  E->graph_valid = false;
+  G.valid = false;
+}
+void invalidate_graph(tsph_engine* E) {
+  for (StepGraphs& G : E->graphs) drop_graphs(G);
 }
 
 // The colour feed's arrays, on first use (an engine that never colours
@@ -604,8 +614,9 @@ int run_step_eager(tsph_engine* E) {
   return L.status;
 }
 
-int build_graphs(tsph_engine* E) {
-  invalidate_graph(E);
+int build_graphs(tsph_engine* E, StepGraphs& G, const StepFlags& flags) {
+  const auto t0 = std::chrono::steady_clock::now();
+  drop_graphs(G);
   const int p0 = E->parity;
   for (int k = 0; k < 2; ++k) {
     const int par = (p0 + k) & 1;
@@ -630,11 +641,14 @@ int build_graphs(tsph_engine* E) {
       E->parity = p0;
       return fail(TSPH_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     }
-    E->graph[par] = ex;
+    G.exec[par] = ex;
   }
   E->parity = p0;
-  E->graph_valid = true;
-  E->graph_flags = step_flags(E);
+  G.valid = true;
+  G.flags = flags;
+  auto& acc = E->timing.acc["capture"];
+  acc.first += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+  acc.second += 1;
   return TSPH_OK;
 }
 
@@ -1311,12 +1325,14 @@ int tsph_step(void* engine, int nsteps) {
   if (E->use_graph && !E->timing.on) {
     // recapture when the residents ask for other step options than the
     // graphs hold (a scene with XSPH, collisions or kernel correction added)
-    if (!E->graph_valid || !(E->graph_flags == step_flags(E))) {
-      int r = build_graphs(E);
+    const StepFlags flags = step_flags(E);
+    StepGraphs& G = E->graphs[flags.small];
+    if (!G.valid || !(G.flags == flags)) {
+      int r = build_graphs(E, G, flags);
       if (r) return r;
     }
     for (int k = 0; k < nsteps; ++k) {
-      HIP_TRY(hipGraphLaunch(E->graph[E->parity], E->stream));
+      HIP_TRY(hipGraphLaunch(G.exec[E->parity], E->stream));
       E->parity ^= 1;
     }
   } else {
