@@ -374,3 +374,28 @@ def test_residents_that_come_and_go_capture_once_per_route():
     alone = run([small[0]], steps)
     for f in STATE:
         np.testing.assert_array_equal(got[f], alone[f], err_msg=f)
+
+
+def test_sort_of_more_slots_than_workgroups():
+    """An engine of more scene slots than the one-workgroup sort launches
+    workgroups: the scenes left in the first and in later turns of one
+    workgroup, and in others, get the bits they have alone."""
+    empty = build_scene(tiny_cfg(r=0.02, domain=(0.1, 0.1, 0.1), block=(0.04, 0.04, 0.0)))
+    keep = {0: shaken(2, (0.5, 0.4, 0.0), 1), 2048: shaken(2, (0.3, 0.8, 0.0), 2), 4096: shaken(2, (0.2, 0.2, 0.0), 3),
+            2047: shaken(2, (0.4, 0.1, 0.0), 4), 4199: shaken(2, (0.1, 0.6, 0.0), 5)}
+    scenes = [keep.get(s, empty) for s in range(4200)]
+    eng = L.Engine(1, 2, sum((s.n + 63) // 64 * 64 for s in scenes), sum(s.geo.grid_num_total for s in scenes), 4200)
+    for sc in scenes:
+        eng.add_scene(sc.desc())
+    for s in range(4200):
+        if s not in keep:
+            eng.remove_scene(s)
+    for s, sc in keep.items():
+        L.upload_scene(eng, s, sc)
+    eng.step(4)
+    eng.sync()
+    for s, sc in keep.items():
+        alone = run([sc], 4)
+        for f in STATE:
+            np.testing.assert_array_equal(eng.download(s, f), alone[f], err_msg=f"slot {s}: {f}")
+    eng.close()

@@ -35,6 +35,7 @@ int fail(int code, const std::string& msg) {
   } while (0)
 
 constexpr int kTileAlign = 64;
+constexpr int kMaxSlots = 65536;
 
 template <class T>
 int dalloc(T** p, size_t count, size_t& bytes) {
@@ -384,7 +385,7 @@ struct Seq {
     KArgs a = E->args();
     const int eb = E->elem_block;
     if (step_flags(E).small) {
-      L.go("sort_small", k_sort_small<DIM>, E->max_scenes, kSmallBlock, a);
+      L.go("sort_small", k_sort_small<DIM>, std::min(E->max_scenes, kSmallGrid), kSmallBlock, a, E->max_scenes);
     } else {
       L.go("hash", k_hash<DIM>, tb(), eb, a);
       const int n = E->ccap;
@@ -1132,7 +1133,8 @@ int tsph_engine_create(int method, int dim, int64_t particle_capacity, int64_t c
     return fail(TSPH_ERR_INVALID_ARG, "particle capacity out of range");
   if (cell_capacity < 1 || cell_capacity > (int64_t)kScanTile * kScanTile)
     return fail(TSPH_ERR_INVALID_ARG, "cell capacity out of range");
-  if (max_scenes < 1 || max_scenes > 65536) return fail(TSPH_ERR_INVALID_ARG, "max_scenes out of range");
+  static_assert(kMaxSlots <= 64 * kSmallGrid, "k_sort_small takes at most 64 slots per workgroup");
+  if (max_scenes < 1 || max_scenes > kMaxSlots) return fail(TSPH_ERR_INVALID_ARG, "max_scenes out of range");
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
     return fail(TSPH_ERR_HIP, "no HIP device available");
