@@ -399,3 +399,28 @@ def test_sort_of_more_slots_than_workgroups():
         for f in STATE:
             np.testing.assert_array_equal(eng.download(s, f), alone[f], err_msg=f"slot {s}: {f}")
     eng.close()
+
+
+def test_read_outs_from_a_thread_on_another_device():
+    """Fields, globals and the colour range are read on the engine's device,
+    whatever device the calling thread has chosen, which it keeps."""
+    if L.device_count() < 2:
+        pytest.skip("needs two devices")
+    import torch
+    sc = shaken(2, (0.3, 0.3, 0.0))
+    eng = L.Engine(1, 2, sc.n, sc.geo.grid_num_total, 1)
+    slot = eng.add_scene(sc.desc())
+    L.upload_scene(eng, slot, sc)
+    eng.step(2)
+    eng.assign_value_color(slot, 3)
+
+    def read():
+        return [eng.download(slot, "vel"), eng.globals(slot), np.array(eng.v_maxmin(slot))]
+
+    here = read()
+    with torch.cuda.device(1):
+        there = read()
+        assert torch.cuda.current_device() == 1
+    eng.close()
+    for a, b in zip(there, here):
+        np.testing.assert_array_equal(a, b)

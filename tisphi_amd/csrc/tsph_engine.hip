@@ -855,7 +855,6 @@ int read_out(tsph_engine* E, const Pack& k, int64_t n, void* host) {
   if (n == 0) return TSPH_OK;
   if (!k.src) return fail(TSPH_ERR_INVALID_ARG, "field not held by this engine's method");
   std::lock_guard<std::mutex> lock(E->reading);
-  const OnDevice on(E->device);
   const size_t row = (size_t)k.comps * (k.kind == kPackI || k.kind == kPackB || k.kind == kPackStart ? 4 : 8);
   const int64_t per = (int64_t)(kReadHalf / row), turns = (n + per - 1) / per;
   auto rows = [&](int64_t t) { return std::min(per, n - t * per); };
@@ -1317,6 +1316,7 @@ int tsph_upload(void* engine, int slot, int field, const void* host, size_t byte
 int tsph_download(void* engine, int slot, int field, void* host, size_t bytes) {
   tsph_engine* E = (tsph_engine*)engine;
   if (!E || !host) return fail(TSPH_ERR_INVALID_ARG, "null argument");
+  const OnDevice on(E->device);
   return transfer(E, slot, field, host, bytes, false);
 }
 
@@ -1448,6 +1448,7 @@ int tsph_globals(void* engine, int slot, double out[4]) {
   tsph_engine* E = (tsph_engine*)engine;
   if (!slot_ok(E, slot) || !out) return fail(TSPH_ERR_INVALID_ARG, "bad argument");
   std::lock_guard<std::mutex> lock(E->reading);
+  const OnDevice on(E->device);
   Launcher L{E};
   if (E->dim == 2) Seq<2>{E, L}.globals(slot, (double*)E->stage);
   else Seq<3>{E, L}.globals(slot, (double*)E->stage);
@@ -1492,6 +1493,7 @@ int tsph_v_maxmin(void* engine, int slot, double given_max, double given_min, in
                   int fix_min, double* out_vmax, double* out_vmin) {
   tsph_engine* E = (tsph_engine*)engine;
   if (!slot_ok(E, slot) || !out_vmax || !out_vmin) return fail(TSPH_ERR_INVALID_ARG, "bad argument");
+  const OnDevice on(E->device);
   int r = ensure_colour(E);
   if (r) return r;
   std::lock_guard<std::mutex> lock(E->reading);
