@@ -83,3 +83,22 @@ def test_unwritable_cache_is_not_fatal(tmp_path, monkeypatch):
     e = FakeEngine()
     r = autotune.tune(e, steps=1, quick=False)
     assert r["shape"] == (64, 256, 2, 512)
+
+
+def test_shape_measured_with_other_kernels_is_retuned(tmp_path, monkeypatch):
+    """A choice cached by another build of the engine library, or by one that
+    did not name itself, is measured anew and replaced."""
+    path = tmp_path / "c.json"
+    lib = tmp_path / "lib.so"
+    monkeypatch.setenv("TSPH_TUNE_CACHE", str(path))
+    monkeypatch.setattr(autotune._lib, "LIB_PATH", str(lib))
+    e = FakeEngine()
+    path.write_text(json.dumps({autotune.tune_key(e): {"shape": [256, 256, 1, 256], "ms_per_step": 1.0}}))
+    lib.write_bytes(b"one")
+    r = autotune.tune(e, steps=1, quick=False)
+    assert not r["cached"] and e.nl == 2
+    assert autotune.tune(FakeEngine())["cached"]
+    lib.write_bytes(b"two")
+    r = autotune.tune(FakeEngine(), steps=1, quick=False)
+    assert not r["cached"] and r["steps_taken"] == 36 * 2
+    assert autotune.tune(FakeEngine())["cached"]

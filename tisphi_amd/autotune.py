@@ -4,8 +4,8 @@ Picks the launch shape of an engine's resident scenes by timing real
 steps: the threads per block of the pair kernels and of the per-particle
 kernels, how the per-step neighbour lists are built (stencil walk over
 global memory, or over cell windows staged in LDS), and the cell tile of
-the LDS build (how many candidate particles a wave stages per row offset:
-128, 256 or 512).  Every shape computes the same per-particle arithmetic in
+the LDS build (how many candidate particles a wave stages at a time: 128,
+256 or 512).  Every shape computes the same per-particle arithmetic in
 the same order (a wave always owns one 64-particle tile; the shape only
 changes how waves are grouped into workgroups and where candidates are
 read from), so the results are bitwise identical whatever shape is chosen:
@@ -15,12 +15,16 @@ as such.
 Choices are cached per (device, method, dimension, particle-count bucket,
 scene-count bucket) in a JSON file (``$TSPH_TUNE_CACHE`` or
 ``~/.cache/tisphi_amd/launch_shapes.json``); a cached choice is applied
-without stepping.
+without stepping, if it was measured with the library that is loaded now (a
+shape that was fast with other kernels may be slow with these).
 """
+import hashlib
 import json
 import math
 import os
 import time
+
+from . import _lib
 
 BLOCKS = (64, 128, 256)
 CELL_TILES = (128, 256, 512)
@@ -59,6 +63,16 @@ def tune_key(eng):
     n = max(1, sum(eng.n.values()))
     s = max(1, len(eng.n))
     return f"m{eng.method}/d{eng.dim}/p{int(math.log2(n))}/s{int(math.log2(s))}"
+
+
+def kernels_id():
+    """Digest of the engine library, by which a cached choice names the
+    kernels it was measured with."""
+    try:
+        with open(_lib.LIB_PATH, "rb") as f:
+            return hashlib.sha256(f.read()).hexdigest()[:16]
+    except OSError:
+        return ""
 
 
 NL_MODES = (1, 2)  # lists built from global memory / from LDS windows
@@ -100,7 +114,8 @@ def tune(eng, steps=2, quick=True, use_cache=True, log=None):
     path = _cache_path()
     key = tune_key(eng)
     cache = _load_cache(path) if use_cache else {}
-    if key in cache and len(cache[key].get("shape", ())) == 4:
+    kernels = kernels_id() if use_cache else ""
+    if key in cache and cache[key].get("kernels") == kernels and len(cache[key].get("shape", ())) == 4:
         shape = tuple(int(v) for v in cache[key]["shape"])
         apply(eng, shape)
         say(f"autotune {key}: cached shape {shape}")
@@ -120,7 +135,7 @@ def tune(eng, steps=2, quick=True, use_cache=True, log=None):
     apply(eng, best)
     if use_cache:
         cache = _load_cache(path)
-        cache[key] = {"shape": list(best), "ms_per_step": trials[best]}
+        cache[key] = {"shape": list(best), "ms_per_step": trials[best], "kernels": kernels}
         _store_cache(path, cache)
     return dict(shape=best, ms_per_step=trials[best], steps_taken=taken, cached=False,
                 trials={f"{p}x{e}/nl{m}/tile{c}": v for (p, e, m, c), v in trials.items()})
