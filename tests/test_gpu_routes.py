@@ -8,6 +8,7 @@ import pytest
 
 from oracle.sph_numpy import NumpySPH
 from tests.common import tiny_cfg
+from tests.test_cell_rule import renorm
 from tisphi_amd import _lib as L
 from tisphi_amd.scene import build_scene
 
@@ -424,3 +425,87 @@ def test_read_outs_from_a_thread_on_another_device():
     eng.close()
     for a, b in zip(there, here):
         np.testing.assert_array_equal(a, b)
+
+
+def test_sort_of_scenes_that_come_and_go():
+    """Small scenes whose slot order is not their cell order, with a gap in
+    the cells, against the same scenes beside one that forces the general
+    sort: state and cell ranges of every scene."""
+    a, b, c = (shaken(2, blk, s) for s, blk in enumerate([(0.4, 0.3, 0.0), (0.3, 0.5, 0.0), (0.5, 0.2, 0.0)]))
+    d = build_scene(tiny_cfg(dim=2, r=0.005, domain=(1.0, 0.6, 0.1), block=(0.3, 0.2, 0.0)))
+    late = build_scene(tiny_cfg(dim=2, r=0.005, domain=(2.4, 1.4, 0.1), block=(0.2, 0.3, 0.0)))
+    wide = build_scene(tiny_cfg(dim=2, r=0.005, domain=(6.0, 3.0, 0.2), block=(0.2, 0.2, 0.0)))
+    assert d.geo.grid_num_total < b.geo.grid_num_total and a.geo.grid_num_total < late.geo.grid_num_total
+    out = []
+    for general in (False, True):
+        eng = L.Engine(1, 2, sum(s.n for s in (a, b, c, d, late, wide)),
+                       sum(s.geo.grid_num_total for s in (a, b, c, d, late, wide)), 5)
+
+        def add(sc):
+            slot = eng.add_scene(sc.desc())
+            L.upload_scene(eng, slot, sc)
+            return slot
+
+        slots = {"a": add(a), "b": add(b), "c": add(c)}
+        if general:
+            add(wide)
+        eng.step(2)
+        # the first goes; a larger one takes its slot but cells past the others'
+        eng.remove_scene(slots.pop("a"))
+        slots["late"] = add(late)
+        eng.step(2)
+        # the middle one goes; a smaller one leaves a gap in its cells
+        eng.remove_scene(slots.pop("b"))
+        slots["d"] = add(d)
+        eng.step(2)
+        eng.sync()
+        out.append({(k, f): eng.download(s, f) for k, s in slots.items() for f in STATE})
+        eng.close()
+    assert out[0].keys() == out[1].keys()
+    for k in out[0]:
+        np.testing.assert_array_equal(out[0][k], out[1][k], err_msg=str(k))
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_cell_update_of_offsets_at_the_edges(dim):
+    """Cell and offset after the sort, bit for bit, of offsets on and beside
+    the edges of a cell: the rule floor(o / grid) in float64, whichever way
+    the kernel takes.  Also -0, and in 2D a z offset that is not zero."""
+    sc = build_scene(tiny_cfg(dim=dim, domain=(0.4, 0.4, 0.4), block=(0.08, 0.08, 0.08)))
+    grid = sc.geo.grid_size
+    top = np.float32(grid)
+    while np.float64(top) >= grid:
+        top = np.nextafter(top, np.float32(0))
+    over = np.nextafter(top, np.float32(1))
+    f = np.float32
+    edges = [f(0), f(-0.0), f(1e-45), f(-1e-45), f(-1e-9), f(0.4 * grid), np.nextafter(top, f(0)), top, over,
+             np.nextafter(over, f(1)), f(1.5 * grid), f(-0.5 * grid), f(-grid), f(2 * grid)]
+    eng = L.Engine(sc.method, dim, sc.n, sc.geo.grid_num_total, 1)
+    slot = eng.add_scene(sc.desc())
+    L.upload_scene(eng, slot, sc)
+    gn = np.asarray(sc.geo.grid_num)
+    flow = np.flatnonzero(sc.mat_type == 1)[: len(edges) * 3]
+    cell0 = np.zeros((sc.n, 3), dtype=np.int64) + np.asarray([3, 3, 3 if dim == 3 else 0])
+    assert (gn[:dim] > 6).all() and flow.size == len(edges) * 3
+    off0 = np.full((sc.n, 3), 0.25 * grid, dtype=np.float32)
+    off0[:, 2] *= dim - 2
+    for k, i in enumerate(flow):
+        off0[i, (k // len(edges)) % 3] = edges[k % len(edges)]
+    eng.upload(slot, "cell", (cell0[:, 0] * gn[1] + cell0[:, 1]) * gn[2] + cell0[:, 2])
+    eng.upload(slot, "offset", off0)
+    eng.upload(slot, "id0", np.arange(sc.n))
+    eng.run("sort")
+    order = np.argsort(eng.download(slot, "id0"))
+    cell, off = eng.download(slot, "cell")[order], eng.download(slot, "offset")[order].astype(np.float32)
+    eng.close()
+    want_c, want_o = cell0.copy(), off0.copy()
+    for i in range(sc.n):
+        for ax in range(3):
+            if dim == 2 and ax == 2:
+                want_o[i, 2] = 0
+                continue
+            k, o = renorm(off0[i, ax], grid)
+            want_c[i, ax] += k
+            want_o[i, ax] = o
+    np.testing.assert_array_equal(cell, (want_c[:, 0] * gn[1] + want_c[:, 1]) * gn[2] + want_c[:, 2])
+    np.testing.assert_array_equal(off.view(np.uint32), want_o.view(np.uint32))
