@@ -509,3 +509,67 @@ def test_cell_update_of_offsets_at_the_edges(dim):
             want_o[i, ax] = o
     np.testing.assert_array_equal(cell, (want_c[:, 0] * gn[1] + want_c[:, 1]) * gn[2] + want_c[:, 2])
     np.testing.assert_array_equal(off.view(np.uint32), want_o.view(np.uint32))
+
+
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("case", ["vx", "vy", "vz", "nan_vz", "wall_vz", "large"])
+def test_two_dimensions_keep_the_third_components_sums(case, kernel):
+    """In 2D the third components' terms are products with 0: +-0, but not a
+    number beside an infinity, which d_vel and d_density then carry (and the
+    step reports).  Against the pairs' forces in numpy: where one is not finite
+    the sum's third component is NaN, and nowhere else."""
+    sc = build_scene(tiny_cfg(dim=2, kernel=kernel, boundary=2, domain=(0.2, 0.2, 0.1)))
+    flow, wall = np.flatnonzero(sc.mat_type == 1), np.flatnonzero(sc.mat_type < 0)
+    hit = int(flow[len(flow) // 2])
+    rng = np.random.default_rng(2)
+    sc.vel[flow, :2] = rng.uniform(-0.1, 0.1, (flow.size, 2))
+    if case == "wall_vz":
+        hit = int(wall[np.argmin(np.abs(sc.pos[wall] - sc.pos[flow[0]]).sum(1))])
+        sc.vel[hit, 2] = np.inf
+    elif case == "large":
+        sc.vel[hit, 0] = 3e38  # its dot product with a distance is finite, the force may not be
+    else:
+        sc.vel[hit, {"vx": 0, "vy": 1}.get(case, 2)] = np.nan if case == "nan_vz" else np.inf
+    got = []
+    for mode in (0, 2):
+        eng = L.Engine(1, 2, sc.n, sc.geo.grid_num_total, 1)
+        eng.set_neighbor_list(mode)
+        slot = eng.add_scene(sc.desc())
+        L.upload_scene(eng, slot, sc)
+        for what in ("sort", "shepard", "init_tmp", "one_step"):
+            eng.run(what)
+        got.append({f: eng.download(slot, f) for f in ("d_vel", "d_density", "type", "v_tmp", "density_tmp", "pressure",
+                                                       "offset", "cell", "m_V")})
+        eng.close()
+    for f in got[0]:
+        np.testing.assert_array_equal(got[0][f], got[1][f], err_msg=f)
+    g = {k: v.astype(np.float32) if v.dtype.kind == "f" else v for k, v in got[0].items()}
+    c = np.stack(np.unravel_index(g["cell"], np.asarray(sc.geo.grid_num)), 1)[:, :2]
+    o = g["offset"][:, :2]
+    desc = sc.desc()
+    c2 = 0.01 * desc["smoothing_len"] ** 2
+    c1, rho0 = 2.0 * 4 * desc["viscosity"], desc["density0"]
+    seen = 0
+    with np.errstate(all="ignore"):
+        for i in np.flatnonzero(g["type"] == 1):
+            # pair vector and reach as the kernels form them: zeros, signs and
+            # the pairs on the edge matter
+            d = (o[i] + (c[i] - c).astype(np.float32) * np.float32(sc.geo.grid_size)) - o
+            r2 = (d[:, 1].astype(np.float64) ** 2 + d[:, 0] * d[:, 0]).astype(np.float32)
+            j = np.flatnonzero((r2 < np.float32(desc["support_radius"]) ** 2) & (np.arange(r2.size) != i))
+            u = g["v_tmp"][i] - g["v_tmp"][j]
+            dot = (u[:, :2] * d[j]).sum(1) + u[:, 2] * np.float32(0)
+            mn = np.where(dot < 0, dot, np.float32(0))
+            rr = np.where(g["type"][j] < 0, rho0 / g["density_tmp"][i], 1.0)
+            vis = (c1 * g["m_V"][j] * rr).astype(np.float32) * mn / (r2[j] + np.float32(c2))
+            q = g["pressure"] / g["density_tmp"] ** 2
+            sc_ = vis - np.float32(rho0) * g["m_V"][j] * (q[i] + q[j])
+            bad_z = not np.isfinite(sc_).all()
+            bad_uz = not np.isfinite(u[:, 2]).all()
+            assert np.isnan(g["d_vel"][i, 2]) == bad_z, (i, sc_, g["d_vel"][i])
+            if bad_uz:
+                assert np.isnan(g["d_density"][i])
+                if not bad_z:
+                    assert np.isfinite(g["d_vel"][i]).all()
+            seen += bad_z or bad_uz
+    assert seen > 0

@@ -1210,17 +1210,22 @@ __global__ __launch_bounds__(256) void k_wc_bdy(KArgs a, int again) {
 // written by the EOS or the boundary pass, sign bit set for a wall) says
 // which it is, so the pass reads position + m_V and q per neighbour and
 // nothing else.
-template <int DIM, bool NL, bool SHEP, int KT, bool KC, int L>
-__device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+//
+// In 2D z = g_z = 0, so the third components' terms are +-0, and the list
+// replay, whose additions are most of its work, leaves them out (Z false).
+// But 0 times an infinity, or a NaN, is not a number, which d_vel and
+// d_density then carry.  So `odd` gathers the bits of the neighbours' v_z (an
+// "or" of two of them with what is there is one instruction), a force that is
+// not finite shows in d_vel, and wc_fluid_one() then forms the sums with all
+// terms.  Batch of 256 in 2D, 1.31 M particles: passes of 92.2 and 81.1 us,
+// without the check 93.7 and 78.7.
+template <int DIM, bool Z, bool NL, bool SHEP, int KT, bool KC, int L, int NT>
+__device__ __forceinline__ void wc_fluid_sums(const KArgs& a, const SceneDev& S, int p, const Own& o, const float4& vi,
+                                              float pri, const float (&M)[9], float (&acc)[NT], uint32_t& odd) {
+  static_assert(NT == (Z ? 4 : 3) + (SHEP ? 1 : 0), "d_density, d_vel, Shepard");
   const float4* __restrict__ vp = a.w.vp;
-  const float4 vi = a.cur.vtmp[p];
-  const float pri = vp[p].w;
   const float c1 = S.visc_c1, c2 = S.visc_c2, rho0 = S.rho0;
   const float rr = rho0 / vi.w;  // rho0 / rho_i of the boundary viscosity
-  float M[9];
-  if (KC) corr_load(a.w.Lc, a.stride, p, M);
-  constexpr int NT = DIM + 1 + (SHEP ? 1 : 0);
-  float acc[NT] = {};  // d_density, d_vel, Shepard
   sum_pairs<DIM, NL, L>(S, a, p, o, acc, [&](int j, float x, float y, float z, float r2, float mVj,
                                              float (&t)[NT]) {
     const float rn = pair_dist(r2);
@@ -1232,12 +1237,11 @@ __device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, 
     const float ux = vi.x - q.x, uy = vi.y - q.y, uz = vi.z - q.z;
     float cg[3] = {gx, gy, gz};
     if (KC) corr_apply(M, cg);
-    // in 2D z = g_z = 0: their products are +-0 and leave the sums' bits
     t[0] = (mVj * ux) * cg[0] + (mVj * uy) * cg[1];
-    if (DIM == 3 || KC) t[0] += (mVj * uz) * cg[2];
+    if (Z || KC) t[0] += (mVj * uz) * cg[2];
     if (SHEP) t[NT - 1] = term_if(!bj, mVj * kernel_W_t<KT>(S, rn));
     // viscosity_force: fluid and boundary neighbours (solver_sph_wc.py:33-45)
-    const float vx_ = DIM == 3 ? ux * x + uy * y + uz * z : ux * x + uy * y;
+    const float vx_ = Z ? ux * x + uy * y + uz * z : ux * x + uy * y;
     const float mn = vx_ < 0.0f ? vx_ : 0.0f;
     const float a0 = c1 * mVj;
     const float aa = bj ? a0 * rr : a0;
@@ -1246,31 +1250,60 @@ __device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, 
     const float sc = vis + pc;
     t[1] = sc * gx;
     t[2] = sc * gy;
-    if (DIM == 3) t[3] = sc * gz;
+    if (Z) t[3] = sc * gz;
+    else odd |= __float_as_uint(q.z);
   });
   if (S.rep) {
     // calc_rep_force_task (solver_sph_wc.py:74-76, 118-121): a second sweep
     // adding the repulsive particles' force after the pair forces
     const int8_t* __restrict__ type = a.cur.type;
-    float dv[DIM];
+    constexpr int NV = Z ? 3 : 2;
+    float dv[NV];
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) dv[c] = acc[1 + c];
+    for (int c = 0; c < NV; ++c) dv[c] = acc[1 + c];
     sum_pairs<DIM, NL, L>(S, a, p, o, dv, [&](int j, float x, float y, float z, float r2, float,
-                                              float (&t)[DIM]) {
+                                              float (&t)[NV]) {
       if (type[j] != kRep) return no_terms(t);
       const float f = rep_fac(S, sqrtf(r2));
       t[0] = f * x;
       t[1] = f * y;
-      if (DIM == 3) t[DIM - 1] = f * z;
+      if (Z) t[NV - 1] = f * z;
     });
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) acc[1 + c] = dv[c];
+    for (int c = 0; c < NV; ++c) acc[1 + c] = dv[c];
+  }
+}
+template <int DIM, bool NL, bool SHEP, int KT, bool KC, int L>
+__device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, int p, const Own& o) {
+  const float4 vi = a.cur.vtmp[p];
+  const float pri = a.w.vp[p].w;
+  float M[9];
+  if (KC) corr_load(a.w.Lc, a.stride, p, M);
+  constexpr int SH = SHEP ? 1 : 0;
+  float sum[4 + SH] = {};  // d_density, d_vel, Shepard
+  constexpr bool kFlat = DIM == 2 && NL;
+  uint32_t odd = 0;
+  if (kFlat) {
+    float acc[3 + SH] = {};
+    wc_fluid_sums<DIM, false, NL, SHEP, KT, KC, L>(a, S, p, o, vi, pri, M, acc, odd);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sum[c] = acc[c];
+    if (SHEP) sum[3 + SH] = acc[2 + SH];
+    odd = (odd | __float_as_uint(vi.z)) << 1;  // any v_z but +-0
+  }
+  // a lane has seen its own neighbours only: the quad's lanes go together
+  if (!kFlat || __any(odd != 0 || !(fabsf(sum[1] + sum[2]) < INFINITY))) {
+    float acc[4 + SH] = {};
+    float4 v = vi;
+    // read again: kept through the loop above, v_z would cost a wave per SIMD
+    wc_fluid_sums<DIM, true, NL, SHEP, KT, KC, L>(a, S, p, o, v, pri, M, acc, odd);
+#pragma unroll
+    for (int c = 0; c < 4 + SH; ++c) sum[c] = acc[c];
   }
   if (!group_head<L>()) return;
-  a.w.drho[p] = acc[0] * vi.w;
-  a.w.dv[p] = make_float4(acc[1] + S.grav[0], acc[2] + S.grav[1],
-                          (DIM == 3 ? acc[3] : 0.0f) + S.grav[2], 0.0f);
-  if (SHEP) a.w.cspm[p] = acc[NT - 1] != 0.0f ? 1.0f / acc[NT - 1] : 1.0f;
+  a.w.drho[p] = sum[0] * vi.w;
+  a.w.dv[p] = make_float4(sum[1] + S.grav[0], sum[2] + S.grav[1], sum[3] + S.grav[2], 0.0f);
+  if (SHEP) a.w.cspm[p] = sum[3 + SH] != 0.0f ? 1.0f / sum[3 + SH] : 1.0f;
 }
 
 // d_vel of a dynamic rigid particle j: g (loop A, solver_sph_wc.py:105-106)
@@ -1314,8 +1347,14 @@ __device__ __forceinline__ float4 wc_rigid_force(const KArgs& a, const SceneDev&
 // Rates of other particles are never written by the reference: zero (by the
 // step's first pass; again: a later one); a static rigid particle's d_vel is
 // zero too (solver_sph_wc.py:125-126).
+//
+// The second sums of the 2D replay hardly ever run and may not cost the first
+// their waves per SIMD (72 registers for seven, 96 for five).
+constexpr int fluid_waves(int dim, bool nl, bool kc) {
+  return dim == 3 || !nl ? 1 : (kc ? 5 : 7);
+}
 template <int DIM, bool NL, bool SHEP, bool KC>
-__global__ __launch_bounds__(256) void k_wc_fluid(KArgs a, int again) {
+__global__ __launch_bounds__(256, fluid_waves(DIM, NL, KC)) void k_wc_fluid(KArgs a, int again) {
   constexpr int L = NL ? kLanes : 1;
   for_work<NL, false>(
       a, again ? kTileFlow : ~0,
