@@ -308,11 +308,13 @@ def test_lists_of_particles_out_of_cell_order(dim, tile):
 
 
 @pytest.mark.parametrize("between", [False, True])  # a step between removal and addition
-def test_scene_in_a_freed_range_is_empty_until_sorted(between):
+@pytest.mark.parametrize("fills", [False, True])    # the new scene's cells end where the next scene's begin
+def test_scene_in_a_freed_range_is_empty_until_sorted(between, fills):
     """A scene that takes the cells of a removed one has no neighbours before
     its first sort, as in a new engine, and the other scenes keep theirs."""
     low, mid, top = (shaken(2, b, s) for s, b in enumerate([(0.3, 0.2, 0.0), (0.4, 0.3, 0.0), (0.2, 0.4, 0.0)]))
-    new = build_scene(tiny_cfg(dim=2, r=0.005, domain=(1.0, 0.6, 0.1), block=(0.2, 0.1, 0.0)))
+    new = build_scene(tiny_cfg(dim=2, r=0.005, domain=(2.0, 1.2, 0.1) if fills else (1.0, 0.6, 0.1), block=(0.2, 0.1, 0.0)))
+    assert (new.geo.grid_num_total == mid.geo.grid_num_total) == fills and new.n <= mid.n
     eng = L.Engine(1, 2, low.n + mid.n + top.n, sum(s.geo.grid_num_total for s in (low, mid, top)), 3)
     slots = []
     for sc in (low, mid, top):

@@ -159,6 +159,7 @@ struct tsph_engine {
   bool nl_lds = true;    // build them from LDS-staged cell windows
   int nl_stage = kStageDefault;  // candidates per staged window (cell tile)
   bool nl_valid = false; // lists match the current order and positions
+  bool removed = false;      // scenes, since the last sort
   bool cflow_valid = false;  // per-cell flow flags match the current order
   bool fresh_sort = false;   // offsets renormalised, no motion since the sort
   int32_t nl_cap = 0;
@@ -1264,15 +1265,17 @@ int tsph_add_scene(void* engine, const tsph_scene_desc* desc, int* out_slot) {
       if (P.flag) HIP_TRY(hipMemsetAsync(P.flag + pb, 0, n * 4, E->stream));
     }
     HIP_TRY(hipMemsetAsync(E->w.status + 2 * slot, 0, 16, E->stream));
-    std::vector<int32_t> first, end;
-    if ((rr = d2h(E, (const int32_t*)E->w.start, cb, 1, first)) ||
-        (rr = d2h(E, (const int32_t*)E->w.start, cb + ncell, 1, end)))
-      return rr;
-    const int32_t delta = end[0] - first[0];
-    const int64_t last = delta ? (int64_t)E->ccap + 1 : cb + ncell;
     const OnDevice on(E->device);
-    hipLaunchKernelGGL(k_empty_cells, dim3((unsigned)((last - cb + 255) / 256)), dim3(256), 0, E->stream, E->w.start,
-                       (int)cb, (int)(cb + ncell), (int)last, first[0], delta);
+    const int first = (int)cb, end = (int)(cb + ncell);
+    bool next = false;
+    for (const SceneDev& o : E->scenes) next = next || (o.active && o.cbase == end);
+    hipLaunchKernelGGL(k_empty_cells, dim3((end - first + 255) / 256), dim3(256), 0, E->stream, E->w.start, first, end,
+                       next ? 1 : 0, E->w.bsum);
+    if (next && E->removed) {
+      const int n = E->ccap + 1;
+      hipLaunchKernelGGL(k_close_cells, dim3((n - end + 255) / 256), dim3(256), 0, E->stream, E->w.start, end, n,
+                         (const int32_t*)E->w.bsum);
+    }
     HIP_TRY(hipGetLastError());
     return TSPH_OK;
   }();
@@ -1304,6 +1307,7 @@ int tsph_remove_scene(void* engine, int slot) {
   E->calloc_.release(E->scenes[slot].cbase);
   E->scenes[slot].active = 0;
   E->nl_valid = E->cflow_valid = E->fresh_sort = false;
+  E->removed = true;
   return upload_tables(E);
 }
 
@@ -1343,6 +1347,7 @@ int tsph_step(void* engine, int nsteps) {
       if (r) return r;
     }
   }
+  E->removed = false;
   for (size_t s = 0; s < E->scenes.size(); ++s)
     if (E->scenes[s].active) E->steps[s] += nsteps;
   return TSPH_OK;
@@ -1388,6 +1393,7 @@ int tsph_run_pass(void* engine, int pass_id) {
   if (E->dim == 2) run(Seq<2>{E, L});
   else run(Seq<3>{E, L});
   if (L.status) return L.status;
+  if (pass_id == TSPH_PASS_SORT || pass_id == TSPH_PASS_STEP) E->removed = false;
   if (pass_id == TSPH_PASS_STEP)
     for (size_t s = 0; s < E->scenes.size(); ++s)
       if (E->scenes[s].active) E->steps[s] += 1;

@@ -396,16 +396,24 @@ __global__ __launch_bounds__(kSmallBlock) void k_sort_small(KArgs a, int nslots)
 
 // The cells [cb, ce) of a scene just added, which no sort has filled yet,
 // hold nothing: its first entry stays (the end of the scene below, if one
-// ends there), the others become v, its value, and all above move down by
-// delta = (entry ce) - v, which leaves the other scenes' ranges as they are,
-// for only differences of entries are used.  A sort of small scenes writes
+// ends there) and the others take its value.  A sort of small scenes writes
 // their own entries only, so a range that a removed scene held keeps that
 // scene's counts, and a pass run before the next sort would walk them.
-__global__ __launch_bounds__(256) void k_empty_cells(int32_t* __restrict__ start, int cb, int ce, int n, int32_t v,
-                                                     int32_t delta) {
-  const int i = cb + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i < ce) start[i] = v;
-  else if (i < n) start[i] -= delta;
+// next: entry ce is the first of another scene.  It is too high by `excess`,
+// the particles of scenes removed since the last sort, by which it and all
+// above then move down: the others' ranges stay as they are, for only
+// differences of entries are used.
+__global__ __launch_bounds__(256) void k_empty_cells(int32_t* __restrict__ start, int cb, int ce, int next,
+                                                     int32_t* __restrict__ excess) {
+  const int i = cb + 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int32_t v = start[cb];
+  if (i < ce || (i == ce && !next)) start[i] = v;
+  if (i == ce && next) *excess = start[ce] - v;
+}
+__global__ __launch_bounds__(256) void k_close_cells(int32_t* __restrict__ start, int ce, int n,
+                                                     const int32_t* __restrict__ excess) {
+  const int i = ce + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < n) start[i] -= *excess;
 }
 
 __global__ __launch_bounds__(256) void k_scatter(KArgs a) {
