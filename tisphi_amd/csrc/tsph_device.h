@@ -611,17 +611,21 @@ __device__ __forceinline__ void sum_list(const SceneDev& S, const uint32_t* __re
     e0 = f0;
     e1 = f1;
   }
-  // the list's end: the padding's terms are left out, which an infinite state
-  // of the particle itself would make 0 * infinity
-  auto last = [&](uint32_t e, int kq) {
-    const bool in = kq + (int)(threadIdx.x & 3) < n;
-    pair(e, rec(e), t);
+  if (k + 4 < n) {
+    pair(e0, rec(e0), t);
+    ordered_add<4>(acc, t);
+    e0 = e1;
+    k += 4;
+  }
+  if (k < n) {
+    // the last quad: the padding's terms are left out, which an infinite state
+    // of the particle itself would make 0 * infinity
+    const bool in = k + (int)(threadIdx.x & 3) < n;
+    pair(e0, rec(e0), t);
 #pragma unroll
     for (int c = 0; c < NT; ++c) t[c] = term_if(in, t[c]);
     ordered_add<4>(acc, t);
-  };
-  if (k < n) last(e0, k);
-  if (k + 4 < n) last(e1, k + 4);
+  }
 }
 
 }  // namespace tsph

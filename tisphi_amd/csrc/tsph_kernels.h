@@ -292,13 +292,13 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(int32_t* __restrict__ 
 // histogram in LDS: one launch for four.  A workgroup takes a scene slot,
 // so a batch of small scenes fills the chip.  Bounded by what a thread's registers hold
 // (kSmallItems particles) and by 64 KiB of LDS, the wave sums included
-// (kSmallCells); two workgroups of 1024 threads are all that a CU holds, so
-// the LDS costs no occupancy (9.1 k particles in 2D: 11.0 us, as with the LDS
-// sized by the scene's cells).  Up to there it is the faster route: per step against the four launches, 1.5 k particles in
-// 1.8 k cells 51 against 60 us, 9.4 k in 14.0 k cells 64 against 68, 15.0 k in
-// 1.8 k cells 60.5 against 61.6, 16.1 k in 7.7 k cells 67 and 67, 16.1 k in
-// 3D 95 against 96; 64 scenes of 14 k particles and cells 297 against 315,
-// 256 of them 1257 against 1334.
+// (kSmallCells); at these registers a CU holds one such workgroup, so the LDS
+// costs no occupancy (9.1 k particles in 2D: 11.0 us, as with the LDS sized by
+// the scene's cells).  Up to there it is the faster route: per step against
+// the four launches, 1.5 k particles in 1.8 k cells 51 against 60 us, 9.4 k in
+// 14.0 k cells 64 against 68, 15.0 k in 1.8 k cells 60.5 against 61.6, 16.1 k
+// in 7.7 k cells 67 and 67, 16.1 k in 3D 95 against 96; 64 scenes of 14 k
+// particles and cells 297 against 315, 256 of them 1257 against 1334.
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallItems = 16;
 constexpr int kSmallParticles = kSmallBlock * kSmallItems;
