@@ -1225,8 +1225,8 @@ __global__ __launch_bounds__(256) void k_wc_bdy(KArgs a, int again) {
 // d_density then carry.  So `odd` gathers the bits of the neighbours' v_z (an
 // "or" of two of them with what is there is one instruction), a force that is
 // not finite shows in d_vel, and wc_fluid_one() then forms the sums with all
-// terms.  Batch of 256 in 2D, 1.31 M particles: passes of 92.2 and 81.1 us,
-// without the check 93.7 and 78.7.
+// terms.  Batch of 256 in 2D, 1.31 M particles: passes of 91.1 and 80.5 us,
+// without the check 93.1 and 79.0.
 template <int DIM, bool Z, bool NL, bool SHEP, int KT, bool KC, int L, int NT>
 __device__ __forceinline__ void wc_fluid_sums(const KArgs& a, const SceneDev& S, int p, const Own& o, const float4& vi,
                                               float pri, const float (&M)[9], float (&acc)[NT], uint32_t& odd) {
@@ -1297,14 +1297,14 @@ __device__ __forceinline__ void wc_fluid_one(const KArgs& a, const SceneDev& S, 
 #pragma unroll
     for (int c = 0; c < 3; ++c) sum[c] = acc[c];
     if (SHEP) sum[3 + SH] = acc[2 + SH];
-    odd = (odd | __float_as_uint(vi.z)) << 1;  // any v_z but +-0
+    odd |= __float_as_uint(vi.z);
   }
   // a lane has seen its own neighbours only: the quad's lanes go together
-  if (!kFlat || __any(odd != 0 || !(fabsf(sum[1] + sum[2]) < INFINITY))) {
+  // (exponents that only together have all bits cost the second sums' time)
+  constexpr uint32_t kInf = 0x7F800000u;
+  if (!kFlat || __any((odd & kInf) == kInf || !(fabsf(sum[1] + sum[2]) < INFINITY))) {
     float acc[4 + SH] = {};
-    float4 v = vi;
-    // read again: kept through the loop above, v_z would cost a wave per SIMD
-    wc_fluid_sums<DIM, true, NL, SHEP, KT, KC, L>(a, S, p, o, v, pri, M, acc, odd);
+    wc_fluid_sums<DIM, true, NL, SHEP, KT, KC, L>(a, S, p, o, vi, pri, M, acc, odd);
 #pragma unroll
     for (int c = 0; c < 4 + SH; ++c) sum[c] = acc[c];
   }
@@ -1703,7 +1703,7 @@ __global__ __launch_bounds__(256) void k_mui_adv1(KArgs a) {
 // order.  (Formed where a candidate hits, they cost every candidate of the
 // wave their time: one of sixteen particles' hits nearly always.)  It reads
 // stress_tmp, which phase 1 makes the stress, and writes the stress.
-// Bound: vector issue (64 % busy) and L1 data return (70 %), of ~730
+// Bound: vector issue (66 % busy) and L1 data return (72 %), of ~730
 // candidates per particle in 3D.  120 k soil particles in 3D (307 k with
 // walls): 278 -> 193 us, 85 k in 2D: 41 -> 24 us, against a
 // lane per particle with the terms where a candidate hits and a copy after.
