@@ -159,7 +159,7 @@ struct tsph_engine {
   bool nl_lds = true;    // build them from LDS-staged cell windows
   int nl_stage = kStageDefault;  // candidates per staged window (cell tile)
   bool nl_valid = false; // lists match the current order and positions
-  bool removed = false;      // scenes, since the last sort
+  bool removed = false;  // a scene was, since the last sort
   bool cflow_valid = false;  // per-cell flow flags match the current order
   bool fresh_sort = false;   // offsets renormalised, no motion since the sort
   int32_t nl_cap = 0;

@@ -289,9 +289,9 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(int32_t* __restrict__ 
 }
 
 // The hash, scan and scatter of one small scene by one workgroup, with the
-// histogram in LDS: one launch for four.  A workgroup takes a scene slot,
-// so a batch of small scenes fills the chip.  Bounded by what a thread's registers hold
-// (kSmallItems particles) and by 64 KiB of LDS, the wave sums included
+// histogram in LDS: one launch for four.  A workgroup takes a scene slot, so a
+// batch of small scenes fills the chip.  Bounded by what a thread's registers
+// hold (kSmallItems particles) and by 64 KiB of LDS, the wave sums included
 // (kSmallCells); at these registers a CU holds one such workgroup, so the LDS
 // costs no occupancy (9.1 k particles in 2D: 11.0 us, as with the LDS sized by
 // the scene's cells).  Up to there it is the faster route: per step against
